@@ -1,0 +1,53 @@
+// fp32 products on the bf16 matrix cores.
+//
+// The fp32 matrix-core instructions run at 157 TFLOP/s on this part and the bf16 ones at 2.5 PFLOP/s.  An fp32 value is
+// the sum of three bf16 values, x = h + m + l: h is x rounded to bf16, m the rest rounded to bf16, l what is left, and
+// the three 8-bit significands hold all 24 bits of x.  A product x*y is then formed from six of the nine bf16 products,
+//     l*h' + m*h' + m*m' + h*m' + h*l' + h*h',
+// each exact in fp32, accumulated in fp32.  Rounding to nearest leaves |m| <= 2^-8 |x| and |l| <= 2^-17 |x|, so the
+// three products left out (m*l', l*m', l*l') are below (2^-25 + 2^-25 + 2^-34) |x y|: less than the 2^-24 |x y| that
+// rounding the fp32 product once would cost.  The accumulation rounds less often than the fp32 instruction's: 16 terms
+// of the depth cost six additions into the accumulator where v_mfma_f32_32x32x2_f32 makes sixteen.  Measured against
+// fp64, the sums are as close as the fp32 instruction's or closer (the tests check both).
+//
+// bf16 has the exponent range of fp32, and the bf16 instructions keep subnormal inputs and results.  Values whose top
+// part rounds beyond the largest bf16 (the last 2^-9 below FLT_MAX), infinities and NaNs come out of a split as
+// non-finite sums; the kernels form such an output again with plain fp32 multiply-adds (dot_fp32), so that infinities
+// keep their sign and values next to FLT_MAX their value.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <cstdint>
+
+namespace dyhip {
+
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float floatx2 __attribute__((ext_vector_type(2)));
+
+// two floats -> their bf16 parts, packed (first value in the low half): 11 instructions
+__device__ __forceinline__ void split3_pair(float a, float b, unsigned& h, unsigned& m, unsigned& l) {
+  h = __builtin_bit_cast(unsigned, __builtin_convertvector(floatx2{a, b}, bf16x2));
+  a -= __uint_as_float(h << 16);
+  b -= __uint_as_float(h & 0xFFFF0000u);
+  m = __builtin_bit_cast(unsigned, __builtin_convertvector(floatx2{a, b}, bf16x2));
+  a -= __uint_as_float(m << 16);
+  b -= __uint_as_float(m & 0xFFFF0000u);
+  l = __builtin_bit_cast(unsigned, __builtin_convertvector(floatx2{a, b}, bf16x2));
+}
+
+__device__ __forceinline__ bool not_finite(float x) { return !(x - x == 0.f); }
+__device__ __forceinline__ bool not_finite(const float4& v) {
+  return !((v.x - v.x) + (v.y - v.y) + (v.z - v.z) + (v.w - v.w) == 0.f);
+}
+
+// sum over k of a[k * step_a] * b[k * step_b], one multiply-add after another
+__device__ __forceinline__ float dot_fp32(const float* a, size_t step_a, const float* b, size_t step_b, unsigned K) {
+  float s = 0.f;
+#pragma unroll 1
+  for (unsigned k = 0; k < K; ++k) s = fmaf(a[size_t(k) * step_a], b[size_t(k) * step_b], s);
+  return s;
+}
+
+}  // namespace dyhip

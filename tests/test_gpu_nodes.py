@@ -1996,3 +1996,58 @@ def test_pool_growth_is_ordered_with_forked_queues_and_refused_inside_a_capture(
         assert not again.numpy().any()
     finally:
         d.close()
+
+
+# Products on the bf16 matrix cores, every fp32 operand as three bf16 values: the kernels' edges (one full round of tiles;
+# tiles cut once and finished in the kernel; tiles cut many times and added by a second kernel).
+SPLIT_GEMM_SHAPES = [(4096, 4096, 256), (4352, 4096, 512), (1000, 1000, 8200)]
+
+
+def _three_forms(dev, M, N, K, l, r, y0, beta):
+    """l: K x M, r: N x K (numpy); the product in the three forms."""
+    for form in ("nn", "tn", "nt"):
+        lt, rt = dev.tensor(f32(l.T) if form == "tn" else l), dev.tensor(f32(r.T) if form == "nt" else r)
+        yt = dev.tensor(y0)
+        getattr(dev, "gemm_" + form)(M, N, K, lt, rt, beta, yt)
+        yield form, yt.numpy()
+        for w in lib_pools():
+            dev.free_pool(w)
+
+
+@pytest.mark.parametrize("M,N,K", SPLIT_GEMM_SHAPES)
+def test_gemm_split_products_have_fp32_precision_over_the_exponent_range(dev, M, N, K):
+    """Rows of l and columns of r scaled by powers of two from 2^-50 to 2^50.  A sum of K random terms accumulated with
+    roundings of at most one ulp is off by about 0.36 * sqrt(K) * 2^-24 of its size (six additions per 16 terms of the
+    depth into a partial sum that grows like a random walk, an rms rounding error of 0.41 ulp): the bound is 0.5 * sqrt(K) *
+    2^-24.  Dropping even one of the three parts' products would leave 2^-17."""
+    rng = np.random.default_rng(M + K)
+    l, r = f32(rng.standard_normal((K, M))), f32(rng.standard_normal((N, K)))
+    sl, sr = 2.0 ** rng.integers(-50, 51, M), 2.0 ** rng.integers(-50, 51, N)
+    exact = (r.astype(np.float64) @ l.astype(np.float64))
+    for form, y in _three_forms(dev, M, N, K, f32(l * sl), f32(r * sr[:, None]), np.zeros((N, M), np.float32), 0.0):
+        err = y.astype(np.float64) / sl / sr[:, None] - exact
+        assert np.linalg.norm(err) <= 0.5 * np.sqrt(K) * 2.0 ** -24 * np.linalg.norm(exact), form
+
+
+@pytest.mark.parametrize("M,N,K", SPLIT_GEMM_SHAPES)
+def test_gemm_split_products_keep_infinities_nans_and_huge_values(dev, M, N, K):
+    """Where an operand is infinite, NaN or rounds beyond the largest bf16, its outputs are formed by plain fp32
+    multiply-adds: the same infinities, NaNs and finite values as fp32 arithmetic gives."""
+    rng = np.random.default_rng(K)
+    l, r = f32(rng.standard_normal((K, M))), f32(rng.standard_normal((N, K)))
+    l[5, 7], r[9, K - 3], l[40, 100], r[50, 5] = np.inf, -np.inf, np.nan, 0.0
+    l[11, 20] = 3.4e38
+    r[:, 11] *= 1e-3
+    y0 = f32(rng.standard_normal((N, M)))
+    with np.errstate(all="ignore"):
+        want = (r.astype(np.float64) @ l.astype(np.float64) + y0)
+    assert np.isinf(want).any() and np.isnan(want).any()
+    for form, y in _three_forms(dev, M, N, K, l, r, y0, 1.0):
+        assert np.array_equal(np.isnan(y), np.isnan(want)), form
+        inf = np.isinf(want)
+        assert np.array_equal(np.isinf(y), inf) and np.array_equal(y[inf], want[inf].astype(np.float32)), form
+        fin = np.isfinite(want)
+        fin[:, 20] = False
+        assert_close(y[fin], want[fin], FWD_RTOL, form, floor=np.sqrt(K))
+        col = np.isfinite(want[:, 20])
+        assert_close(y[col, 20], want[col, 20], FWD_RTOL, form + ": the column of the huge value")
