@@ -1,5 +1,5 @@
-// Internal interface of the fp32 MFMA GEMM (gemm.hip), shared with the fused
-// LSTM launchers.
+// Internal interface of the fp32 GEMM (gemm.hip), shared with the fused LSTM
+// launchers.
 #pragma once
 
 #include "common.h"
@@ -47,6 +47,26 @@ struct GemmBatch {
   size_t stride_a, stride_b, stride_c;
 };
 
+// Which output tile a block takes.  Blocks go to the XCDs round robin, so block index modulo 8 names an XCD; each XCD
+// gets a contiguous range of tiles in an order that walks panels of `panel` tile rows, column by column: its range is
+// then a rectangle whose rows and columns (what its L2 has to fetch from beyond) are balanced.
+struct TileOrder {
+  unsigned tiles_m, tiles_n, panel;
+  // em, en: extents of a tile along m and n, in any unit
+  static TileOrder of(unsigned tiles_m, unsigned tiles_n, unsigned em, unsigned en) {
+    TileOrder o{tiles_m, tiles_n, 1};
+    const unsigned share = (tiles_m * tiles_n + 7) / 8;
+    while (o.panel < tiles_m && (o.panel + 1) * o.panel * em <= share * en) ++o.panel;
+    return o;
+  }
+  __device__ __forceinline__ void locate(unsigned block, unsigned& tm, unsigned& tn) const {
+    const unsigned T = tiles_m * tiles_n, xcd = block % 8, tile = xcd * (T / 8) + min(xcd, T % 8) + block / 8;
+    const unsigned p = tile / (panel * tiles_n), r = tile - p * (panel * tiles_n), rows = min(panel, tiles_m - p * panel);
+    tn = __builtin_amdgcn_readfirstlane(r / rows);  // the division's result is not known to be uniform otherwise
+    tm = __builtin_amdgcn_readfirstlane(p * panel + r - tn * rows);
+  }
+};
+
 // C is M x N column-major (ldc = M).  Segments share the operand layouts.
 int gemm_run(dyhip_device* dev, bool a_kmajor, bool b_kmajor, size_t M, size_t N, int nseg, const GemmSeg* segs,
              float* C, const GemmEpiParams& epi, const GemmBatch* batch = nullptr);
@@ -54,10 +74,24 @@ int gemm_run(dyhip_device* dev, bool a_kmajor, bool b_kmajor, size_t M, size_t N
 // reduce.hip: out[j] (+)= sum over `splits` partial rows of n floats, in ascending order
 int combine_partial_rows(dyhip_device* dev, size_t n, unsigned splits, const float* partial, float* out, bool accumulate);
 
+// gemm_direct.hip, gemm_tile.hip: products of ordinary size, tiles of 32*tm x 32*tn outputs with the depth over `waves`
+// wavefronts (tm, tn, waves: 1,1,4  1,1,8  2,1,4  2,1,8  2,2,4), and tiles of 128 x 128.  The depth is split over about
+// splits_wanted blocks; *splits is their number; with `partial` their slices of M x N floats go there, else (one split) the
+// epilogue is applied.
+int gemm_direct_launch(dyhip_device* dev, bool a_kmajor, bool b_kmajor, size_t M, size_t N, int nseg, const GemmSeg* segs,
+                       float* C, float* partial, const GemmEpiParams& epi, const GemmBatch* batch, int tm, int tn,
+                       int waves, unsigned splits_wanted, unsigned* splits);
+int gemm_tile_launch(dyhip_device* dev, bool a_kmajor, bool b_kmajor, size_t M, size_t N, int nseg, const GemmSeg* segs,
+                     float* C, float* partial, const GemmEpiParams& epi, const GemmBatch* batch, unsigned splits_wanted,
+                     unsigned* splits);
+
+// gemm.hip: C = epilogue(sum of `splits` slices of M x N floats, in ascending order)
+int gemm_slices_sum(dyhip_device* dev, size_t M, size_t N, unsigned splits, const float* partial, float* C,
+                    const GemmEpiParams& epi);
+
 // gemm_small.hip: one-launch products for operands of a few hundred KB, any layout, single or strided-batched, with
 // the axpby or the bias epilogue.
-bool gemm_small_eligible(const dyhip_device* dev, size_t M, size_t N, size_t K, const GemmEpiParams& epi, unsigned batch,
-                         bool tile_kernel_vectorizes);
+bool gemm_small_eligible(const dyhip_device* dev, size_t M, size_t N, size_t K, const GemmEpiParams& epi, unsigned batch);
 int gemm_small_run(dyhip_device* dev, bool a_kmajor, bool b_kmajor, size_t M, size_t N, const GemmSeg& s, float* C,
                    const GemmEpiParams& epi, const GemmBatch* batch);
 

@@ -1,315 +1,21 @@
-// fp32 GEMM on the CDNA matrix cores (v_mfma_f32_32x32x2_f32: fp32 inputs,
-// fp32 accumulate, no reduced-precision shortcut), in the three forms DyNet's
-// GEMM shim needs (dynet/matrix-multiply.h:16-37,97-117,162-180), replacing its
-// cublasSgemm calls.
-//
-// Tiling.  A 256-thread block (4 wavefronts, 2 x 2) owns a 128 x (64*WN) tile of
-// C; each wavefront owns 64 x (32*WN) of it as 2 x WN accumulators of 32x32.  K
-// advances in steps of 32 through a double-buffered LDS stage.  Both operand
-// tiles sit in LDS as lds[k][mn], whatever their orientation in memory, so one
-// lane fetches the operand values of two (WN) neighbouring rows with a single
-// 64-bit LDS read: the rows of a wave's tile are interleaved over its MFMA
-// blocks (tile row 2*i + b belongs to block b), which is only a relabelling of
-// the output rows.  The row pitch is W+4 floats for an operand stored along mn
-// (128-bit LDS writes) and W+2 for one stored along k (transposing 32-bit writes
-// land on 32 distinct banks).
-//
-// The MFMA "row" index is fed from B and the "column" index (lane % 32) from A,
-// so a lane ends up holding two consecutive rows m of C for each of its columns
-// and a wavefront stores 256 contiguous bytes per column.
-//
-// Schedule per K-tile: issue the global loads of the next tile, run the 16 MFMA
-// steps with the LDS reads of step s+1 in flight under the MFMAs of step s
-// (pinned with scheduling barriers: left alone the compiler waits for every read
-// right before its use), park the next tile in the other LDS buffer three
-// quarters of the way through, barrier.  Two blocks per CU (LDS-limited) cover
-// each other's barrier bubbles; more resident wavefronts per SIMD lower the
-// matrix-core issue rate, fewer expose the bubbles.
-//
-// Tile count rarely divides the 256 CUs, and skinny problems (the LSTM gate
-// GEMMs have N = batch) have far too few tiles, so K is split across blocks when
-// the estimate says it pays: each split writes its partial tile to a workspace
-// and a second kernel adds the splits in ascending order (deterministic, no
-// atomics) and applies the epilogue: C = beta*C + sum, + bias, or the fused LSTM
-// gate epilogue.  The fused LSTM cell kernels consume the unreduced slices.
+// Dispatch of the fp32 products in the three forms DyNet's GEMM shim needs (dynet/matrix-multiply.h:16-37,97-117,162-180,
+// replacing its cublasSgemm calls), and the streaming kernels for a few rows or columns:
+//   * outputs of hundreds of 256 x 256 tiles: gemm_wide.hip;
+//   * a right operand of 5 to 256 columns, small outputs with deep sums: the fragment-order products of lstm.hip;
+//   * at most four (nine to 32) columns, a depth of at most 32, at most 32 rows: the kernels below, which stream the large
+//     operand once;
+//   * operands of a few hundred KB: gemm_small.hip;
+//   * everything else: 128 x 128 tiles (gemm_tile.hip) or smaller ones (gemm_direct.hip), chosen with a split of the depth
+//     by the cost model plan_mid.
+// Where the depth is split over blocks each writes its slice to a workspace and a second kernel adds the slices in
+// ascending order (deterministic, no atomics) and applies the epilogue: C = beta*C + sum, + bias, or the fused LSTM gate
+// epilogue.  The fused LSTM cell kernels consume the unreduced slices.
 #include "gemm.h"
 
 namespace dyhip {
 
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef float fvec2 __attribute__((ext_vector_type(2)));
-
-constexpr int kBM = 128;
-constexpr int kBK = 32;
-constexpr int kGemmThreads = 256;
-constexpr int kWritePos = (kBK / 2) * 3 / 4;  // MFMA step after which the next tile goes to LDS
-
-struct GemmArgs {
-  GemmSeg seg[kGemmMaxSeg];
-  int nseg;
-  unsigned ktiles0;  // k-tiles of segment 0
-  unsigned ktiles_total;
-  unsigned ktiles_per_split;
-  size_t M, N;
-  float* C;           // used when partial == nullptr
-  float beta;         // used when partial == nullptr
-  const float* bias;  // when set (and partial == nullptr): C = bias[i] + sum
-  float* partial;     // [splits][M*N] or nullptr
-  size_t stride_a, stride_b, stride_c;  // floats between consecutive batch items (blockIdx.z); 0 = shared operand
-  int vec_ok;         // every operand 16-byte aligned with a leading dimension that is a multiple of 4
-  int edge4_ok;       // vec_ok, and no 128-bit group of any operand straddles the matrix edge
-};
-
-// ---- global -> register tile loads ------------------------------------------------
-// An operand tile is W (mn extent) x 32 (k extent) floats; thread t loads float4 number t + 256*u.
-template <int W>
-struct TileRegs {
-  static constexpr int NV = (W * kBK / 4) / kGemmThreads;
-  float4 v[NV];
-};
-
-// EDGE == 0: the whole tile lies inside the matrix and is 16-byte aligned.
-// EDGE == 1: 16-byte aligned operands whose extent along the vectorised direction is a multiple of 4,
-//            so every 128-bit group is wholly inside or wholly outside: branch-free clamped 128-bit loads.
-// EDGE == 2: branch-free clamped scalar loads, zeros outside the matrix.
-template <bool KMAJOR, int W, int EDGE>
-__device__ __forceinline__ void load_tile(TileRegs<W>& r, const float* __restrict__ p, size_t ld, size_t mn0,
-                                          size_t k0, size_t MN, size_t K) {
-#pragma unroll
-  for (int u = 0; u < TileRegs<W>::NV; ++u) {
-    const int f = threadIdx.x + kGemmThreads * u;
-    size_t mn, kk;
-    if (!KMAJOR) {
-      mn = mn0 + size_t(f % (W / 4)) * 4;
-      kk = k0 + f / (W / 4);
-    } else {
-      mn = mn0 + f / (kBK / 4);
-      kk = k0 + size_t(f % (kBK / 4)) * 4;
-    }
-    if (EDGE == 0) {
-      r.v[u] = *reinterpret_cast<const float4*>(KMAJOR ? p + kk + mn * ld : p + mn + kk * ld);
-    } else if (EDGE == 1) {
-      const bool ok = mn < MN && kk < K;
-      const size_t mc = ok ? mn : 0, kc = ok ? kk : 0;
-      const float4 x = *reinterpret_cast<const float4*>(KMAJOR ? p + kc + mc * ld : p + mc + kc * ld);
-      r.v[u] = make_float4(ok ? x.x : 0.f, ok ? x.y : 0.f, ok ? x.z : 0.f, ok ? x.w : 0.f);
-    } else {
-      float e[4];
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        const size_t mi = KMAJOR ? mn : mn + c, ki = KMAJOR ? kk + c : kk;
-        const bool ok = mi < MN && ki < K;
-        const size_t mc = mi < MN ? mi : MN - 1, kc = ki < K ? ki : K - 1;
-        const float x = KMAJOR ? p[kc + mc * ld] : p[mc + kc * ld];
-        e[c] = ok ? x : 0.f;
-      }
-      r.v[u] = make_float4(e[0], e[1], e[2], e[3]);
-    }
-  }
-}
-
-template <bool KMAJOR, int W>
-constexpr int lds_pitch() {
-  return KMAJOR ? W + 2 : W + 4;
-}
-
-template <bool KMAJOR, int W>
-__device__ __forceinline__ void store_tile(const TileRegs<W>& r, float* __restrict__ lds) {
-  constexpr int P = lds_pitch<KMAJOR, W>();
-#pragma unroll
-  for (int u = 0; u < TileRegs<W>::NV; ++u) {
-    const int f = threadIdx.x + kGemmThreads * u;
-    if (!KMAJOR) {
-      const int k = f / (W / 4), m4 = f % (W / 4);
-      *reinterpret_cast<float4*>(lds + k * P + m4 * 4) = r.v[u];
-    } else {
-      const int k4 = f % (kBK / 4), mn_l = f / (kBK / 4);
-      float* q = lds + (k4 * 4) * P + mn_l;
-      q[0] = r.v[u].x;
-      q[P] = r.v[u].y;
-      q[2 * P] = r.v[u].z;
-      q[3 * P] = r.v[u].w;
-    }
-  }
-}
-
-template <int V>
-__device__ __forceinline__ void lds_read(const float* p, float (&out)[V]) {
-  if constexpr (V == 1) {
-    out[0] = *p;
-  } else {
-    const fvec2 t = *reinterpret_cast<const fvec2*>(p);
-    out[0] = t[0];
-    out[1] = t[1];
-  }
-}
-
-// k-tile kt of the (up to two) concatenated K segments -> its segment and offset
-__device__ __forceinline__ void locate_ktile(const GemmArgs& g, unsigned kt, GemmSeg& sg, size_t& k0) {
-  if (g.nseg > 1 && kt >= g.ktiles0) {
-    sg = g.seg[1];
-    k0 = size_t(kt - g.ktiles0) * kBK;
-  } else {
-    sg = g.seg[0];
-    k0 = size_t(kt) * kBK;
-  }
-}
-
-template <bool A_KMAJOR, bool B_KMAJOR, int WN>
-__device__ __forceinline__ void load_pair(const GemmArgs& g, unsigned kt, bool interior, size_t m0, size_t n0,
-                                          TileRegs<kBM>& ra, TileRegs<64 * WN>& rb) {
-  constexpr int BN = 64 * WN;
-  GemmSeg sg;
-  size_t k0;
-  locate_ktile(g, kt, sg, k0);
-  if (interior && k0 + kBK <= sg.K) {
-    load_tile<A_KMAJOR, kBM, 0>(ra, sg.A, sg.lda, m0, k0, g.M, sg.K);
-    load_tile<B_KMAJOR, BN, 0>(rb, sg.B, sg.ldb, n0, k0, g.N, sg.K);
-  } else if (g.edge4_ok) {
-    load_tile<A_KMAJOR, kBM, 1>(ra, sg.A, sg.lda, m0, k0, g.M, sg.K);
-    load_tile<B_KMAJOR, BN, 1>(rb, sg.B, sg.ldb, n0, k0, g.N, sg.K);
-  } else {
-    load_tile<A_KMAJOR, kBM, 2>(ra, sg.A, sg.lda, m0, k0, g.M, sg.K);
-    load_tile<B_KMAJOR, BN, 2>(rb, sg.B, sg.ldb, n0, k0, g.N, sg.K);
-  }
-}
-
-// One K-tile of the main loop: MFMA steps on LDS buffer `buf`, with the global loads of
-// tile i+PF issued first (into register slot S) and the tile i+1 (register slot S^1 for
-// PF == 2, S for PF == 1) parked in the other LDS buffer three quarters of the way through.
-template <bool A_KMAJOR, bool B_KMAJOR, int WN, int PF, int S>
-__device__ __forceinline__ void ktile_iter(const GemmArgs& g, unsigned kt_begin, unsigned n_tiles, unsigned i,
-                                           bool interior, size_t m0, size_t n0, TileRegs<kBM> (&ra)[PF],
-                                           TileRegs<64 * WN> (&rb)[PF], float* lds_a, float* lds_b,
-                                           floatx16 (&acc)[WN][2], int wm, int wn, int l32, int lhi) {
-  constexpr int BN = 64 * WN;
-  constexpr int PA = lds_pitch<A_KMAJOR, kBM>(), PB = lds_pitch<B_KMAJOR, BN>();
-  constexpr int NEXT = PF == 2 ? (S ^ 1) : S;  // register slot holding tile i+1
-  const int buf = i & 1;
-  if (i + PF < n_tiles) load_pair<A_KMAJOR, B_KMAJOR, WN>(g, kt_begin + i + PF, interior, m0, n0, ra[S], rb[S]);
-  const bool more = i + 1 < n_tiles;
-  const float* la = lds_a + buf * (kBK * PA) + wm * 64 + 2 * l32 + lhi * PA;
-  const float* lb = lds_b + buf * (kBK * PB) + wn * 32 * WN + WN * l32 + lhi * PB;
-  float av[2][2], bv[2][WN];
-  lds_read<2>(la, av[0]);
-  lds_read<WN>(lb, bv[0]);
-#pragma unroll
-  for (int s = 0; s < kBK / 2; ++s) {
-    const int cur = s & 1;
-    if (s + 1 < kBK / 2) {
-      lds_read<2>(la + (2 * s + 2) * PA, av[cur ^ 1]);
-      lds_read<WN>(lb + (2 * s + 2) * PB, bv[cur ^ 1]);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int a = 0; a < WN; ++a)
-#pragma unroll
-      for (int b = 0; b < 2; ++b)
-        acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x2f32(bv[cur][a], av[cur][b], acc[a][b], 0, 0, 0);
-    __builtin_amdgcn_sched_barrier(0);
-    if (s == kWritePos && more) {
-      // the other buffer was last read in the previous iteration, which every wave has left
-      store_tile<A_KMAJOR, kBM>(ra[NEXT], lds_a + (buf ^ 1) * (kBK * PA));
-      store_tile<B_KMAJOR, BN>(rb[NEXT], lds_b + (buf ^ 1) * (kBK * PB));
-      __builtin_amdgcn_sched_barrier(0);
-    }
-  }
-  __syncthreads();
-}
-
-// PF = how many K-tiles ahead the global loads run (register stages).  Two for the 64-wide
-// tile: its blocks are the skinny, split-K ones whose few K-tiles are bound by load latency.
-template <bool A_KMAJOR, bool B_KMAJOR, int WN, int PF>
-__global__ __launch_bounds__(kGemmThreads, 2) void gemm_tile_kernel(GemmArgs g, unsigned tiles_m) {
-  constexpr int BN = 64 * WN;
-  if (gridDim.z > 1) {  // strided batch: item blockIdx.z of every operand (single K segment, no split)
-    g.seg[0].A += size_t(blockIdx.z) * g.stride_a;
-    g.seg[0].B += size_t(blockIdx.z) * g.stride_b;
-    g.C += size_t(blockIdx.z) * g.stride_c;
-  }
-  constexpr int PA = lds_pitch<A_KMAJOR, kBM>(), PB = lds_pitch<B_KMAJOR, BN>();
-  __shared__ __attribute__((aligned(16))) float lds_a[2 * kBK * PA];
-  __shared__ __attribute__((aligned(16))) float lds_b[2 * kBK * PB];
-
-  const unsigned tm = blockIdx.x % tiles_m, tn = blockIdx.x / tiles_m;
-  const unsigned split = blockIdx.y;
-  const size_t m0 = size_t(tm) * kBM, n0 = size_t(tn) * BN;
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int wm = w & 1, wn = w >> 1;
-  const int l32 = lane & 31, lhi = lane >> 5;
-
-  floatx16 acc[WN][2];
-#pragma unroll
-  for (int a = 0; a < WN; ++a)
-#pragma unroll
-    for (int b = 0; b < 2; ++b)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[a][b][r] = 0.f;
-
-  const unsigned kt_begin = split * g.ktiles_per_split;
-  const unsigned kt_end = min(g.ktiles_total, kt_begin + g.ktiles_per_split);
-  const bool interior = g.vec_ok && (m0 + kBM <= g.M) && (n0 + BN <= g.N);
-
-  if (kt_begin < kt_end) {
-    const unsigned n_tiles = kt_end - kt_begin;
-    TileRegs<kBM> ra[PF];
-    TileRegs<BN> rb[PF];
-    load_pair<A_KMAJOR, B_KMAJOR, WN>(g, kt_begin, interior, m0, n0, ra[0], rb[0]);
-    if (PF == 2 && n_tiles > 1)
-      load_pair<A_KMAJOR, B_KMAJOR, WN>(g, kt_begin + 1, interior, m0, n0, ra[PF - 1], rb[PF - 1]);
-    store_tile<A_KMAJOR, kBM>(ra[0], lds_a);
-    store_tile<B_KMAJOR, BN>(rb[0], lds_b);
-    __syncthreads();
-    if (PF == 1) {
-      for (unsigned i = 0; i < n_tiles; ++i)
-        ktile_iter<A_KMAJOR, B_KMAJOR, WN, PF, 0>(g, kt_begin, n_tiles, i, interior, m0, n0, ra, rb, lds_a, lds_b, acc,
-                                                   wm, wn, l32, lhi);
-    } else {
-      for (unsigned i = 0; i < n_tiles; i += 2) {
-        ktile_iter<A_KMAJOR, B_KMAJOR, WN, PF, 0>(g, kt_begin, n_tiles, i, interior, m0, n0, ra, rb, lds_a, lds_b, acc,
-                                                   wm, wn, l32, lhi);
-        if (i + 1 < n_tiles)
-          ktile_iter<A_KMAJOR, B_KMAJOR, WN, PF, PF - 1>(g, kt_begin, n_tiles, i + 1, interior, m0, n0, ra, rb, lds_a,
-                                                          lds_b, acc, wm, wn, l32, lhi);
-      }
-    }
-  }
-
-  // ---- write back ----------------------------------------------------------------
-  // acc[a][b][r] of lane l: row m = m0 + 64*wm + 2*(l%32) + b,
-  //                         column n = n0 + 32*WN*wn + WN*i + a with i = 8*(r/4) + 4*(l/32) + r%4
-  float* out = g.partial ? g.partial + size_t(split) * g.M * g.N : g.C;
-  const bool direct = g.partial == nullptr;
-  const size_t m = m0 + wm * 64 + 2 * l32;
-  if (m >= g.M) return;
-  const bool pair = (m + 1 < g.M) && (g.M % 2 == 0) && ((reinterpret_cast<uintptr_t>(out) & 7u) == 0);
-  float bias0 = 0.f, bias1 = 0.f;
-  if (direct && g.bias != nullptr) {
-    bias0 = g.bias[m];
-    if (m + 1 < g.M) bias1 = g.bias[m + 1];
-  }
-#pragma unroll
-  for (int a = 0; a < WN; ++a)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int i = 8 * (r / 4) + 4 * lhi + (r % 4);
-      const size_t n = n0 + wn * 32 * WN + WN * i + a;
-      if (n >= g.N) continue;
-      float* p = out + m + n * g.M;
-      float v0 = acc[a][0][r] + bias0, v1 = acc[a][1][r] + bias1;
-      if (pair) {
-        if (direct && g.beta != 0.f) {
-          const fvec2 o = *reinterpret_cast<const fvec2*>(p);
-          v0 = g.beta * o[0] + v0;
-          v1 = g.beta * o[1] + v1;
-        }
-        *reinterpret_cast<fvec2*>(p) = fvec2{v0, v1};
-      } else {
-        p[0] = (direct && g.beta != 0.f) ? g.beta * p[0] + v0 : v0;
-        if (m + 1 < g.M) p[1] = (direct && g.beta != 0.f) ? g.beta * p[1] + v1 : v1;
-      }
-    }
-}
 
 // C[e] = epilogue(sum_s partial[s][e]), splits added in ascending order
 template <int EPI>
@@ -341,48 +47,64 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(size_t M, size_
   }
 }
 
-template <bool A_KMAJOR, bool B_KMAJOR>
-static void launch_tiles(dyhip_device* dev, const GemmArgs& g, unsigned tiles_m, unsigned tiles_n, unsigned splits,
-                         int wn, unsigned batch = 1) {
-  const dim3 grid(tiles_m * tiles_n, splits, batch), block(kGemmThreads);
-  if (wn == 1)
-    hipLaunchKernelGGL((gemm_tile_kernel<A_KMAJOR, B_KMAJOR, 1, 2>), grid, block, 0, dev->stream, g, tiles_m);
+int gemm_slices_sum(dyhip_device* dev, size_t M, size_t N, unsigned splits, const float* partial, float* C,
+                    const GemmEpiParams& epi) {
+  const size_t total = M * N;
+  const dim3 grid((unsigned)cdiv<size_t>(total, 256)), block(256);
+  if (epi.kind == kEpiLstmGates)
+    hipLaunchKernelGGL(gemm_splitk_reduce_kernel<kEpiLstmGates>, grid, block, 0, dev->stream, M, total, splits, partial, C, epi);
+  else if (epi.kind == kEpiBias)
+    hipLaunchKernelGGL(gemm_splitk_reduce_kernel<kEpiBias>, grid, block, 0, dev->stream, M, total, splits, partial, C, epi);
   else
-    hipLaunchKernelGGL((gemm_tile_kernel<A_KMAJOR, B_KMAJOR, 2, 1>), grid, block, 0, dev->stream, g, tiles_m);
+    hipLaunchKernelGGL(gemm_splitk_reduce_kernel<kEpiAxpby>, grid, block, 0, dev->stream, M, total, splits, partial, C, epi);
+  DYHIP_CHECK_LAUNCH();
+  return DYHIP_OK;
 }
 
-// Tile width and split count by a small cost model.  Measured on MI355X: the matrix cores
-// sustain ~2.0 GHz under this kernel (131 TFLOP/s over 256 CUs); a CU running two blocks
-// keeps them ~95 % busy, a lone block ~77 %; the 64-wide tile reads more LDS per MFMA.
-struct GemmPlan {
-  int wn;
+// Which kernel, tile and split of the depth.  Times measured on this GPU (us, in a graph of dependent launches): a launch
+// with its first loads and its end, and per 1000 k for one, two or three blocks on a CU.
+struct MidConfig {
+  int tm, tn, waves;  // gemm_direct.hip: 32-row and 32-column tiles of a block, its wavefronts; tm = 4: gemm_tile.hip
+  int per_cu;         // blocks a CU holds
+  double base, per_k[3];
+};
+//                                           measured at
+constexpr MidConfig kMidConfigs[] = {
+    {1, 1, 4, 3, 4.6, {5.8, 10.3, 15.0}},   // 1024 x 512 x 784: 11.8, x 2048: 24.1
+    {1, 1, 8, 2, 4.6, {5.5, 10.5, 0.0}},    // 50 x 512 x 1024 in 8 parts: 8.1 with the sum of the parts
+    {2, 1, 4, 2, 4.9, {9.1, 17.8, 0.0}},    // 1024 x 512 x 2048: 23.9; 1024 x 1024 x 512: 14.1
+    {2, 1, 8, 1, 4.9, {8.2, 0.0, 0.0}},     // 1024 x 512 x 1024: 13.0, x 4096: 38.2
+    {2, 2, 4, 2, 5.5, {14.5, 31.0, 0.0}},   // 4096 x 256 x 4480: 69.3; 2048 x 2240 x 512: 47.0
+    {4, 4, 4, 2, 6.5, {65.0, 104.0, 0.0}},  // 4096 x 384 x 256: 24.1; 10 000 x 700 x 650: 73.7
+};
+
+struct MidPlan {
+  const MidConfig* c;
   unsigned splits;
 };
 
-static GemmPlan plan_gemm(const dyhip_device* dev, size_t M, size_t N, unsigned ktiles, size_t max_splits_ws,
-                          bool must_use_partials) {
+static MidPlan plan_mid(const dyhip_device* dev, size_t M, size_t N, size_t K, unsigned items, size_t max_splits_ws) {
+  MidPlan best{&kMidConfigs[0], 1};
+  if (K < 32) return best;  // the fp32 instruction, one form
   const double cus = dev->num_cus > 0 ? dev->num_cus : 256;
-  const double peak = cus * 256.0 * 2.0e9, ws_bw = 3.0e12;
-  GemmPlan best{2, 1};
   double best_t = 1e30;
-  for (int wn = 2; wn >= 1; --wn) {
-    if (wn == 2 && N <= 64) continue;
-    const double tiles = double(cdiv<size_t>(M, kBM)) * double(cdiv<size_t>(N, size_t(64) * wn));
-    // a tile costs its full multiply-adds whatever part of it lies inside the matrix (a 650 x 1 product priced by
-    // its own multiply-adds was never split over the depth: one block per 128 rows walked all k-tiles, 53 us)
-    const double flops = 2.0 * tiles * double(kBM) * 64.0 * wn * double(ktiles) * kBK;
+  for (const MidConfig& c : kMidConfigs) {
+    const double tiles = double(cdiv<size_t>(M, size_t(32) * c.tm)) * double(cdiv<size_t>(N, size_t(32) * c.tn)) * items;
     for (unsigned s = 1; s <= 32; ++s) {
-      if (s > 1 && (ktiles / s < 2 || s > max_splits_ws)) break;
-      const double blocks = tiles * s;
-      const double rounds = blocks <= cus ? 1.0 : double(cdiv<size_t>(size_t(blocks), size_t(cus)));
-      const double eff = blocks / (rounds * cus);
-      double inloop = blocks >= 2 * cus ? 0.95 : (blocks > cus ? 0.85 : 0.77);
-      if (wn == 1) inloop *= 0.9;
-      double t = flops / (peak * eff * inloop) + rounds * 1.0e-6;
-      if (s > 1 || must_use_partials) t += 2.0 * double(M) * double(N) * 4.0 * s / ws_bw + 2.0e-6;
+      if (s > 1 && (K / s < 128 || s > max_splits_ws || items > 1)) break;
+      // blocks a CU gets: so many rounds of a full CU, and a last one
+      const double n = tiles * s / cus, rounds = double(size_t(n / c.per_cu)), rest = n - rounds * c.per_cu;
+      const int last = rest <= 0.0 ? 0 : int(rest) + (rest > double(int(rest)) ? 1 : 0);
+      const double per_k = rounds * c.per_k[c.per_cu - 1] + (last > 0 ? c.per_k[last - 1] : 0.0);
+      // a further round starts cold: beside other blocks of the CU or on an empty one
+      const double more = rounds + (last > 0 ? 1.0 : 0.0) - 1.0;
+      double t = c.base + per_k * 1e-3 * double(K) / s + (more > 0.0 ? more * (c.per_cu == 1 ? 4.0 : 2.2) : 0.0);
+      // operands that are not in the L2s: what the blocks read, and the slices of a split
+      t += tiles * 128.0 * (c.tm + c.tn) * double(K) / 40e6;
+      if (s > 1) t += 2.6 + double(M) * double(N) * 4.0 * (s + 2) / 8e6;
       if (t < best_t) {
         best_t = t;
-        best = GemmPlan{wn, s};
+        best = MidPlan{&c, s};
       }
     }
   }
@@ -1169,12 +891,12 @@ int gemm_run(dyhip_device* dev, bool a_kmajor, bool b_kmajor, size_t M, size_t N
   if (nseg == 1 && (batch == nullptr || batch->count <= 1) && segs[0].A != nullptr && segs[0].B != nullptr &&
       (epi.kind == kEpiAxpby || (epi.kind == kEpiBias && epi.bias != nullptr && aligned16(epi.bias)))) {
     const GemmSeg& s0 = segs[0];
-    // leading full rounds first: at small depths the 128-wide kernel finishes a few remaining tile columns (96 of its
-    // tiles) sooner than one sequence of k-tiles over all tiles does
+    // leading full rounds first: at small depths smaller tiles finish a few remaining tile columns sooner than one
+    // sequence of k-tiles over all tiles does
     size_t cols = gemm_wide_whole_rounds_columns(dev, a_kmajor, b_kmajor, M, N, s0.K, s0.A, s0.lda, s0.B, s0.ldb, C);
     if (cols == 0 && gemm_wide_eligible(dev, a_kmajor, b_kmajor, M, N, s0.K, s0.A, s0.lda, s0.B, s0.ldb, C)) cols = N;
     if (cols > 0) {
-      const size_t K32 = s0.K / kBK * kBK;
+      const size_t K32 = s0.K / 32 * 32;
       DYHIP_CHECK_STATUS(gemm_wide_run(dev, a_kmajor, b_kmajor, M, cols, K32, s0.A, s0.lda, s0.B, s0.ldb, C,
                                        epi.kind == kEpiAxpby ? epi.beta : 0.f,
                                        epi.kind == kEpiBias ? epi.bias : nullptr));
@@ -1244,99 +966,57 @@ int gemm_run(dyhip_device* dev, bool a_kmajor, bool b_kmajor, size_t M, size_t N
       gemm_shallow_nt_eligible(dev, M, N, segs[0].K, segs[0].A, segs[0].lda, segs[0].B, segs[0].ldb, C))
     return gemm_shallow_nt_run(dev, M, N, segs[0].K, segs[0].A, segs[0].lda, segs[0].B, segs[0].ldb, C, epi.beta);
   const bool batched = batch != nullptr && batch->count > 1;
-  const bool tile_vec = nseg == 1 && aligned16(segs[0].A) && segs[0].lda % 4 == 0 && aligned16(segs[0].B) &&
-                        segs[0].ldb % 4 == 0 && (!batched || (batch->stride_a % 4 == 0 && batch->stride_b % 4 == 0));
-  if (nseg == 1 && !to_caller && C != nullptr && segs[0].A != nullptr && segs[0].B != nullptr &&
-      gemm_small_eligible(dev, M, N, segs[0].K, epi, batch ? batch->count : 1, tile_vec)) {
-    if (batch != nullptr && batch->count > 1)
-      DYHIP_REQUIRE(batch->stride_c >= M * N, "batch items of the GEMM output overlap");
-    return gemm_small_run(dev, a_kmajor, b_kmajor, M, N, segs[0], C, epi, batch);
-  }
-  GemmArgs g;
-  g.nseg = nseg;
-  g.M = M;
-  g.N = N;
-  g.C = C;
-  g.beta = epi.kind == kEpiAxpby ? epi.beta : 0.f;
-  g.bias = epi.kind == kEpiBias ? epi.bias : nullptr;
-  g.ktiles_total = 0;
-  g.ktiles0 = 0;
-  g.seg[1] = GemmSeg{nullptr, 0, nullptr, 0, 0};
-  const unsigned items = batch ? batch->count : 1;
-  g.stride_a = g.stride_b = g.stride_c = 0;
-  bool vec = true;
-  if (items > 1) {
+  if (batched) {
     DYHIP_REQUIRE(nseg == 1 && epi.kind == kEpiAxpby, "a strided-batched GEMM has one K segment and the axpby epilogue");
     DYHIP_REQUIRE(batch->stride_c >= M * N, "batch items of the GEMM output overlap");
-    g.stride_a = batch->stride_a;
-    g.stride_b = batch->stride_b;
-    g.stride_c = batch->stride_c;
-    vec = g.stride_a % 4 == 0 && g.stride_b % 4 == 0;
   }
+  if (nseg == 1 && !to_caller && C != nullptr && segs[0].A != nullptr && segs[0].B != nullptr &&
+      gemm_small_eligible(dev, M, N, segs[0].K, epi, batch ? batch->count : 1))
+    return gemm_small_run(dev, a_kmajor, b_kmajor, M, N, segs[0], C, epi, batch);
+  size_t K = 0;
   for (int s = 0; s < nseg; ++s) {
     DYHIP_REQUIRE(segs[s].A != nullptr && segs[s].B != nullptr, "null GEMM operand");
-    g.seg[s] = segs[s];
-    const unsigned kt = static_cast<unsigned>(cdiv<size_t>(segs[s].K, kBK));
-    if (s == 0) g.ktiles0 = kt;
-    g.ktiles_total += kt;
-    vec = vec && aligned16(segs[s].A) && segs[s].lda % 4 == 0 && aligned16(segs[s].B) && segs[s].ldb % 4 == 0;
+    K += segs[s].K;
   }
-  g.vec_ok = vec ? 1 : 0;
-  // a group of four runs along k for a k-major operand and along m (or n) otherwise
-  bool edge4 = vec && (a_kmajor || M % 4 == 0) && (b_kmajor || N % 4 == 0);
-  for (int s = 0; s < nseg; ++s) edge4 = edge4 && (!(a_kmajor || b_kmajor) || segs[s].K % 4 == 0);
-  g.edge4_ok = edge4 ? 1 : 0;
+  DYHIP_REQUIRE(M < (size_t(1) << 31) && N < (size_t(1) << 31) && K < (size_t(1) << 31) &&
+                cdiv<size_t>(M, 32) * cdiv<size_t>(N, 32) < (size_t(1) << 31), "GEMM too large");
+  const unsigned items = batch ? batch->count : 1;
   const size_t out_bytes = M * N * sizeof(float);
   const size_t ws_bytes = to_caller ? epi.partials_bytes : dev->gemm_ws_bytes;
-  void* ws = to_caller ? static_cast<void*>(epi.partials) : dev->gemm_ws;
-  const bool fused_epi = epi.kind == kEpiLstmGates;  // needs the whole sum before the activation
-  const bool must_partial = fused_epi || to_caller;
-  GemmPlan plan{N <= 64 ? 1 : 2, 1};
-  if (g.ktiles_total > 0)
-    plan = plan_gemm(dev, M, N, g.ktiles_total, items > 1 ? 1 : ws_bytes / out_bytes, must_partial);
-  unsigned splits = plan.splits;
-  const size_t tiles_m = cdiv<size_t>(M, kBM), tiles_n = cdiv<size_t>(N, size_t(64) * plan.wn);
-  DYHIP_REQUIRE(tiles_m * tiles_n < (size_t(1) << 31), "GEMM too large");
-  g.ktiles_per_split = g.ktiles_total == 0 ? 1 : cdiv<unsigned>(g.ktiles_total, splits);
-  splits = g.ktiles_total == 0 ? 1 : cdiv<unsigned>(g.ktiles_total, g.ktiles_per_split);
-  const bool use_partial = splits > 1 || must_partial;
+  float* const ws = static_cast<float*>(to_caller ? static_cast<void*>(epi.partials) : dev->gemm_ws);
+  const MidPlan plan = plan_mid(dev, M, N, K, items, ws != nullptr ? ws_bytes / out_bytes : 1);
+  const bool use_partial = plan.splits > 1 || to_caller;
   if (use_partial)
-    DYHIP_REQUIRE(ws != nullptr && ws_bytes >= out_bytes * splits,
+    DYHIP_REQUIRE(ws != nullptr && ws_bytes >= out_bytes * plan.splits,
                   "GEMM output of %zu bytes x %u splits does not fit the %zu-byte split-K workspace", out_bytes,
-                  splits, ws_bytes);
-  g.partial = use_partial ? static_cast<float*>(ws) : nullptr;
+                  plan.splits, ws_bytes);
+  float* const partial = use_partial ? ws : nullptr;
+  unsigned splits = 1;
   // grid z holds at most 65535 batch items per launch
   for (unsigned first = 0; first < items; first += 65535u) {
-    const unsigned nb = items - first < 65535u ? items - first : 65535u;
-    GemmArgs h = g;
-    h.seg[0].A += size_t(first) * g.stride_a;
-    h.seg[0].B += size_t(first) * g.stride_b;
-    if (h.C != nullptr) h.C += size_t(first) * g.stride_c;
-    if (a_kmajor && b_kmajor) launch_tiles<true, true>(dev, h, (unsigned)tiles_m, (unsigned)tiles_n, splits, plan.wn, nb);
-    else if (a_kmajor && !b_kmajor) launch_tiles<true, false>(dev, h, (unsigned)tiles_m, (unsigned)tiles_n, splits, plan.wn, nb);
-    else if (!a_kmajor && b_kmajor) launch_tiles<false, true>(dev, h, (unsigned)tiles_m, (unsigned)tiles_n, splits, plan.wn, nb);
-    else launch_tiles<false, false>(dev, h, (unsigned)tiles_m, (unsigned)tiles_n, splits, plan.wn, nb);
+    GemmSeg seg[kGemmMaxSeg];
+    for (int s = 0; s < nseg; ++s) seg[s] = segs[s];
+    GemmBatch part{};
+    float* out = C;
+    if (batched) {
+      part = *batch;
+      part.count = items - first < 65535u ? items - first : 65535u;
+      seg[0].A += size_t(first) * part.stride_a;
+      seg[0].B += size_t(first) * part.stride_b;
+      out += size_t(first) * part.stride_c;
+    }
+    if (plan.c->tm == 4)
+      DYHIP_CHECK_STATUS(gemm_tile_launch(dev, a_kmajor, b_kmajor, M, N, nseg, seg, out, partial, epi, batched ? &part : nullptr,
+                                          plan.splits, &splits));
+    else
+      DYHIP_CHECK_STATUS(gemm_direct_launch(dev, a_kmajor, b_kmajor, M, N, nseg, seg, out, partial, epi,
+                                            batched ? &part : nullptr, plan.c->tm, plan.c->tn, plan.c->waves, plan.splits, &splits));
   }
-  DYHIP_CHECK_LAUNCH();
   if (to_caller) {
     *epi.splits_out = splits;
     return DYHIP_OK;
   }
-  if (use_partial) {
-    const size_t total = M * N;
-    const dim3 grid((unsigned)cdiv<size_t>(total, 256));
-    if (fused_epi)
-      hipLaunchKernelGGL(gemm_splitk_reduce_kernel<kEpiLstmGates>, grid, dim3(256), 0, dev->stream, M, total, splits,
-                         g.partial, C, epi);
-    else if (epi.kind == kEpiBias)
-      hipLaunchKernelGGL(gemm_splitk_reduce_kernel<kEpiBias>, grid, dim3(256), 0, dev->stream, M, total, splits,
-                         g.partial, C, epi);
-    else
-      hipLaunchKernelGGL(gemm_splitk_reduce_kernel<kEpiAxpby>, grid, dim3(256), 0, dev->stream, M, total, splits,
-                         g.partial, C, epi);
-    DYHIP_CHECK_LAUNCH();
-  }
-  return DYHIP_OK;
+  return use_partial ? gemm_slices_sum(dev, M, N, splits, partial, C, epi) : DYHIP_OK;
 }
 
 static GemmEpiParams axpby(float beta) {

@@ -1,8 +1,7 @@
 // Small products C = A * B in any of the three layouts (l*r, l^T*r, l*r^T), single or strided-batched, in one launch.
 //
-// The 128 x 128-tile kernel with its split over the depth and a second launch to sum the slices costs 9..18 us on
-// products whose operands are a few hundred KB (128 x 128 x 128 as l^T*r: 9.4 us; 200 x 100 x 50: 13 us; 7 x 5 x 9
-// times 1000 items: 11 us): that is launch and pipeline latency, not arithmetic.  Here a wavefront owns a 32 x 32
+// On products whose operands are a few hundred KB the time is launch and pipeline latency, not arithmetic.  Here a
+// wavefront owns a 32 x 32
 // tile of C and feeds v_mfma_f32_32x32x2_f32 straight from global memory (the operands stay in the L2s): lane l
 // fetches, for row l % 32 of A and column l % 32 of B, the four depth indices 4 * (l / 32) .. + 3 of every group of
 // eight, as one 128-bit load where the operand is contiguous along the depth and aligned, as four loads (adjacent
@@ -148,24 +147,21 @@ static int small_depth_waves(size_t K, size_t tiles, size_t cus) {
   return K >= 512 && tiles <= 2 * cus ? 8 : 4;
 }
 
-// Which products come here instead of the 128 x 128-tile kernel (measured on 60 shapes in the three layouts).  A
-// wavefront's depth costs one memory round trip per stage of 32 indices, hidden only by other blocks on the CU, and
-// nothing is reused through LDS: the tile kernel wins from about four stages per wavefront on, unless it would run
-// its scalar-load form (operands not 16-byte aligned or leading dimensions not multiples of four), which is two to
-// ten times slower on narrow outputs.
-bool gemm_small_eligible(const dyhip_device* dev, size_t M, size_t N, size_t K, const GemmEpiParams& epi, unsigned batch,
-                         bool tile_kernel_vectorizes) {
+// Which products come here instead of gemm_direct.hip (measured on 17 shapes in the three layouts).  A wavefront's depth
+// costs one memory round trip per stage of 32 indices, hidden only by other blocks on the CU, and the fp32 matrix
+// instruction: good for one stage (512 x 300 x 100: 3.8 against 4.6 us), for two of them on few tiles (256 x 256 x 256:
+// 4.9 against 4.8..5.2; 512 x 512 x 512: 10.0 / 8.5 / 6.5 against 7.1 / 7.6 / 6.8) or on more than two one-wavefront tiles
+// per CU (2000 x 500 x 40: 5.7 against 7.1; 1024 x 512 x 50, two: 5.5..6.0 against 5.0..5.2).
+bool gemm_small_eligible(const dyhip_device* dev, size_t M, size_t N, size_t K, const GemmEpiParams& epi, unsigned batch) {
   if (epi.kind != kEpiAxpby && !(epi.kind == kEpiBias && epi.bias != nullptr)) return false;
   if (M == 0 || N == 0 || K == 0 || M > (size_t(1) << 20) || N > (size_t(1) << 20) || K > 65536 || batch > 65535u) return false;
   const size_t cus = dev->num_cus > 0 ? size_t(dev->num_cus) : 256;
   const size_t tiles = cdiv<size_t>(M, 32) * cdiv<size_t>(N, 32) * (batch > 0 ? batch : 1);
   const size_t work = tiles * cdiv<size_t>(K, 32);  // in units of one tile x one stage
   if (tiles > 16 * cus || work > 64 * cus) return false;
-  const size_t stages = cdiv<size_t>(cdiv<size_t>(K, small_depth_waves(K, tiles, cus)), 8 * kSmallGroups);
-  if (stages <= 3 || (stages <= 4 && tiles <= cus / 2)) return true;
-  if (batch > 1) return true;  // the tile kernel does not split the depth of batch items
-  if (tile_kernel_vectorizes) return false;
-  return N <= 4 || (stages <= 6 && tiles >= cus);
+  const int waves = small_depth_waves(K, tiles, cus);
+  const size_t stages = cdiv<size_t>(cdiv<size_t>(K, waves), 8 * kSmallGroups);
+  return stages <= 1 || (stages <= 2 && (tiles < cus || (waves == 1 && tiles > 2 * cus)));
 }
 
 int gemm_small_run(dyhip_device* dev, bool a_kmajor, bool b_kmajor, size_t M, size_t N, const GemmSeg& s, float* C,

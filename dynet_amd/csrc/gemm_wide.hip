@@ -41,7 +41,7 @@
 //     from beyond its L2), so every part goes to the workspace and a second kernel, 16 blocks per tile, adds them in
 //     segment order and applies the epilogue.
 // When the tiles are a whole number of rounds plus a few tile columns, the caller gives this kernel the leading
-// columns (whole rounds, nothing cut) and the rest to the 128-wide kernel.
+// columns (whole rounds, nothing cut) and the rest to the 128 x 128-tile kernel.
 #include "gemm.h"
 #include "split3.h"
 
@@ -667,7 +667,7 @@ int launch_wide(dyhip_device* dev, const WideArgs& g, unsigned blocks, unsigned 
 
 }  // namespace
 
-// How the k-tiles are dealt to the blocks.  ok = false: leave the problem to the 128-wide kernel.
+// How the k-tiles are dealt to the blocks.  ok = false: leave the problem to the smaller tiles.
 struct WidePlan {
   bool ok;
   bool finish_in_kernel;  // segments at least a tile long: a tile is cut at most once, and finished inside the kernel
@@ -685,7 +685,7 @@ static WidePlan plan_wide(const dyhip_device* dev, size_t M, size_t N, size_t K3
   p.segments = cus;
   const size_t per = units / cus;
   p.finish_in_kernel = per >= p.nt;
-  // Measured against the 128-wide kernel: a block's set-up, its share of partial tiles and of the second kernel cost
+  // Measured against 128 x 128 tiles: a block's set-up, its share of partial tiles and of the second kernel cost
   // about three k-tiles, so a problem of fewer tiles than CUs (nothing but cut tiles) needs long segments.
   p.ok = units < (size_t(1) << 31) && (p.finish_in_kernel ? p.nt >= 8 : per >= 16);
   return p;
@@ -704,7 +704,7 @@ bool gemm_wide_eligible(const dyhip_device* dev, bool a_kmajor, bool b_kmajor, s
   const size_t cus = dev->num_cus > 0 ? size_t(dev->num_cus) : 256;
   // and 32-bit byte offsets from a tile's first element
   if (lda >= (size_t(1) << 21) || ldb >= (size_t(1) << 21)) return false;
-  // edge tiles compute whole 256 x 256 tiles: ragged shapes stay with the 128-wide kernel
+  // edge tiles compute whole 256 x 256 tiles: ragged shapes stay with the smaller tiles
   if (double(M) * double(N) < 0.8 * double(tiles) * double(kSlotFloats)) return false;
   if (dev->gemm_ws == nullptr || dev->gemm_flags == nullptr || dev->gemm_ws_bytes < (2 * cus) * kSlotFloats * sizeof(float) ||
       cus + 1 > size_t(kGemmFlagWords))
@@ -773,7 +773,7 @@ bool gemm_shallow_nt_eligible(const dyhip_device* dev, size_t M, size_t N, size_
     return false;
   if (K * lda >= (size_t(1) << 31) || K * ldb >= (size_t(1) << 31) || M * N >= (size_t(1) << 31)) return false;
   const size_t cus = dev->num_cus > 0 ? size_t(dev->num_cus) : 256;
-  return cdiv<size_t>(M, 128) * cdiv<size_t>(N, 128) * 2 >= cus;  // fewer tiles: the 128-wide kernel cuts the depth
+  return cdiv<size_t>(M, 128) * cdiv<size_t>(N, 128) * 2 >= cus;  // fewer tiles: smaller ones fill the GPU
 }
 
 int gemm_shallow_nt_run(dyhip_device* dev, size_t M, size_t N, size_t K, const float* A, size_t lda, const float* B,

@@ -1998,9 +1998,11 @@ def test_pool_growth_is_ordered_with_forked_queues_and_refused_inside_a_capture(
         d.close()
 
 
-# Products on the bf16 matrix cores, every fp32 operand as three bf16 values: the kernels' edges (one full round of tiles;
-# tiles cut once and finished in the kernel; tiles cut many times and added by a second kernel).
-SPLIT_GEMM_SHAPES = [(4096, 4096, 256), (4352, 4096, 512), (1000, 1000, 8200)]
+# Products on the bf16 matrix cores, every fp32 operand as three bf16 values: the 256 x 256-tile kernel (one full round of
+# tiles; tiles cut once and finished in the kernel; tiles cut many times and added by a second kernel), 128 x 128 tiles and
+# smaller ones with ragged edges, with the depth split over blocks and not.
+SPLIT_GEMM_SHAPES = [(4096, 4096, 256), (4352, 4096, 512), (1000, 1000, 8200), (2051, 2050, 650), (333, 290, 1001),
+                     (301, 750, 96)]
 
 
 def _three_forms(dev, M, N, K, l, r, y0, beta):
@@ -2051,3 +2053,34 @@ def test_gemm_split_products_keep_infinities_nans_and_huge_values(dev, M, N, K):
         assert_close(y[fin], want[fin], FWD_RTOL, form, floor=np.sqrt(K))
         col = np.isfinite(want[:, 20])
         assert_close(y[col, 20], want[col, 20], FWD_RTOL, form + ": the column of the huge value")
+
+
+# Edges of the tiles of ordinary products: fewer than four rows (or columns) in the last tile or in the whole matrix, groups
+# of four that straddle the edge, depths at and around one and two 16-deep steps, a depth split over blocks; 128 x 128
+# tiles from about 250 of them on.
+@pytest.mark.parametrize("M,N,K,off", [(3, 700, 333, 0), (700, 3, 333, 1), (33, 290, 31, 0), (65, 289, 32, 0), (130, 257, 33, 3),
+                                       (300, 259, 47, 2), (1025, 515, 130, 1), (66, 300, 4099, 0), (2050, 2178, 79, 1),
+                                       (1921, 2053, 650, 2), (2304, 2176, 48, 0)])
+def test_gemm_ordinary_products_at_the_edges_of_tiles_and_steps(dev, M, N, K, off):
+    """l*r, l^T*r, l*r^T and the affine layer at any alignment (operands that start 4, 8 or 12 bytes into a 16-byte line)
+    against the fp64 product of the same inputs; nothing is written around the output."""
+    rng = np.random.default_rng(M + N + K + off)
+    l, r, y0, b = (f32(rng.standard_normal(s)) for s in ((K, M), (N, K), (N, M), M))
+    exact = r.astype(np.float64) @ l.astype(np.float64)
+
+    def placed(a):
+        t = dev.tensor(np.concatenate([np.full(off, np.nan, np.float32), a.ravel(), np.full(8, np.nan, np.float32)]))
+        return t, t.offset(off, a.shape)
+
+    for form, beta in (("nn", 1.0), ("tn", 0.5), ("nt", 0.0), ("affine", 0.0)):
+        (_, lt), (_, rt) = placed(f32(l.T) if form == "tn" else l), placed(f32(r.T) if form == "nt" else r)
+        whole, yt = placed(y0)
+        if form == "affine":
+            dev.affine_forward(M, N, K, dev.tensor(b), lt, rt, yt)
+            want = exact + b
+        else:
+            getattr(dev, "gemm_" + form)(M, N, K, lt, rt, beta, yt)
+            want = beta * y0 + exact
+        assert_close(yt.numpy(), want, FWD_RTOL, form, floor=np.sqrt(K))
+        around = whole.numpy()
+        assert np.isnan(around[:off]).all() and np.isnan(around[off + M * N:]).all(), form
