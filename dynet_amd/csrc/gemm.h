@@ -127,7 +127,12 @@ int thin_tn_batched(dyhip_device* dev, size_t M, size_t N, size_t K, const float
 
 // lstm.hip: C = epilogue(A0 B0 [+ A1 B1]) in one launch for a right operand of a few 32-column tiles (A: M x K with rows
 // contiguous, B: K x N with k contiguous; two segments only with the gates epilogue); *taken tells whether it ran.
+// masks: one a segment, multiplies the segment's B (as K x N) element by element; only with the gates epilogue.
+struct NnMask {
+  const float* p;
+  size_t ld;  // 0: one mask for all columns
+};
 int skinny_nn_gemm(dyhip_device* dev, size_t M, size_t N, int nseg, const GemmSeg* segs, float* C, const GemmEpiParams& epi,
-                   bool* taken);
+                   bool* taken, const NnMask* masks = nullptr);
 
 }  // namespace dyhip

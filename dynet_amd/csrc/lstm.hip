@@ -14,6 +14,7 @@
 #include <initializer_list>
 
 #include "gemm.h"
+#include "split3.h"
 
 namespace dyhip {
 
@@ -714,6 +715,8 @@ struct NnOperand {
   const float* v;  // K x N, k contiguous, leading dimension ldv
   unsigned K;
   size_t ldw, ldv;
+  const float* mask;  // multiplies v element by element (dropout), or null; only skinny_nn_deep_kernel reads it
+  size_t ldm;         // 0: one mask for all columns
 };
 enum { kNnGates = 0, kNnBias = 1, kNnAxpby = 2 };
 
@@ -828,13 +831,167 @@ __global__ __launch_bounds__(256) void skinny_nn_kernel(unsigned M, unsigned H, 
   }
 }
 
+// The same product for depths of kNnDeep and more, on the bf16 matrix cores (split3.h).  At a small batch the kernel
+// above has fewer blocks than the GPU has CUs (82 at H = 650), and a wavefront walks a quarter of the depth in rounds of
+// loads that nothing hides.  Here the depths of both products, laid end to end in chunks of 32 k, are dealt to sixteen
+// (eight with 64 rows) wavefronts; each has its next chunk in flight.  v comes in whole 128-byte lines, eight columns an
+// instruction, and goes through a wavefront's own piece of LDS into fragments: read in fragment order, 32 columns x 32
+// bytes an instruction, its line lookups alone took as long as the product.
+// MASKED: v is multiplied by its dropout mask on the way in, which saves the launches that would form the products.
+// A chunk that would run past an operand's end is moved back inside, and the k that the chunk before has already
+// multiplied are zeroed in v.
+typedef float stepx4u __attribute__((ext_vector_type(4), aligned(4)));
+constexpr unsigned kNnPitch = 36;  // 32 k and four floats of padding: fragment reads of 16 columns cover all banks
+
+template <int TILES, int WAVES, int EPI, bool MASKED>
+__global__ __launch_bounds__(64 * WAVES) void skinny_nn_deep_kernel(unsigned M, unsigned H, unsigned B, NnOperand op0,
+                                                                    NnOperand op1, const float* __restrict__ bias,
+                                                                    float beta, int mode, float* __restrict__ fx,
+                                                                    float* __restrict__ partial) {
+  constexpr unsigned ROWS = 32 * TILES;
+  constexpr unsigned LDS = WAVES * 32 * (kNnPitch > TILES * kStepPitchR ? kNnPitch : TILES * kStepPitchR);
+  __shared__ __attribute__((aligned(16))) float red[LDS];
+  const unsigned RP = (M + ROWS - 1) / ROWS;  // rows past the end are computed on the last row and dropped
+  const unsigned rp = blockIdx.x % RP, ct = blockIdx.x / RP;
+  const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64;
+  const unsigned l32 = lane % 32, lhi = lane / 32;
+  const float bias_row = EPI == kNnAxpby ? 0.f : bias[min(rp * ROWS + threadIdx.x % ROWS, M - 1)];
+  unsigned row[TILES], vcol[4];
+  stepx16 acc[TILES];
+#pragma unroll
+  for (int t = 0; t < TILES; ++t) {
+    row[t] = min(rp * ROWS + 32 * t + l32, M - 1);
+    acc[t] = stepx16{0};
+  }
+#pragma unroll
+  for (unsigned i = 0; i < 4; ++i) vcol[i] = min(ct * 32 + 8 * i + lane / 8, B - 1);  // past the batch: dropped
+  const unsigned C0 = (op0.K + 31) / 32, C = C0 + (op1.K + 31) / 32;
+  const unsigned part = blockIdx.y * WAVES + wave, parts = gridDim.y * WAVES;
+  const unsigned lo = C * part / parts, hi = C * (part + 1) / parts;
+  float* const mine = red + wave * 32 * kNnPitch;
+
+  float a[2][2][TILES][8];  // [buffer][step of 16 k]
+  stepx4u v[4], mk[4];
+  unsigned fresh;  // the first k of the chunk in v that counts
+#define DYHIP_NN_LOAD(buf, chunk)                                                                                     \
+  do {                                                                                                                \
+    const unsigned c_ = (chunk);                                                                                      \
+    const bool one = c_ < C0;                                                                                         \
+    const float* W = one ? op0.W : op1.W;                                                                             \
+    const float* x = one ? op0.v : op1.v;                                                                             \
+    const float* m = one ? op0.mask : op1.mask;                                                                       \
+    const size_t ldw = one ? op0.ldw : op1.ldw, ldv = one ? op0.ldv : op1.ldv, ldm = one ? op0.ldm : op1.ldm;         \
+    const unsigned K = one ? op0.K : op1.K, want = 32 * (one ? c_ : c_ - C0), k0 = min(want, K - 32);                 \
+    fresh = want - k0;                                                                                                \
+    _Pragma("unroll") for (unsigned i = 0; i < 4; ++i) {                                                              \
+      v[i] = *reinterpret_cast<const stepx4u*>(x + size_t(vcol[i]) * ldv + k0 + 4 * (lane % 8));                      \
+      if (MASKED) mk[i] = *reinterpret_cast<const stepx4u*>(m + size_t(vcol[i]) * ldm + k0 + 4 * (lane % 8));         \
+    }                                                                                                                 \
+    const float* pw = W + size_t(k0 + 8 * lhi) * ldw;                                                                 \
+    _Pragma("unroll") for (int q = 0; q < 2; ++q)                                                                     \
+      _Pragma("unroll") for (int j = 0; j < 8; ++j)                                                                   \
+        _Pragma("unroll") for (int t = 0; t < TILES; ++t) a[buf][q][t][j] = pw[size_t(16 * q + j) * ldw + row[t]];    \
+  } while (0)
+  if (lo < hi) {
+    DYHIP_NN_LOAD(0, lo);
+    for (unsigned c = lo; c < hi; c += 2) {
+#pragma unroll
+      for (unsigned r = 0; r < 2; ++r) {
+        if (r > 0 && c + r >= hi) break;
+#pragma unroll
+        for (unsigned i = 0; i < 4; ++i) {
+          stepx4u x = v[i];
+          if (MASKED) x *= mk[i];
+          if (fresh != 0) {  // uniform
+#pragma unroll
+            for (unsigned j = 0; j < 4; ++j) x[j] = 4 * (lane % 8) + j < fresh ? 0.f : x[j];
+          }
+          *reinterpret_cast<float4*>(mine + (8 * i + lane / 8) * kNnPitch + 4 * (lane % 8)) = make_float4(x[0], x[1], x[2], x[3]);
+        }
+        DYHIP_NN_LOAD(r ^ 1, min(c + r + 1, hi - 1));  // past the range its last chunk again: the compiler counts loads in flight
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+          Split3 fa[TILES], fb;
+          const float4* pb = reinterpret_cast<const float4*>(mine + l32 * kNnPitch + 16 * q + 8 * lhi);
+          fb.from(pb[0], pb[1]);
+#pragma unroll
+          for (int t = 0; t < TILES; ++t)
+            fa[t].from(make_float4(a[r][q][t][0], a[r][q][t][1], a[r][q][t][2], a[r][q][t][3]),
+                       make_float4(a[r][q][t][4], a[r][q][t][5], a[r][q][t][6], a[r][q][t][7]));
+#define DYHIP_NN_MMA(x, y)                                                    \
+  _Pragma("unroll") for (int t = 0; t < TILES; ++t) acc[t] =                  \
+      __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[t].x, fb.y, acc[t], 0, 0, 0);
+          DYHIP_NN_MMA(l, h) DYHIP_NN_MMA(h, l) DYHIP_NN_MMA(m, m) DYHIP_NN_MMA(m, h) DYHIP_NN_MMA(h, m) DYHIP_NN_MMA(h, h)
+#undef DYHIP_NN_MMA
+        }
+        __builtin_amdgcn_wave_barrier();
+      }
+    }
+  }
+#undef DYHIP_NN_LOAD
+  __syncthreads();  // the partial sums take the operands' place
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    const unsigned i = 8 * (r / 4) + 4 * lhi + (r % 4);
+#pragma unroll
+    for (int t = 0; t < TILES; ++t) red[(wave * ROWS + 32 * t + i) * kStepPitchR + l32] = acc[t][r];
+  }
+  __syncthreads();
+#pragma unroll
+  for (unsigned o = threadIdx.x; o < ROWS * 32; o += 64 * WAVES) {
+    const unsigned orow = o % ROWS, col = o / ROWS, erow = rp * ROWS + orow, ecol = ct * 32 + col;
+    if (ecol >= B || erow >= M) continue;
+    float t = red[orow * kStepPitchR + col];
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w) t += red[(w * ROWS + orow) * kStepPitchR + col];
+    if (not_finite(t)) {  // formed again without the parts: see split3.h
+      t = 0.f;
+      const unsigned c0 = C * blockIdx.y / gridDim.y, c1 = C * (blockIdx.y + 1) / gridDim.y;  // this block's chunks
+      for (int which = 0; which < 2; ++which) {
+        const NnOperand& op = which == 0 ? op0 : op1;
+        const unsigned before = which == 0 ? 0 : C0;
+        const unsigned k0 = min(32 * (max(c0, before) - before), op.K), k1 = min(32 * (max(c1, before) - before), op.K);
+        const float* x = op.v + size_t(ecol) * op.ldv;
+        const float* m = MASKED ? op.mask + size_t(ecol) * op.ldm : nullptr;
+#pragma unroll 4
+        for (unsigned k = k0; k < k1; ++k) t = fmaf(op.W[erow + size_t(k) * op.ldw], MASKED ? x[k] * m[k] : x[k], t);
+      }
+    }
+    if (partial != nullptr) {
+      partial[(size_t(blockIdx.y) * B + ecol) * M + erow] = t;
+      continue;
+    }
+    float* out = fx + size_t(ecol) * M + erow;
+    if (EPI == kNnGates) {
+      float pre = bias_row;
+      if (erow >= H && erow < 2 * H) pre += 1.0f;  // forget-gate bias
+      pre += t;
+      *out = erow < 3 * H ? logistic(mode, pre) : tanh_accurate(pre);
+    } else {
+      if (EPI == kNnBias) t += bias_row;
+      else if (beta != 0.f) t += beta * *out;
+      *out = t;
+    }
+  }
+}
+
 // 32-row blocks as long as they do not outnumber the CUs (gates forward, I = H = 1024: B = 20 13.9 us against 25 us
 // with 64-row blocks and 17.0 us for the two-launch small-batch product; B = 64 15.4 against 23.7 us; I = H = 2048,
 // B = 20 32.4 against 42.3 and 36.6 us; more blocks than CUs lose: B = 96 39.3 against 24.4 us, B = 128 39.8 against
 // 25.7 us).  Not for a block that would walk more than 2 MB of weights alone (a few rows over a very long depth), nor
 // for odd depths (v's fragments are 128-bit loads along k, or two 64-bit ones).
+//
+// skinny_nn_deep_kernel from a depth of 512 (384 in all at 256 + 128, H = 256: nothing gained) while its blocks are one
+// round of the CUs (us in a graph, before and after): gates forward, I = H = 650, B = 20 with dropout 16.3 -> 11.4
+// (three launches, now two: three blocks share the depth), I = H = 1024, B = 64 14.8 -> 14.8, B = 128 23.4 -> 22.4,
+// I = H = 512, B = 32 8.6 -> 7.8; affine 1024 x 64 x 1024 8.3 -> 7.7, 2000 x 20 x 4096 23.4 -> 14.3 (four blocks share
+// the depth), 10 000 x 32 x 1024 14.8 -> 14.6.  More blocks than CUs lose: 10 000 x 64 x 512 18.6 -> 19.0.  Bound by what
+// a CU can have in flight towards the Infinity Cache (20-25 GB/s of weights a CU): only more CUs a weight help.
+constexpr size_t kNnDeep = 512;
+
 int skinny_nn_gemm(dyhip_device* dev, size_t M, size_t N, int nseg, const GemmSeg* segs, float* C, const GemmEpiParams& epi,
-                   bool* taken) {
+                   bool* taken, const NnMask* masks) {
   *taken = false;
   if (nseg < 1 || nseg > 2 || C == nullptr || N == 0 || N > 256 || M < 1 || M >= (size_t(1) << 31)) return DYHIP_OK;
   const int kind = epi.kind == kEpiLstmGates ? kNnGates : epi.kind == kEpiBias ? kNnBias : epi.kind == kEpiAxpby ? kNnAxpby : -1;
@@ -857,11 +1014,39 @@ int skinny_nn_gemm(dyhip_device* dev, size_t M, size_t N, int nseg, const GemmSe
   const unsigned blocks64 = cdiv<unsigned>(unsigned(M), 64) * ct;
   const unsigned tiles = blocks64 <= cus / 2 ? 1 : 2;
   if (size_t(32) * tiles * Kt * sizeof(float) > (size_t(2) << 20)) return DYHIP_OK;
-  const NnOperand op0{segs[0].A, segs[0].B, unsigned(segs[0].K), segs[0].lda, segs[0].ldb};
-  const NnOperand op1 = nseg > 1 ? NnOperand{segs[1].A, segs[1].B, unsigned(segs[1].K), segs[1].lda, segs[1].ldb}
-                                 : NnOperand{segs[0].A, segs[0].B, 0u, segs[0].lda, segs[0].ldb};
+  const NnMask none{nullptr, 0}, &m0 = masks != nullptr ? masks[0] : none, &m1 = masks != nullptr ? masks[nseg - 1] : none;
+  const NnOperand op0{segs[0].A, segs[0].B, unsigned(segs[0].K), segs[0].lda, segs[0].ldb, m0.p, m0.ld};
+  const NnOperand op1 = nseg > 1 ? NnOperand{segs[1].A, segs[1].B, unsigned(segs[1].K), segs[1].lda, segs[1].ldb, m1.p, m1.ld}
+                                 : NnOperand{segs[0].A, segs[0].B, 0u, segs[0].lda, segs[0].ldb, m0.p, m0.ld};
   const dim3 grid(cdiv<unsigned>(unsigned(M), 32 * tiles) * ct), block(256);
   const float beta = kind == kNnAxpby ? epi.beta : 0.f;
+  if (Kt >= kNnDeep && segs[0].K >= 32 && segs[nseg - 1].K >= 32 && grid.x <= cus) {
+    // Few blocks: the depth over several of them, whose slices a second launch adds up.  The host pays for that launch
+    // too, so only where it is worth much, or where the masks have saved two.
+    const size_t least = masks != nullptr ? 384 : 1024;
+    unsigned splits = 1;
+    while (grid.x * (splits + 1) <= cus && Kt / (splits + 1) >= least) ++splits;
+    if (dev->gemm_ws == nullptr || dev->gemm_ws_bytes < sizeof(float) * M * N * splits) splits = 1;
+    float* const partial = splits > 1 ? static_cast<float*>(dev->gemm_ws) : nullptr;
+#define DYHIP_NN_DEEP(T, E, MK)                                                                                          \
+  hipLaunchKernelGGL((skinny_nn_deep_kernel<T, 8, E, MK>), dim3(grid.x, splits), dim3(512), 0, dev->stream, unsigned(M), epi.H, \
+                     unsigned(N), op0, op1, epi.bias, beta, epi.logistic_mode, C, partial)
+#define DYHIP_NN_DEEP_T(T)                                             \
+  do {                                                                 \
+    if (masks != nullptr) DYHIP_NN_DEEP(T, kNnGates, true);            \
+    else if (kind == kNnGates) DYHIP_NN_DEEP(T, kNnGates, false);      \
+    else if (kind == kNnBias) DYHIP_NN_DEEP(T, kNnBias, false);        \
+    else DYHIP_NN_DEEP(T, kNnAxpby, false);                            \
+  } while (0)
+    if (tiles == 1) DYHIP_NN_DEEP_T(1);
+    else DYHIP_NN_DEEP_T(2);
+#undef DYHIP_NN_DEEP_T
+#undef DYHIP_NN_DEEP
+    DYHIP_CHECK_LAUNCH();
+    *taken = true;
+    return splits > 1 ? gemm_slices_sum(dev, M, N, splits, partial, C, epi) : DYHIP_OK;
+  }
+  if (masks != nullptr) return DYHIP_OK;
 #define DYHIP_SKINNY_NN_B(T, E, BB)                                                                                 \
   hipLaunchKernelGGL((skinny_nn_kernel<T, E, BB>), grid, block, 0, dev->stream, unsigned(M), epi.H, unsigned(N), op0, op1, \
                      epi.bias, beta, epi.logistic_mode, C)
@@ -1342,10 +1527,17 @@ int dyhip_lstm_gates_forward(dyhip_device* dev, unsigned num_inputs, const float
   char* wsp = static_cast<char*>(ws);
   float* xbuf = reinterpret_cast<float*>(wsp);
   float* hbuf = reinterpret_cast<float*>(wsp + ((num_inputs > 1 || gi.dropout) ? align256(sizeof(float) * size_t(gi.I) * B) : 0));
+  const size_t G = size_t(4) * H;
+  if (gi.dropout && num_inputs == 1 && B >= 5) {  // the product reads x, h and their masks itself, if it is one for it
+    const NnMask masks[2] = {{mask_x, mask_x_bd > 1 ? gi.I : 0u}, {mask_h, mask_h_bd > 1 ? H : 0u}};
+    const GemmSeg segs[2] = {{Wx, G, xs_host[0], gi.I, gi.I}, {Wh, G, h_tm1, H, H}};
+    bool taken = false;
+    DYHIP_CHECK_STATUS(skinny_nn_gemm(dev, G, B, 2, segs, fx, GemmEpiParams{kEpiLstmGates, 0.f, b, H, logistic_mode}, &taken, masks));
+    if (taken) return DYHIP_OK;
+  }
   const float *x_eff = nullptr, *h_eff = nullptr;
   DYHIP_CHECK_STATUS(prepare_x(dev, num_inputs, xs_host, x_dims_host, gi.I, B, mask_x, mask_x_bd, xbuf, &x_eff));
   DYHIP_CHECK_STATUS(prepare_h(dev, H, B, h_tm1, mask_h, mask_h_bd, hbuf, &h_eff));
-  const size_t G = size_t(4) * H;
   // gemm_run picks the form: up to four columns (the un-batched graph, decoding) the matrix-times-vector kernels,
   // whose second kernel adds the depth slabs with the gates' epilogue (I = H = 1024, one column: 22 -> 9.4 us); from
   // five columns the one-launch fragment-order kernel on the operands as they lie (see skinny_nn_gemm)

@@ -47,6 +47,21 @@ __device__ __forceinline__ void split3_pair(float a, float b, unsigned& h, unsig
   l = __builtin_bit_cast(unsigned, __builtin_convertvector(floatx2{a, b}, bf16x2));
 }
 
+// eight floats -> the fragments of their three parts
+struct Split3 {
+  bf16x8 h, m, l;
+  __device__ __forceinline__ void from(const float4& x, const float4& y) {
+    uint4 ph, pm, pl;
+    split3_pair(x.x, x.y, ph.x, pm.x, pl.x);
+    split3_pair(x.z, x.w, ph.y, pm.y, pl.y);
+    split3_pair(y.x, y.y, ph.z, pm.z, pl.z);
+    split3_pair(y.z, y.w, ph.w, pm.w, pl.w);
+    h = __builtin_bit_cast(bf16x8, ph);
+    m = __builtin_bit_cast(bf16x8, pm);
+    l = __builtin_bit_cast(bf16x8, pl);
+  }
+};
+
 __device__ __forceinline__ bool not_finite(float x) { return !(x - x == 0.f); }
 __device__ __forceinline__ bool not_finite(const float4& v) {
   return !((v.x - v.x) + (v.y - v.y) + (v.z - v.z) + (v.w - v.w) == 0.f);

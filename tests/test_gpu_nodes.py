@@ -667,6 +667,67 @@ def test_lstm_cell_forward_backward(dev, I, H, B, dims, dropout, mask_full):
                          floor=max(1.0, float(floors[i])))
 
 
+# The gates' product over a depth of 512 and more: depths that are and are not whole chunks of 32 k, columns and rows past
+# the end of a tile, 32- and 64-row blocks, the depth over one block and over several, masks a column and one for all.
+@pytest.mark.parametrize("I,H,B,dropout,mask_full", [
+    (256, 256, 5, False, True), (34, 490, 33, False, True), (480, 32, 7, True, True), (650, 650, 20, True, True),
+    (650, 650, 20, True, False), (62, 514, 40, True, True), (1024, 1024, 20, False, True), (1024, 1024, 128, True, True),
+    (1024, 1024, 130, True, False), (30, 600, 9, True, True),
+])
+def test_gates_over_a_deep_sum(dev, I, H, B, dropout, mask_full):
+    """Forward against the CPU path and fp64; dx and dh, which are added under the mask, against fp64.  Tolerances as in
+    test_lstm_cell_forward_backward."""
+    rng = np.random.default_rng(I + H + B)
+    x, h, c_prev, Wx, Wh, b = _lstm_case(rng, I, H, B)
+    mx = mh = None
+    kw, o_kw = {}, {}
+    if dropout:
+        mbd = B if mask_full else 1
+        mx, mh = f32(rng.integers(0, 2, (mbd, I)) * 0.9), f32(rng.integers(0, 2, (mbd, H)) * 0.8)
+        kw = dict(mask_x=dev.tensor(mx), mask_x_bd=mbd, mask_h=dev.tensor(mh), mask_h_bd=mbd)
+        o_kw = dict(mask_x=mx, mask_x_bd=mbd, mask_h=mh, mask_h_bd=mbd)
+    xt, ht, Wxt, Wht, bt = (dev.tensor(a) for a in (x, h, Wx, Wh, b))
+    fx = dev.empty((B, 4 * H))
+    dev.lstm_gates_forward([xt], [I], H, B, ht, Wxt, Wht, bt, fx, **kw)
+    ref = orc.lstm_gates_forward([x], [I], H, B, h, Wx, Wh, b, **o_kw)
+    scale = float(np.sqrt(I + H) * max(rms(Wx), rms(Wh)))
+    assert_close(fx.numpy(), ref, FWD_RTOL, "gates fwd", floor=max(1.0, scale))
+    g64, _, _ = _lstm_exact_step(x, h, c_prev, Wx, Wh, b, mx, mh)
+    _assert_gates_shadow(fx.numpy(), ref, g64, H, "gates fwd")
+    dgates = f32(rng.standard_normal((B, 4 * H)))
+    reft, dgt, dpre = dev.tensor(ref), dev.tensor(dgates), dev.empty((B, 4 * H))
+    dev.lstm_gates_dpre(H, B, reft, dgt, dpre)
+    d64 = dpre.numpy().astype(np.float64)
+    for i, (n, W, m) in enumerate(((I, Wx, mx), (H, Wh, mh))):
+        g0 = f32(rng.standard_normal((B, n)))
+        gt = dev.tensor(g0)
+        dev.lstm_gates_backward([xt], [I], H, B, ht, Wxt, Wht, reft, dgt, i, gt, dpre=dpre, **kw)
+        want = g0 + (d64 @ W.astype(np.float64).T) * (1.0 if m is None else m)
+        assert_close(gt.numpy(), want, GRAD_RTOL, "gates bwd arg %d" % i, floor=max(1.0, float(np.sqrt(4 * H) * rms(W))))
+
+
+@pytest.mark.parametrize("M,N,K", [(333, 9, 2100), (70, 33, 514), (1000, 20, 640)])
+def test_deep_sums_of_a_small_batch_keep_infinities_and_nans(dev, M, N, K):
+    """The affine layer where operands are infinite, NaN or next to FLT_MAX: what fp32 arithmetic gives."""
+    rng = np.random.default_rng(M)
+    W, x, b = f32(rng.standard_normal((K, M))), f32(rng.standard_normal((N, K))), f32(rng.standard_normal(M))
+    W[5, 7], x[4, K - 3], W[40, 60], x[2, 5], W[11, 20] = np.inf, -np.inf, np.nan, 0.0, 3.4e38
+    x[:, 11] *= 1e-3
+    y = dev.empty((N, M))
+    dev.affine_forward(M, N, K, dev.tensor(b), dev.tensor(W), dev.tensor(x), y)
+    with np.errstate(all="ignore"):
+        want = x.astype(np.float64) @ W.astype(np.float64) + b
+    y = y.numpy()
+    assert np.array_equal(np.isnan(y), np.isnan(want))
+    inf = np.isinf(want)
+    assert inf.any() and np.array_equal(np.isinf(y), inf) and np.array_equal(y[inf], want[inf].astype(np.float32))
+    fin = np.isfinite(want)
+    fin[:, 20] = False
+    assert_close(y[fin], want[fin], FWD_RTOL, "finite outputs", floor=np.sqrt(K))
+    col = np.isfinite(want[:, 20])
+    assert_close(y[col, 20], want[col, 20], FWD_RTOL, "the column of the huge value")
+
+
 def test_fused_nodes_equal_unfused_path_over_three_steps(dev):
     """tests/test-rnn.cc:155-184,214-243: gates/C/H equal affine -> logistic/tanh -> cmult."""
     rng = np.random.default_rng(9)
