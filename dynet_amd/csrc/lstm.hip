@@ -40,15 +40,28 @@ __global__ __launch_bounds__(256) void rows_copy_mask_kernel(unsigned rows, unsi
   }
 }
 
-// out[b*rows + r] += tmp[b*rows + r] * mask[(mask_b ? b : 0)*mask_ld + off + r]
-__global__ __launch_bounds__(256) void acc_mul_mask_kernel(unsigned rows, unsigned mask_ld, unsigned off,
-                                                           const float* __restrict__ tmp,
+// out[b*rows + r] += (slices[0] + slices[1] + ...)[b*rows + r] * mask[(mask_b ? b : 0)*mask_ld + off + r]; slices of
+// rows * B floats, added in ascending order
+__global__ __launch_bounds__(256) void acc_mul_mask_kernel(unsigned rows, unsigned mask_ld, unsigned off, unsigned splits,
+                                                           const float* __restrict__ slices,
                                                            const float* __restrict__ mask, int mask_b,
                                                            float* __restrict__ out, unsigned B) {
   const unsigned r = blockIdx.x * 256 + threadIdx.x;
   if (r >= rows) return;
-  for (unsigned b = blockIdx.y; b < B; b += gridDim.y)
-    out[size_t(b) * rows + r] += tmp[size_t(b) * rows + r] * mask[size_t(mask_b ? b : 0) * mask_ld + off + r];
+  for (unsigned b = blockIdx.y; b < B; b += gridDim.y) {
+    const size_t e = size_t(b) * rows + r;
+    const float m = mask[size_t(mask_b ? b : 0) * mask_ld + off + r], old = out[e];  // fetched beside the slices
+    float s = 0.f;
+    for (unsigned k0 = 0; k0 < splits; k0 += 8) {  // eight slices in flight
+      float v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = slices[size_t(min(k0 + u, splits - 1)) * rows * B + e];
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        if (k0 + u < splits) s += v[u];
+    }
+    out[e] = old + s * m;
+  }
 }
 
 // dpre[i, b] = i < 3H ? d*f*(1-f) : d*(1-f*f)      (dynet/nodes-lstm.cc:358-361)
@@ -1618,9 +1631,21 @@ int dyhip_lstm_gates_backward(dyhip_device* dev, unsigned num_inputs, const floa
       if (taken) return DYHIP_OK;
     }
     if (!gi.dropout) return gemm_run(dev, true, true, rows, B, 1, &s, dEdxi, acc);
-    DYHIP_CHECK_STATUS(gemm_run(dev, true, true, rows, B, 1, &s, tmp, ovw));
+    // the product's slices are added up where the mask is applied; one in tmp if the device's workspace holds none
+    const float* slices = tmp;
+    unsigned splits = 1;
+    if (dev->gemm_ws != nullptr && dev->gemm_ws_bytes >= sizeof(float) * size_t(rows) * B) {
+      GemmEpiParams parts{kEpiPartials, 0.f, nullptr, 0, 0};
+      parts.partials = static_cast<float*>(dev->gemm_ws);
+      parts.partials_bytes = dev->gemm_ws_bytes;
+      parts.splits_out = &splits;
+      DYHIP_CHECK_STATUS(gemm_run(dev, true, true, rows, B, 1, &s, nullptr, parts));
+      slices = parts.partials;
+    } else {
+      DYHIP_CHECK_STATUS(gemm_run(dev, true, true, rows, B, 1, &s, tmp, ovw));
+    }
     hipLaunchKernelGGL(acc_mul_mask_kernel, dim3(cdiv<unsigned>(rows, 256), grid_y(B)), dim3(256), 0, dev->stream, rows,
-                       mask_ld, off, tmp, mask, mask_bd > 1 ? 1 : 0, dEdxi, B);
+                       mask_ld, off, splits, slices, mask, mask_bd > 1 ? 1 : 0, dEdxi, B);
     DYHIP_CHECK_LAUNCH();
     return DYHIP_OK;
   }
