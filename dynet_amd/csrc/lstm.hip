@@ -511,6 +511,104 @@ __global__ __launch_bounds__(256 * TILES) void lstm_step_fwd_kernel(unsigned H, 
   if (hp != nullptr) hp[((size_t(ct) * (H / 8) + TILES * rp + tile) * 64 + (u / 4) * 32 + col) * 4 + u % 4] = hv * mh;
 }
 
+// The same timestep for up to 16 columns: half a row tile a block, four hidden units, so that twice the CUs fetch weights.
+// At one column (H = 1024, depth 2048) the kernel above keeps 128 CUs busy, and a CU gets no more than 20-25 GB/s of
+// weights from beyond its L2 however much it has in flight.  Eight wavefronts deal the depth of both products among them in
+// steps of 16 k (sixteen take 0.5-1.2 us longer to start and to meet); v_mfma_f32_16x16x4_f32, rows gate*4 + unit.  Lane
+// 16*lq + l16 of a step holds k = 4*lq + s, s = 0..3, of row (column) l16: group lq/2, half lq%2 of the packed order above.
+// Blocks of the two halves of a tile are eight apart: the same XCD.
+// us in a graph, before and after, plain states, I = 256: H = 512, B = 4 6.1 -> 4.3; H = 768, B = 16 7.6 -> 5.7;
+// H = 1024, B = 1 8.5 -> 6.8, B = 16 8.8 -> 8.0.  Two column tiles lose: H = 1024, B = 32 9.6 -> 11.5.
+typedef float stepx4 __attribute__((ext_vector_type(4)));
+
+template <bool PLAIN>
+__global__ __launch_bounds__(512) void lstm_step_fwd_small_kernel(unsigned H, unsigned B, StepOperand op0, StepOperand op1,
+                                                                   const float* xproj, const float* __restrict__ bias,
+                                                                   const float* __restrict__ c_prev, int mode, float* gates,
+                                                                   float* __restrict__ c, float* __restrict__ h,
+                                                                   float* __restrict__ hp, const float* __restrict__ mask_h) {
+  constexpr int WAVES = 8, COLS = 16, PITCH = COLS + 1;
+  constexpr unsigned RAW = 8;  // steps in flight
+  __shared__ float red[WAVES * 16 * PITCH];
+  __shared__ float sums[16 * PITCH];
+  const unsigned rt = blockIdx.x / 16 * 8 + blockIdx.x % 8, half = blockIdx.x / 8 % 2;
+  const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64;
+  const unsigned l16 = lane % 16, lq = lane / 16;
+
+  // operands of the cell update, one thread per (unit, column), fetched under the product
+  const unsigned u = threadIdx.x % 4, col = threadIdx.x / 4 % COLS, ej = rt * 8 + half * 4 + u;
+  const unsigned lcol = min(col, B - 1);  // past the batch: clamped, dropped
+  float bq[4], xq[4], cp = 0.f, mh = 1.f;
+  if (threadIdx.x < 4 * COLS) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      bq[q] = bias[q * H + ej];
+      xq[q] = xproj != nullptr ? xproj[size_t(lcol) * 4 * H + ej + size_t(q) * H] : 0.f;
+    }
+    if (c_prev != nullptr) cp = c_prev[size_t(lcol) * H + ej];
+    if (mask_h != nullptr) mh = mask_h[size_t(lcol) * H + ej];
+  }
+
+  stepx4 acc = {0.f, 0.f, 0.f, 0.f};
+  const unsigned S0 = op0.Wp != nullptr ? op0.K / 16 : 0, S = S0 + (op1.Wp != nullptr ? op1.K / 16 : 0);
+  const unsigned lo = S * wave / WAVES, hi = S * (wave + 1) / WAVES;
+  if (lo < hi) {
+    const unsigned arow = l16 / 4 * 8 + half * 4 + l16 % 4;  // of the 32-row tile
+    const unsigned part = lq / 2 * 64 + lq % 2 * 32;         // of a step's two groups
+    float4 a[RAW], v[RAW];
+    const auto load = [&](unsigned r, unsigned s) {
+      const bool one = s < S0;
+      const float* Wp = one ? op0.Wp : op1.Wp;
+      const float* vp = one ? op0.vp : op1.vp;
+      const unsigned K = one ? op0.K : op1.K, G = K / 8, g = 2 * (one ? s : s - S0);
+      a[r] = *reinterpret_cast<const float4*>(Wp + ((size_t(rt) * G + g) * 64 + part + arow) * 4);
+      v[r] = *reinterpret_cast<const float4*>(PLAIN ? vp + size_t(min(l16, B - 1)) * K + 8 * g + 4 * lq
+                                                    : vp + (size_t(g) * 64 + part + l16) * 4);
+    };
+#pragma unroll
+    for (unsigned r = 0; r < RAW; ++r) load(r, min(lo + r, hi - 1));
+    __builtin_amdgcn_sched_barrier(0);
+    for (unsigned s = lo; s < hi; s += RAW) {
+      const bool more = s + RAW < hi;  // uniform
+#pragma unroll
+      for (unsigned r = 0; r < RAW; ++r) {
+        if (s + r >= hi) break;
+#define STEP_MMA(x) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[r].x, v[r].x, acc, 0, 0, 0);
+        STEP_MMA(x) STEP_MMA(y) STEP_MMA(z) STEP_MMA(w)
+#undef STEP_MMA
+        if (more) load(r, min(s + RAW + r, hi - 1));
+      }
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r) red[(wave * 16 + 4 * lq + r) * PITCH + l16] = acc[r];
+  __syncthreads();
+  if (threadIdx.x < 16 * COLS) {
+    const unsigned row = threadIdx.x / COLS, cc = threadIdx.x % COLS;
+    float t = red[row * PITCH + cc];
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w) t += red[(w * 16 + row) * PITCH + cc];
+    sums[row * PITCH + cc] = t;
+  }
+  __syncthreads();
+  if (threadIdx.x >= 4 * COLS || col >= B) return;
+  float pre[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) pre[q] = (q == 1 ? bq[q] + 1.0f : bq[q]) + xq[q] + sums[(q * 4 + u) * PITCH + col];
+  const float gi = logistic(mode, pre[0]), gf = logistic(mode, pre[1]), go = logistic(mode, pre[2]);
+  const float gg = tanh_accurate(pre[3]);
+  const float cv = c_prev != nullptr ? gi * gg + gf * cp : gi * gg;
+  const float hv = go * tanh_accurate(cv);
+  const size_t g0 = size_t(col) * 4 * H + ej, s0 = size_t(col) * H + ej;
+  gates[g0] = gi;
+  gates[g0 + H] = gf;
+  gates[g0 + 2 * size_t(H)] = go;
+  gates[g0 + 3 * size_t(H)] = gg;
+  c[s0] = cv;
+  h[s0] = hv;
+  if (hp != nullptr) hp[(size_t(rt) * 64 + half * 32 + col) * 4 + u] = hv * mh;
+}
+
 // ---- single-launch backward step: recurrent product Wh^T * dpre_{t+1} and the cell backward of step t -----------
 // The mirror of lstm_step_fwd_kernel.  The output of the product is H x B with a 4H-deep sum, so a block that is to
 // run the cell backward in its epilogue must keep the whole depth: it owns 16 hidden units x 32 batch columns (256
@@ -554,8 +652,6 @@ __global__ void lstm_pack_state16_kernel(unsigned K, unsigned B, const float* __
   const unsigned col = ct * 16 + l16, k = 16 * kg + 4 * lq + s;
   vp[o] = col < B ? v[size_t(col) * K + k] : 0.f;
 }
-
-typedef float stepx4 __attribute__((ext_vector_type(4)));
 
 __global__ __launch_bounds__(512) void lstm_step_bwd_kernel(unsigned H, unsigned B, const float* __restrict__ WTp,
                                                             const float* __restrict__ dpre_next_p,
@@ -1926,6 +2022,19 @@ static int step_forward(dyhip_device* dev, unsigned I, unsigned H, unsigned B, c
   DYHIP_REQUIRE(logistic_mode == DYHIP_LOGISTIC_PACKET || logistic_mode == DYHIP_LOGISTIC_SCALAR,
                 "unknown logistic mode %d", logistic_mode);
   const StepOperand op0{packed_Wx, x, I}, op1{packed_Wh, h_tm1, H};
+  // up to 16 columns: 16 rows a block, from a depth of 256 (H = 128, depth 128: 3.4 -> 3.6 us) and while the blocks do not
+  // outnumber the CUs
+  const unsigned depth = (packed_Wx != nullptr ? I : 0) + (packed_Wh != nullptr ? H : 0);
+  if (B <= 16 && depth >= 256 && H / 4 <= unsigned(dev->num_cus > 0 ? dev->num_cus : 256)) {
+#define DYHIP_STEP_SMALL(PLAIN)                                                                                       \
+  hipLaunchKernelGGL(lstm_step_fwd_small_kernel<PLAIN>, dim3(H / 4), dim3(512), 0, dev->stream, H, B, op0, op1, xproj, b, \
+                     c_tm1, logistic_mode, gates, c, h, hp_out, mask_h)
+    if (states_packed) DYHIP_STEP_SMALL(false);
+    else DYHIP_STEP_SMALL(true);
+#undef DYHIP_STEP_SMALL
+    DYHIP_CHECK_LAUNCH();
+    return DYHIP_OK;
+  }
   // 64-row tiles (fewest operand bytes per CU) once they give half the CUs a block, 32-row tiles below that
   const unsigned blocks2 = (H / 16) * cdiv<unsigned>(B, 32);
   const bool two = blocks2 * 2 >= unsigned(dev->num_cus > 0 ? dev->num_cus : 256);

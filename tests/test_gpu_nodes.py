@@ -706,6 +706,42 @@ def test_gates_over_a_deep_sum(dev, I, H, B, dropout, mask_full):
         assert_close(gt.numpy(), want, GRAD_RTOL, "gates bwd arg %d" % i, floor=max(1.0, float(np.sqrt(4 * H) * rms(W))))
 
 
+# One timestep for up to 16 columns: a depth that gives some wavefronts nothing (H = 128 and nothing else: the kernel for
+# more columns), odd shares, packed and plain states, the batch's edge, with and without a state and a recurrent mask.
+@pytest.mark.parametrize("I,H,B", [(128, 128, 1), (384, 256, 16), (128, 640, 3), (256, 1024, 16), (1152, 384, 7)])
+def test_step_of_a_few_columns(dev, I, H, B):
+    """dyhip_lstm_step_forward_x and _packed_dropout against the CPU path and fp64, and the packed copy of h."""
+    rng = np.random.default_rng(I + H + B)
+    x, h, c_prev, Wx, Wh, b = _lstm_case(rng, I, H, B)
+    xt, ht, ct, Wxt, Wht, bt = (dev.tensor(a) for a in (x, h, c_prev, Wx, Wh, b))
+    pWx, pWh = dev.empty(4 * H * I), dev.empty(4 * H * H)
+    dev.lstm_pack_input(I, H, Wxt, pWx)
+    dev.lstm_pack_recurrent(H, Wht, pWh)
+    n = dev.lstm_packed_state_floats(H, B)
+    hp, hp_out, want_hp, xproj = dev.empty(n), dev.empty(n), dev.empty(n), dev.empty((B, 4 * H))
+    dev.lstm_pack_state(H, B, ht, hp)
+    dev.gemm_nn(4 * H, B, I, Wxt, xt, 0.0, xproj)
+    mask = f32(rng.integers(0, 2, (B, H)) * 2.0)
+    for form in ("x", "x from zero", "packed"):
+        g, c, h2 = dev.empty((B, 4 * H)), dev.empty((B, H)), dev.empty((B, H))
+        h0, c0 = (np.zeros_like(h), np.zeros_like(c_prev)) if form == "x from zero" else (h, c_prev)
+        if form == "x":
+            dev.lstm_step_forward_x(I, H, B, pWx, xt, pWh, ht, bt, ct, g, c, h2)
+        elif form == "x from zero":
+            dev.lstm_step_forward_x(I, H, B, pWx, xt, None, None, bt, None, g, c, h2)
+        else:
+            dev.lstm_step_forward_packed(H, B, pWh, hp, xproj, bt, ct, g, c, h2, hp_out, mask_h=dev.tensor(mask))
+        ref = orc.lstm_gates_forward([x], [I], H, B, h0, Wx, Wh, b)
+        g64, c64, h64 = _lstm_exact_step(x, h0, c0, Wx, Wh, b)
+        _assert_gates_shadow(g.numpy(), ref, g64, H, form)
+        scale = max(1.0, float(np.sqrt(I + H) * max(rms(Wx), rms(Wh))))
+        assert_close(c.numpy(), c64, FWD_RTOL, form + " c", floor=scale)
+        assert_close(h2.numpy(), h64, FWD_RTOL, form + " h", floor=scale)
+    dev.lstm_pack_state(H, B, dev.tensor(h2.numpy() * mask), want_hp)
+    cols = (np.arange(n) // 4) % 32 < B  # what lies past the batch is never read into a result
+    assert np.array_equal(hp_out.numpy()[cols], want_hp.numpy()[cols])
+
+
 @pytest.mark.parametrize("M,N,K", [(333, 9, 2100), (70, 33, 514), (1000, 20, 640)])
 def test_deep_sums_of_a_small_batch_keep_infinities_and_nans(dev, M, N, K):
     """The affine layer where operands are infinite, NaN or next to FLT_MAX: what fp32 arithmetic gives."""
