@@ -1091,10 +1091,10 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_nn_deep_kernel(unsigned M, 
 // 25.7 us).  Not for a block that would walk more than 2 MB of weights alone (a few rows over a very long depth), nor
 // for odd depths (v's fragments are 128-bit loads along k, or two 64-bit ones).
 //
-// skinny_nn_deep_kernel from a depth of 512 (384 in all at 256 + 128, H = 256: nothing gained) while its blocks are one
-// round of the CUs (us in a graph, before and after): gates forward, I = H = 650, B = 20 with dropout 16.3 -> 11.4
-// (three launches, now two: three blocks share the depth), I = H = 1024, B = 64 14.8 -> 14.8, B = 128 23.4 -> 22.4,
-// I = H = 512, B = 32 8.6 -> 7.8; affine 1024 x 64 x 1024 8.3 -> 7.7, 2000 x 20 x 4096 23.4 -> 14.3 (four blocks share
+// skinny_nn_deep_kernel from a depth of 512 (I = H = 256, B = 20: 5.8 -> 5.6, where its gain ends) while its blocks are
+// one round of the CUs (us in a graph, before and after): gates forward, I = H = 650, B = 20 with dropout 16.3 -> 11.4
+// (three launches, now two: three blocks share the depth), I = H = 1024, B = 64 14.8 -> 14.1, B = 128 23.4 -> 21.6,
+// I = H = 512, B = 32 8.6 -> 8.0; affine 1024 x 64 x 1024 8.3 -> 7.7, 2000 x 20 x 4096 23.4 -> 14.3 (four blocks share
 // the depth), 10 000 x 32 x 1024 14.8 -> 14.6.  More blocks than CUs lose: 10 000 x 64 x 512 18.6 -> 19.0.  Bound by what
 // a CU can have in flight towards the Infinity Cache (20-25 GB/s of weights a CU): only more CUs a weight help.
 constexpr size_t kNnDeep = 512;
