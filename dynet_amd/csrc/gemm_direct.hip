@@ -331,6 +331,8 @@ __global__ __launch_bounds__(64 * WAVES, 2) void gemm_direct_kernel(DirectArgs g
           }
           fs += count;
         }
+      } else if (SPLIT) {
+        v *= kSplitOut;
       }
       float* p = out + m + size_t(n) * g.M;
       if (g.partial == nullptr) {

@@ -248,6 +248,8 @@ __global__ __launch_bounds__(256, 2) void gemm_tile_kernel(TileArgs g) {
             }
             first += count;
           }
+        } else {
+          v[t] *= kSplitOut;
         }
         if (direct) {
           v[t] += bias[t];

@@ -417,6 +417,7 @@ __global__ __launch_bounds__(kWideThreads, 1) void gemm_wide_kernel(WideArgs g) 
             again |= 1u << (16 * u + r);
             continue;
           }
+          v[q].x *= kSplitOut; v[q].y *= kSplitOut; v[q].z *= kSplitOut; v[q].w *= kSplitOut;
           if (!AK) {
             const unsigned m = out_row<AK>(wm_e, 0, l32_e);
             if (m >= mlim) continue;
@@ -493,6 +494,7 @@ __global__ __launch_bounds__(kWideThreads) void gemm_wide_fixup_kernel(WideArgs 
       finish_group_fp32<AK, BKM>(g, m0, n0, tid, ur);
       continue;
     }
+    v.x *= kSplitOut; v.y *= kSplitOut; v.z *= kSplitOut; v.w *= kSplitOut;
     if (!AK) {
       const unsigned m = out_row<AK>(wm, 0, l32);
       if (m >= mlim) continue;

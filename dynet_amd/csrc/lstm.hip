@@ -1066,6 +1066,8 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_nn_deep_kernel(unsigned M, 
 #pragma unroll 4
         for (unsigned k = k0; k < k1; ++k) t = fmaf(op.W[erow + size_t(k) * op.ldw], MASKED ? x[k] * m[k] : x[k], t);
       }
+    } else {
+      t *= kSplitOut;
     }
     if (partial != nullptr) {
       partial[(size_t(blockIdx.y) * B + ecol) * M + erow] = t;

@@ -10,10 +10,13 @@
 // of the depth cost six additions into the accumulator where v_mfma_f32_32x32x2_f32 makes sixteen.  Measured against
 // fp64, the sums are as close as the fp32 instruction's or closer (the tests check both).
 //
-// bf16 has the exponent range of fp32, and the bf16 instructions keep subnormal inputs and results.  Values whose top
-// part rounds beyond the largest bf16 (the last 2^-9 below FLT_MAX), infinities and NaNs come out of a split as
+// The smallest bf16 value is 2^-133, so the parts of x hold all of it only if its last bit is at least that: |x| >= 2^-110.
+// fp32 values reach down to 2^-149 (probabilities of a confident softmax are that small), so every operand is multiplied
+// by 2^16 on its way into the parts, exactly, and a sum by 2^-32 on its way out: all fp32 values are then split exactly,
+// subnormals included (at 2^-120, unscaled, a product was off by 4e-5, below 2^-134 it was zero).  The bf16 instructions
+// keep subnormal inputs and results.  Infinities, NaNs, operands from 2^111 on and sums from 2^96 on come out as
 // non-finite sums; the kernels form such an output again with plain fp32 multiply-adds (dot_fp32), so that infinities
-// keep their sign and values next to FLT_MAX their value.
+// keep their sign and huge values their value.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -26,7 +29,10 @@ typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float floatx2 __attribute__((ext_vector_type(2)));
 
-// Two floats -> their bf16 parts, packed (first value in the low half): 7 instructions.  What is left of a value is the
+constexpr float kSplitIn = 65536.f;                // of an operand on its way into its parts
+constexpr float kSplitOut = 1.f / (65536.f * 65536.f);  // of a sum of products of parts
+
+// Two floats -> the bf16 parts of 2^16 times them, packed (first value in the low half): 9 instructions.  What is left of a value is the
 // two-term dot product v + p.lo * s.lo + p.hi * s.hi with a selector s that takes one part of the pair away: one
 // instruction where shift (or mask) and subtraction are two (11 instructions a pair; a loop of splits 1470 -> 1130 us).
 // The difference is exact, subnormals included, so that the parts are the same bit for bit.  The other part is
@@ -38,6 +44,8 @@ __device__ __forceinline__ float take_away(unsigned parts, unsigned selector, fl
 
 __device__ __forceinline__ void split3_pair(float a, float b, unsigned& h, unsigned& m, unsigned& l) {
   constexpr unsigned kLow = 0x8000BF80u, kHigh = 0xBF808000u;  // (-1, -0) and (-0, -1), low half first
+  a *= kSplitIn;
+  b *= kSplitIn;
   h = __builtin_bit_cast(unsigned, __builtin_convertvector(floatx2{a, b}, bf16x2));
   a = take_away(h, kLow, a);
   b = take_away(h, kHigh, b);
@@ -47,7 +55,7 @@ __device__ __forceinline__ void split3_pair(float a, float b, unsigned& h, unsig
   l = __builtin_bit_cast(unsigned, __builtin_convertvector(floatx2{a, b}, bf16x2));
 }
 
-// eight floats -> the fragments of their three parts
+// eight floats -> the fragments of the parts of 2^16 times them
 struct Split3 {
   bf16x8 h, m, l;
   __device__ __forceinline__ void from(const float4& x, const float4& y) {

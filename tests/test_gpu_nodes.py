@@ -2128,6 +2128,18 @@ def test_gemm_split_products_have_fp32_precision_over_the_exponent_range(dev, M,
         assert np.linalg.norm(err) <= 0.5 * np.sqrt(K) * 2.0 ** -24 * np.linalg.norm(exact), form
 
 
+@pytest.mark.parametrize("M,N,K", SPLIT_GEMM_SHAPES + [(1000, 20, 640)])  # the last: the deep sum of a small batch
+@pytest.mark.parametrize("e", [-112, -126, -140])
+def test_gemm_split_products_keep_the_bits_of_tiny_values(dev, M, N, K, e):
+    """Operands of the size 2^e, subnormals at 2^-140, times large ones: products of ordinary size, to the same bound as
+    above (bf16 ends at 2^-133: parts of unscaled values would leave 2^-22, 2^-8 and nothing)."""
+    rng = np.random.default_rng(M + K)
+    l, r = f32(rng.standard_normal((K, M)) * 2.0 ** e), f32(rng.standard_normal((N, K)) * 2.0 ** 100)
+    exact = r.astype(np.float64) @ l.astype(np.float64)
+    for form, y in _three_forms(dev, M, N, K, l, r, np.zeros((N, M), np.float32), 0.0):
+        assert np.linalg.norm(y - exact) <= 0.5 * np.sqrt(K) * 2.0 ** -24 * np.linalg.norm(exact), form
+
+
 @pytest.mark.parametrize("M,N,K", SPLIT_GEMM_SHAPES)
 def test_gemm_split_products_keep_infinities_nans_and_huge_values(dev, M, N, K):
     """Where an operand is infinite, NaN or rounds beyond the largest bf16, its outputs are formed by plain fp32
