@@ -12,6 +12,7 @@
 // it is contiguous along its rows.  Two steps are in flight.  Rows past the matrix are read at a clamped row and their
 // outputs dropped; a depth that is not a multiple of 16 ends in a step of clamped, zeroed loads.
 #include <algorithm>
+#include <type_traits>
 
 #include "gemm.h"
 #include "split3.h"
@@ -40,12 +41,13 @@ struct DirectArgs {
 // of row r at position c ^ (r/4 % 4) (fragment reads of 16 neighbouring rows then cover all banks); tile t is rows
 // 32*t + l32.  Stored along its rows: an instruction is 8/T k x 128*T bytes, LDS holds [k][32*T rows]; tile t is rows
 // T*l32 + t.
-template <bool KMAJOR, int T>
+// Offsets are in bytes from the tile's first row: 32 bits (Off) where a leading dimension is small enough for them.
+template <bool KMAJOR, int T, typename Off>
 struct DirectOperand {
   static constexpr int L = 2 * T;  // 128-bit loads a lane and step
   const float* base;  // the tile's first row, k = 0 (uniform)
   size_t ld;
-  size_t off[KMAJOR ? L : 1];
+  Off off[KMAJOR ? L : 1];
   unsigned K, rows;              // depth; rows inside the matrix from the tile's first
   // Groups of four rows past the matrix edge are moved to its last four rows; one that straddles the edge is shifted back
   // into place on its way to LDS.  few: fewer than four rows, every load is checked (uniform).
@@ -62,10 +64,10 @@ struct DirectOperand {
     shift = 0;
     if (KMAJOR) {
 #pragma unroll
-      for (int i = 0; i < L; ++i) off[i] = size_t(min(16u * i + lane / 4, rows - 1)) * ld + 4 * (((lane % 4) ^ (lane / 16)) % 4);
+      for (int i = 0; i < L; ++i) off[i] = 4 * (Off(min(16u * i + lane / 4, rows - 1)) * Off(ld) + 4 * (((lane % 4) ^ (lane / 16)) % 4));
     } else {
       const unsigned r0 = 4 * (lane % (8 * T)), moved = min(r0, rows >= 4 ? rows - 4 : 0u);
-      off[0] = (lane / (8 * T)) * ld + moved;
+      off[0] = 4 * (Off(lane / (8 * T)) * Off(ld) + moved);
       shift = min(r0 - moved, 3u);  // (3: a group wholly past the edge, whatever it holds)
     }
   }
@@ -73,7 +75,7 @@ struct DirectOperand {
     const float* p = base + size_t(step) * (KMAJOR ? 16 : 16 * ld);
 #pragma unroll
     for (int i = 0; i < L; ++i) {
-      v[i] = *reinterpret_cast<const float4u*>(p + off[KMAJOR ? i : 0]);
+      v[i] = *reinterpret_cast<const float4u*>(reinterpret_cast<const char*>(p) + off[KMAJOR ? i : 0]);
       if (!KMAJOR) p += (8 / T) * ld;
     }
   }
@@ -175,24 +177,21 @@ struct DirectFrags<false, T> {
   }
 };
 
-// a step's products, in two parts: four of the six bf16 products and the last two (all of the fp32 ones first)
+// A step's products.  The bf16 ones of the h parts have an accumulator of their own, the five small ones share another
+// (split3.h); the fp32 ones have one.
 template <int TM, int TN>
-__device__ __forceinline__ void direct_step_head(const DirectFrags<true, TM>& a, const DirectFrags<true, TN>& b,
-                                                 directx16 (&acc)[TN][TM]) {
-  direct_mma<TM, TN>(a.l, b.h, acc);
-  direct_mma<TM, TN>(a.h, b.l, acc);
-  direct_mma<TM, TN>(a.m, b.m, acc);
-  direct_mma<TM, TN>(a.m, b.h, acc);
-}
-template <int TM, int TN>
-__device__ __forceinline__ void direct_step_tail(const DirectFrags<true, TM>& a, const DirectFrags<true, TN>& b,
-                                                 directx16 (&acc)[TN][TM]) {
-  direct_mma<TM, TN>(a.h, b.m, acc);
+__device__ __forceinline__ void direct_step(const DirectFrags<true, TM>& a, const DirectFrags<true, TN>& b,
+                                            directx16 (&acc)[TN][TM], directx16 (&low)[TN][TM]) {
+  direct_mma<TM, TN>(a.l, b.h, low);
+  direct_mma<TM, TN>(a.h, b.l, low);
+  direct_mma<TM, TN>(a.m, b.m, low);
+  direct_mma<TM, TN>(a.m, b.h, low);
+  direct_mma<TM, TN>(a.h, b.m, low);
   direct_mma<TM, TN>(a.h, b.h, acc);
 }
 template <int TM, int TN>
-__device__ __forceinline__ void direct_step_head(const DirectFrags<false, TM>& a, const DirectFrags<false, TN>& b,
-                                                 directx16 (&acc)[TN][TM]) {
+__device__ __forceinline__ void direct_step(const DirectFrags<false, TM>& a, const DirectFrags<false, TN>& b,
+                                            directx16 (&acc)[TN][TM], directx16 (&)[TN][TM]) {
 #pragma unroll
   for (int k = 0; k < 8; ++k)
 #pragma unroll
@@ -200,11 +199,14 @@ __device__ __forceinline__ void direct_step_head(const DirectFrags<false, TM>& a
 #pragma unroll
       for (int t = 0; t < TM; ++t) acc[u][t] = __builtin_amdgcn_mfma_f32_32x32x2f32(b.x[u][k], a.x[t][k], acc[u][t], 0, 0, 0);
 }
+
+// 2 x 2 tiles: accumulators and fragments fill the registers
 template <int TM, int TN>
-__device__ __forceinline__ void direct_step_tail(const DirectFrags<false, TM>&, const DirectFrags<false, TN>&, directx16 (&)[TN][TM]) {}
+constexpr bool kDirectFull = TM * TN == 4;
 
 template <bool AK, bool BKM, int TM, int TN, int WAVES, bool SPLIT>
 __global__ __launch_bounds__(64 * WAVES, 2) void gemm_direct_kernel(DirectArgs g) {
+  using Off = std::conditional_t<kDirectFull<TM, TN>, unsigned, size_t>;
   constexpr int R = 16 * TM * TN;                  // accumulator registers a lane
   constexpr int STAGE = 512 * (TM + TN);           // floats of a wavefront's step
   constexpr int LDS = WAVES * (R * 64 > STAGE ? R * 64 : STAGE);
@@ -220,13 +222,13 @@ __global__ __launch_bounds__(64 * WAVES, 2) void gemm_direct_kernel(DirectArgs g
   const unsigned w0 = s0 + (s1 - s0) * w / WAVES, w1 = s0 + (s1 - s0) * (w + 1) / WAVES;
   float* const la = lds + w * STAGE;
   float* const lb = la + 512 * TM;
-  directx16 acc[TN][TM];
+  directx16 acc[TN][TM], low[TN][TM];
 #pragma unroll
   for (int u = 0; u < TN; ++u)
 #pragma unroll
     for (int t = 0; t < TM; ++t)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) acc[u][t][r] = 0.f;
+      for (int r = 0; r < 16; ++r) acc[u][t][r] = low[u][t][r] = 0.f;
 
   unsigned first = 0;  // first step of the segment
   for (int sg = 0; sg < g.nseg; ++sg) {
@@ -237,20 +239,24 @@ __global__ __launch_bounds__(64 * WAVES, 2) void gemm_direct_kernel(DirectArgs g
     const unsigned e = mine ? a1 - first : a0;  // this wave's steps of the segment: [a0, e)
     first += count;
     if (!mine) continue;
-    DirectOperand<AK, TM> oa;
-    DirectOperand<BKM, TN> ob;
+    DirectOperand<AK, TM, Off> oa;
+    DirectOperand<BKM, TN, Off> ob;
     oa.init(q.A + size_t(blockIdx.z) * g.stride_a, q.lda, K, m0, g.M, lane);
     ob.init(q.B + size_t(blockIdx.z) * g.stride_b, q.ldb, K, n0, g.N, lane);
-    constexpr int RAW = TM * TN == 4 ? 2 : 4;  // steps of loads in flight
+    // Steps of loads in flight, and whether a step is read from LDS when its fragments are formed or one step ahead:
+    // 2 x 2 tiles have no registers to spare beside their accumulators.
+    constexpr bool LATE = kDirectFull<TM, TN>;
+    constexpr int RAW = LATE ? 1 : 4;
     float4u ra[RAW][2 * TM], rb[RAW][2 * TN];
     float xa[TM][8], xb[TN][8];
     DirectFrags<SPLIT, TM> fa;
     DirectFrags<SPLIT, TN> fb;
     // Through LDS: write, then read; nobody else touches a wavefront's piece, and its LDS accesses stay in order.
-#define DYHIP_DIRECT_PASS(buf, checked)                  \
+#define DYHIP_DIRECT_STORE(buf, checked)                 \
   oa.template store<checked>(la, ra[buf], lane);         \
   ob.template store<checked>(lb, rb[buf], lane);         \
-  __builtin_amdgcn_wave_barrier();                       \
+  __builtin_amdgcn_wave_barrier();
+#define DYHIP_DIRECT_READ                                \
   oa.read(xa, la, l32, lhi);                             \
   ob.read(xb, lb, l32, lhi);                             \
   __builtin_amdgcn_wave_barrier();
@@ -263,20 +269,22 @@ __global__ __launch_bounds__(64 * WAVES, 2) void gemm_direct_kernel(DirectArgs g
   ob.load(rb[buf], min((s), full - 1));
 #pragma unroll
       for (int r = 0; r < RAW; ++r) { DYHIP_DIRECT_LOAD(r, a0 + r) }
-      DYHIP_DIRECT_PASS(0, false)
+      DYHIP_DIRECT_STORE(0, false)
+      if (!LATE) { DYHIP_DIRECT_READ }
       DYHIP_DIRECT_LOAD(0, a0 + RAW)
       for (unsigned s = a0; s < full; s += RAW) {
 #pragma unroll
         for (int r = 0; r < RAW; ++r) {
           if (r > 0 && s + r >= full) break;
           constexpr int NB = RAW - 1;
+          if (LATE) { DYHIP_DIRECT_READ }
           fa.from(xa);
           fb.from(xb);
           __builtin_amdgcn_sched_barrier(0);
-          DYHIP_DIRECT_PASS((r + 1) & NB, false)
+          DYHIP_DIRECT_STORE((r + 1) & NB, false)
+          if (!LATE) { DYHIP_DIRECT_READ }
           DYHIP_DIRECT_LOAD((r + 1) & NB, s + r + 1 + RAW)
-          direct_step_head<TM, TN>(fa, fb, acc);
-          direct_step_tail<TM, TN>(fa, fb, acc);
+          direct_step<TM, TN>(fa, fb, acc, low);
           __builtin_amdgcn_sched_barrier(0);
         }
       }
@@ -285,13 +293,14 @@ __global__ __launch_bounds__(64 * WAVES, 2) void gemm_direct_kernel(DirectArgs g
     for (unsigned s = full; s < e; ++s) {
       oa.load_checked(ra[0], s, lane);
       ob.load_checked(rb[0], s, lane);
-      DYHIP_DIRECT_PASS(0, true)
+      DYHIP_DIRECT_STORE(0, true)
+      DYHIP_DIRECT_READ
       fa.from(xa);
       fb.from(xb);
-      direct_step_head<TM, TN>(fa, fb, acc);
-      direct_step_tail<TM, TN>(fa, fb, acc);
+      direct_step<TM, TN>(fa, fb, acc, low);
     }
-#undef DYHIP_DIRECT_PASS
+#undef DYHIP_DIRECT_STORE
+#undef DYHIP_DIRECT_READ
   }
 
   __syncthreads();
@@ -300,7 +309,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void gemm_direct_kernel(DirectArgs g
 #pragma unroll
     for (int t = 0; t < TM; ++t)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) lds[((w * TN + u) * TM + t) * 1024 + r * 64 + lane] = acc[u][t][r];
+      for (int r = 0; r < 16; ++r) lds[((w * TN + u) * TM + t) * 1024 + r * 64 + lane] = SPLIT ? acc[u][t][r] + low[u][t][r] : acc[u][t][r];
   __syncthreads();
   // wavefront w finishes 16 * TN / WAVES groups of TM outputs a lane
   float* out = g.partial != nullptr ? g.partial + size_t(blockIdx.y) * g.M * g.N : g.C + size_t(blockIdx.z) * g.stride_c;
@@ -368,16 +377,18 @@ int gemm_direct_launch(dyhip_device* dev, bool a_kmajor, bool b_kmajor, size_t M
   g.partial = partial;
   g.epi = epi;
   g.steps = 0;
-  size_t depth = 0;
+  size_t depth = 0, ld = 0;
   for (int s = 0; s < kGemmMaxSeg; ++s) {
     g.seg[s] = s < nseg ? segs[s] : GemmSeg{nullptr, 0, nullptr, 0, 0};
     g.steps += unsigned((g.seg[s].K + 15) / 16);
     depth += g.seg[s].K;
+    ld = std::max({ld, g.seg[s].lda, g.seg[s].ldb});
   }
   const unsigned items = batch != nullptr && batch->count > 1 ? batch->count : 1;
   g.stride_a = items > 1 ? batch->stride_a : 0;
   g.stride_b = items > 1 ? batch->stride_b : 0;
   g.stride_c = items > 1 ? batch->stride_c : 0;
+  if (tn == 2 && ld >= (size_t(1) << 24)) tn = 1;  // 2 x 2 tiles: 32-bit offsets over 64 rows
   g.order = TileOrder::of(cdiv<unsigned>(g.M, 32 * tm), cdiv<unsigned>(g.N, 32 * tn), tm, tn);
   g.steps_per_split = std::max(1u, cdiv<unsigned>(std::max(1u, g.steps), splits_wanted));
   *splits = std::max(1u, cdiv<unsigned>(g.steps, g.steps_per_split));

@@ -127,10 +127,10 @@ __global__ __launch_bounds__(256, 2) void gemm_tile_kernel(TileArgs g) {
   bf16x8 ah[2], am[2], al[2], bh[2][2], bm[2], bl[2];
 #define DYHIP_TILE_READ(f, o, plane) \
   _Pragma("unroll") for (int t_ = 0; t_ < 2; ++t_) f[t_] = *reinterpret_cast<const bf16x8*>(lds + (o) + (plane) * kTilePlane + t_ * 512);
-#define DYHIP_TILE_MMA(fa, fb)                                    \
+#define DYHIP_TILE_MMA(fa, fb, sum)                               \
   _Pragma("unroll") for (int u_ = 0; u_ < 2; ++u_)                \
-      _Pragma("unroll") for (int t_ = 0; t_ < 2; ++t_) acc[u_][t_] = \
-          __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[u_], fa[t_], acc[u_][t_], 0, 0, 0);
+      _Pragma("unroll") for (int t_ = 0; t_ < 2; ++t_) sum[u_][t_] = \
+          __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[u_], fa[t_], sum[u_][t_], 0, 0, 0);
 #define DYHIP_TILE_FENCE __builtin_amdgcn_sched_barrier(0);
 #define DYHIP_TILE_MIX(id, n, valu, rd, wr)                                \
   _Pragma("unroll") for (int x_ = 0; x_ < (n); ++x_) {                     \
@@ -139,13 +139,13 @@ __global__ __launch_bounds__(256, 2) void gemm_tile_kernel(TileArgs g) {
     if (valu) __builtin_amdgcn_sched_group_barrier(0x002, valu, id);       \
     if (wr) __builtin_amdgcn_sched_group_barrier(0x200, wr, id);           \
   }
-  tilex16 acc[2][2];
+  tilex16 acc[2][2], low[2][2];  // sums of the products of the h parts, and of the five small ones (split3.h)
 #pragma unroll
   for (int u = 0; u < 2; ++u)
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) acc[u][t][r] = 0.f;
+      for (int r = 0; r < 16; ++r) acc[u][t][r] = low[u][t][r] = 0.f;
 
   if (s0 < s1) {
     DYHIP_TILE_SEG
@@ -167,7 +167,7 @@ __global__ __launch_bounds__(256, 2) void gemm_tile_kernel(TileArgs g) {
         if (e == 1 && s + 1 >= s1) break;
         DYHIP_TILE_READ(ah, oa[e], 0)
         DYHIP_TILE_READ(bl, ob[e], 2)
-        DYHIP_TILE_MMA(al, bh[e])
+        DYHIP_TILE_MMA(al, bh[e], low)
         DYHIP_TILE_MIX(0, 1, 0, 4, 0)
         DYHIP_TILE_MIX(0, 3, 0, 0, 0)
         DYHIP_TILE_FENCE
@@ -175,7 +175,7 @@ __global__ __launch_bounds__(256, 2) void gemm_tile_kernel(TileArgs g) {
         // is refilled below two steps ahead
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
         DYHIP_TILE_FENCE
-            DYHIP_TILE_MMA(am, bh[e])
+            DYHIP_TILE_MMA(am, bh[e], low)
         DYHIP_TILE_READ(al, oa[e ^ 1], 2)
         DYHIP_TILE_READ(bh[e ^ 1], ob[e ^ 1], 0)
         DYHIP_TILE_SPLIT(0, e)
@@ -183,20 +183,20 @@ __global__ __launch_bounds__(256, 2) void gemm_tile_kernel(TileArgs g) {
         DYHIP_TILE_MIX(1, 2, 12, 2, 0)
         DYHIP_TILE_MIX(1, 2, 12, 0, 3)
         DYHIP_TILE_FENCE
-        DYHIP_TILE_MMA(am, bm)
+        DYHIP_TILE_MMA(am, bm, low)
         DYHIP_TILE_SPLIT(2, e)
         DYHIP_TILE_SPLIT(3, e)
         DYHIP_TILE_MIX(2, 2, 12, 0, 0)
         DYHIP_TILE_MIX(2, 2, 12, 0, 3)
         DYHIP_TILE_FENCE
         DYHIP_TILE_READ(am, oa[e ^ 1], 1)
-        DYHIP_TILE_MMA(ah, bm)
+        DYHIP_TILE_MMA(ah, bm, low)
         DYHIP_TILE_FENCE
         DYHIP_TILE_LOAD
         DYHIP_TILE_READ(bm, ob[e ^ 1], 1)
-        DYHIP_TILE_MMA(ah, bl)
+        DYHIP_TILE_MMA(ah, bl, low)
         DYHIP_TILE_FENCE
-        DYHIP_TILE_MMA(ah, bh[e])
+        DYHIP_TILE_MMA(ah, bh[e], acc)
         DYHIP_TILE_FENCE
       }
     }
@@ -229,7 +229,7 @@ __global__ __launch_bounds__(256, 2) void gemm_tile_kernel(TileArgs g) {
     for (int u = 0; u < 2; ++u) {
       const unsigned i = 8 * (r / 4) + 4 * lhi + r % 4, n = n0 + (BKM ? 64 * wn + 32 * u + i : 4 * i + 2 * wn + u);
       if (n >= g.N) continue;
-      float v[2] = {acc[u][0][r], acc[u][1][r]};
+      float v[2] = {acc[u][0][r] + low[u][0][r], acc[u][1][r] + low[u][1][r]};
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
         if (m[t] >= g.M) continue;

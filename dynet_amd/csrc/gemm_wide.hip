@@ -5,23 +5,32 @@
 // cublasSgemm for).
 //
 // What bounds it.  Six bf16 products for one fp32 product: at the 2.2-2.4 PFLOP/s that register-resident 32x32x16 MFMAs
-// reach here the ceiling is about 370 TFLOP/s of fp32 work.  The MFMAs keep the matrix cores 79-90 % busy (counters), and
-// under that load the shader clock falls to 1.4-1.9 GHz: power, not the schedule, is what is left.  Measured, random
-// operands, against v_mfma_f32_32x32x2_f32 in the same tiling (94 % busy, 157 TFLOP/s at most):
-//   10000 x 4480 x 1024 l*r     708 -> 440 us (130 -> 208 TFLOP/s)   1024 x 4480 x 10000 l^T*r   712 -> 436 us
-//   10000 x 1024 x 4480 l*r^T   688 -> 410 us (133 -> 224)            4096 x 1024 x 4480 l*r^T    285 -> 174 us
+// reach here the ceiling is about 370 TFLOP/s of fp32 work.  The MFMAs keep the matrix cores 61 % busy (counters, 10000 x
+// 4480 x 1024) at a shader clock that falls to 1.9 GHz; a third stage in LDS, which takes the two wavefronts of a SIMD out
+// of step, changed nothing.  Measured, random operands, against v_mfma_f32_32x32x2_f32 in the same tiling (94 % busy,
+// 157 TFLOP/s at most):
+//   10000 x 4480 x 1024 l*r     708 -> 486 us (130 -> 189 TFLOP/s)   1024 x 4480 x 10000 l^T*r   712 -> 488 us
+//   10000 x 1024 x 4480 l*r^T   688 -> 457 us (133 -> 201)            4096 x 1024 x 4480 l*r^T    285 -> 194 us
 //
 // Step of 16 k.  Operands are fetched as fp32 into registers (four 128-bit loads a thread), split there and written to
-// LDS as three bf16 planes: splitting in the block re-does the work for every tile that shares an operand, but 88 vector
+// LDS as three bf16 planes: splitting in the block re-does the work for every tile that shares an operand, but 72 vector
 // instructions a wave and step hide under 48 MFMAs, where a pass of its own over the operands would move 10 bytes per
 // element (450 MB for a 10000 x 4480 operand).  LDS holds two stages of 48 KiB; fragments are read as 128 bits a lane.
 //
-// Schedule of a step (48 MFMAs per wave, in six groups by plane: l*h, m*h, m*m, h*m, h*l, h*h).  The order frees the
-// fragment registers of the small planes early, so that the next step's first four fragment sets are read into them
-// under this step's MFMAs and only the h plane of A and the l plane of B are read in the step that uses them.  One barrier
-// after the first group: there every wave holds the last fragments of this step's stage, which is refilled two steps
-// ahead under the second and third group; the loads for the step after that leave under the fourth.  Vector and LDS
-// instructions are dealt between the MFMAs one by one (left alone the compiler puts them in front: 10 % slower).
+// Sums.  A matrix instruction rounds what it adds to, so six of them into one accumulator round a long sum six times in 16
+// k, where the fp32 instruction rounds it once a product that is not zero: with half of the products zero (a rectifier's
+// outputs) the sums were 13 % further from fp64 than the fp32 instruction's, with nine tenths zero 76 % (K = 512).  So the
+// six products of a 32 x 32 tile form a sum of their own, from zero, which vector instructions add to the accumulator:
+// one rounding of the long sum in 16 k.  Three times closer than the fp32 instruction on dense operands, as close with 3 %
+// of the products left (1.0-1.2 times), 1.15-1.3 times as far with 1 %.  (An accumulator each for the large and the small
+// products, as in the other kernels, does not fit beside 128 sums a lane.)  It costs 6 %: 128 vector instructions a step.
+//
+// Schedule of a step (48 MFMAs per wave): tile by tile, two column tiles for each of four row tiles.  A tile's sum is added
+// up under the MFMAs of the next one.  The second tile of a pair uses the small planes of the row tile first, so that the
+// next row tile's planes are read into the same registers as they fall free.  One barrier before the last row tile: there
+// every wave holds the last fragments of this step's stage, which is refilled two steps ahead under what is left, and the
+// loads for the step after that leave last.  Vector and LDS instructions are dealt between the MFMAs one by one (left
+// alone the compiler puts them in front).
 //
 // Work distribution.  The tile count rarely divides the CU count, and a round of one tile per CU that is not full
 // leaves CUs idle for the whole round.  So the units of work are k-tiles: all k-tiles of all tiles, tile by tile, form
@@ -86,8 +95,9 @@ struct WideArgs {
 // half are permuted by xor 4, which puts the two halves of a row's 64 bytes on different banks.
 // Waves 0-3 stage A, waves 4-7 stage B: four 128-bit loads a lane (16 values), split into 4 rows x 4 k, three 64-bit
 // LDS writes a row.
-constexpr unsigned kPlaneBytes = 8192, kOperandBytes = 3 * kPlaneBytes, kStageBytes = 2 * kOperandBytes;
-constexpr size_t kWideLdsBytes = 2 * kStageBytes;  // 96 KiB
+// LDS: [operand][stage][plane], so that the second stage is in reach of an LDS instruction's offset.
+constexpr unsigned kPlaneBytes = 8192, kStageBytes = 3 * kPlaneBytes, kOperandBytes = 2 * kStageBytes;
+constexpr size_t kWideLdsBytes = 2 * kOperandBytes;  // 96 KiB
 
 // byte offsets (from the tile's first row and the step's first k) of this lane's four loads; rows and groups of
 // four past the matrix edge are clamped to the last one inside (their values only reach outputs the epilogue masks)
@@ -191,11 +201,9 @@ __global__ __launch_bounds__(kWideThreads, 1) void gemm_wide_kernel(WideArgs g) 
   const int wm = w & 1, wn = w >> 1;
   const int l32 = lane & 31, lhi = lane >> 5;
   const unsigned frag = lhi * 4096 + (l32 ^ (4 * lhi)) * 16;
-  // this lane's fragments of A and B in both stages, and its first row in both: a register each (the second stage lies
-  // beyond the reach of an LDS instruction's offset; an addition in front of every access would break up the schedule)
-  unsigned oa[2], ob[2], ow[2];
-  oa[0] = frag + wm * (AK ? 128 : 32) * 16;
-  ob[0] = kOperandBytes + frag + (BKM ? wn * 64 : (wn & 1) * 128 + (wn >> 1) * 32) * 16;
+  // this lane's fragments of A and B, and its first row (below)
+  const unsigned oa = frag + wm * (AK ? 128 : 32) * 16;
+  const unsigned ob = kOperandBytes + frag + (BKM ? wn * 64 : (wn & 1) * 128 + (wn >> 1) * 32) * 16;
   constexpr unsigned ta = AK ? 512 : 1024, tb = BKM ? 512 : 1024;  // bytes between a wave's row (column) tiles
   const unsigned nt = g.nt;
 
@@ -213,11 +221,7 @@ __global__ __launch_bounds__(kWideThreads, 1) void gemm_wide_kernel(WideArgs g) 
   const float* const operand = stage_b ? g.B : g.A;
   const bool kmajor = AK == BKM ? AK : stage_b ? BKM : AK;
   const size_t step = kmajor ? 16 : size_t(16) * ld;
-  ow[0] = (stage_b ? kOperandBytes : 0u) + write_offset(kmajor);
-  oa[1] = oa[0] + kStageBytes;
-  ob[1] = ob[0] + kStageBytes;
-  ow[1] = ow[0] + kStageBytes;
-  asm volatile("" : "+v"(oa[1]), "+v"(ob[1]), "+v"(ow[1]));
+  const unsigned ow = (stage_b ? kOperandBytes : 0u) + write_offset(kmajor);
   const unsigned last = 2 * u1 - 1;
   unsigned load_at = 2 * u0, load_end, off[4];
   const float* load_p;
@@ -240,17 +244,32 @@ __global__ __launch_bounds__(kWideThreads, 1) void gemm_wide_kernel(WideArgs g) 
     load_p += more_ * step;                                                                      \
   }
 #define DYHIP_WIDE_LOAD_NEXT_TILE if (load_at == load_end) DYHIP_WIDE_TILE(0u)
-#define DYHIP_WIDE_SPLIT(j, stage) split_row(kmajor, raw, (j), lds + ow[stage]);
-  bf16x8 ah[4], am[4], al[4], bh[2][2], bm[2], bl[2];
-#define DYHIP_WIDE_READ_A(f, plane, stage) \
-  _Pragma("unroll") for (int t_ = 0; t_ < 4; ++t_) f[t_] = read_frag(lds + oa[stage] + (plane) * kPlaneBytes + t_ * ta);
-#define DYHIP_WIDE_READ_B(f, plane, stage) \
-  _Pragma("unroll") for (int u_ = 0; u_ < 2; ++u_) f[u_] = read_frag(lds + ob[stage] + (plane) * kPlaneBytes + u_ * tb);
-#define DYHIP_WIDE_MMA(fa, fb)                                    \
-  _Pragma("unroll") for (int u_ = 0; u_ < 2; ++u_)                \
-      _Pragma("unroll") for (int t_ = 0; t_ < 4; ++t_) acc[u_][t_] = \
-          __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[u_], fa[t_], acc[u_][t_], 0, 0, 0);
-// n times: one MFMA, then so many vector instructions, LDS reads, LDS writes and global loads
+#define DYHIP_WIDE_SPLIT(j, stage) split_row(kmajor, raw, (j), lds + ow + (stage) * kStageBytes);
+  // Fragments (h, m, l) of one of the wave's row tiles and of both of its column tiles.  A step's products go tile by tile,
+  // x = 2 t + u; a plane of the row tile is fetched for the next one where its last product has been issued.
+  bf16x8 fa[3], fb[2][3];
+#define DYHIP_WIDE_READ_A(p, t, stage) fa[p] = read_frag(lds + oa + (stage) * kStageBytes + (p) * kPlaneBytes + (t) * ta);
+#define DYHIP_WIDE_READ_B(u, stage) \
+  _Pragma("unroll") for (int p_ = 0; p_ < 3; ++p_) fb[u][p_] = read_frag(lds + ob + (stage) * kStageBytes + p_ * kPlaneBytes + (u) * tb);
+#define DYHIP_WIDE_MMA(x, pa, pb) \
+  sum[(x) % 2] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[(x) % 2][pb], fa[pa], sum[(x) % 2], 0, 0, 0);
+#define DYHIP_WIDE_CHAIN(x)                              \
+  _Pragma("unroll") for (int r_ = 0; r_ < 16; ++r_) sum[(x) % 2][r_] = 0.f; \
+  DYHIP_WIDE_MMA(x, 2, 0) DYHIP_WIDE_MMA(x, 1, 1) DYHIP_WIDE_MMA(x, 1, 0) DYHIP_WIDE_MMA(x, 0, 2) DYHIP_WIDE_MMA(x, 0, 1) \
+  DYHIP_WIDE_MMA(x, 0, 0)
+// the second tile of a pair, and the next row tile t of a stage behind it
+#define DYHIP_WIDE_CHAIN_NEXT(x, t, stage)                              \
+  _Pragma("unroll") for (int r_ = 0; r_ < 16; ++r_) sum[(x) % 2][r_] = 0.f; \
+  DYHIP_WIDE_MMA(x, 2, 0) DYHIP_WIDE_READ_A(2, t, stage) DYHIP_WIDE_MMA(x, 1, 1) DYHIP_WIDE_MMA(x, 1, 0) \
+  DYHIP_WIDE_READ_A(1, t, stage) DYHIP_WIDE_MMA(x, 0, 2) DYHIP_WIDE_MMA(x, 0, 1) DYHIP_WIDE_MMA(x, 0, 0) \
+  DYHIP_WIDE_READ_A(0, t, stage)
+#define DYHIP_WIDE_ADD(x) _Pragma("unroll") for (int r_ = 0; r_ < 16; ++r_) acc[(x) % 2][(x) / 2][r_] += sum[(x) % 2][r_];
+// (keeps the additions where they are: the compiler would move them out of the loop, and spill the sums)
+#define DYHIP_WIDE_PIN(x) _Pragma("unroll") for (int r_ = 0; r_ < 16; r_ += 8) {                                            \
+    float* a_ = acc[(x) % 2][(x) / 2] + r_;                                                                               \
+    asm volatile("" : "+v"(a_[0]), "+v"(a_[1]), "+v"(a_[2]), "+v"(a_[3]), "+v"(a_[4]), "+v"(a_[5]), "+v"(a_[6]), "+v"(a_[7])); \
+  }
+// n times: one MFMA, then so many LDS reads, vector instructions, LDS writes and global loads
 #define DYHIP_WIDE_MIX(id, n, valu, rd, wr, ld_)                               \
   _Pragma("unroll") for (int x_ = 0; x_ < (n); ++x_) {                     \
     __builtin_amdgcn_sched_group_barrier(0x008, 1, id);                     \
@@ -274,62 +293,99 @@ __global__ __launch_bounds__(kWideThreads, 1) void gemm_wide_kernel(WideArgs g) 
       DYHIP_WIDE_LOAD
       DYHIP_WIDE_LOAD_NEXT_TILE
       __syncthreads();
-      DYHIP_WIDE_READ_A(al, 2, 0)
-      DYHIP_WIDE_READ_B(bh[0], 0, 0)
-      DYHIP_WIDE_READ_A(am, 1, 0)
-      DYHIP_WIDE_READ_B(bm, 1, 0)
+      DYHIP_WIDE_READ_A(2, 0, 0)
+      DYHIP_WIDE_READ_A(1, 0, 0)
+      DYHIP_WIDE_READ_A(0, 0, 0)
+      DYHIP_WIDE_READ_B(0, 0)
     }
     pos += kt1 - kt0;
-    floatx16 acc[2][4];
+    float acc[2][4][16];
+    floatx16 sum[2];
 #pragma unroll
-    for (int u = 0; u < 2; ++u)
+    for (int u = 0; u < 2; ++u) {
 #pragma unroll
       for (int t = 0; t < 4; ++t)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) acc[u][t][r] = 0.f;
+        for (int r = 0; r < 16; ++r) acc[u][t][r] = sum[u][r] = 0.f;
+    }
     for (unsigned i = kt0; i < kt1; ++i) {
 #pragma unroll
       for (int e = 0; e < 2; ++e) {
-        DYHIP_WIDE_READ_A(ah, 0, e)
-        DYHIP_WIDE_READ_B(bl, 2, e)
-        DYHIP_WIDE_MMA(al, bh[e])
-        DYHIP_WIDE_MIX(0, 1, 0, 6, 0, 0)
-        DYHIP_WIDE_MIX(0, 7, 0, 0, 0, 0)
+        DYHIP_WIDE_READ_B(1, e)
+        DYHIP_WIDE_CHAIN(0)
+        DYHIP_WIDE_ADD(7)  // of the step before
+        DYHIP_WIDE_MIX(0, 2, 0, 2, 0, 0)
+        DYHIP_WIDE_MIX(0, 4, 4, 0, 0, 0)
+        DYHIP_WIDE_PIN(7)
+        DYHIP_WIDE_FENCE
+        DYHIP_WIDE_CHAIN_NEXT(1, 1, e)
+        DYHIP_WIDE_ADD(0)
+        DYHIP_WIDE_MIX(1, 1, 0, 0, 0, 0)
+        DYHIP_WIDE_MIX(1, 1, 0, 1, 0, 0)
+        DYHIP_WIDE_MIX(1, 1, 5, 0, 0, 0)
+        DYHIP_WIDE_MIX(1, 1, 5, 1, 0, 0)
+        DYHIP_WIDE_MIX(1, 2, 3, 0, 0, 0)
+        DYHIP_WIDE_PIN(0)
+        DYHIP_WIDE_FENCE
+        DYHIP_WIDE_CHAIN(2)
+        DYHIP_WIDE_ADD(1)
+        DYHIP_WIDE_MIX(2, 2, 0, 0, 0, 0)
+        DYHIP_WIDE_MIX(2, 4, 4, 0, 0, 0)
+        DYHIP_WIDE_PIN(1)
+        DYHIP_WIDE_FENCE
+        DYHIP_WIDE_CHAIN_NEXT(3, 2, e)
+        DYHIP_WIDE_ADD(2)
+        DYHIP_WIDE_MIX(3, 1, 0, 0, 0, 0)
+        DYHIP_WIDE_MIX(3, 1, 0, 1, 0, 0)
+        DYHIP_WIDE_MIX(3, 1, 5, 0, 0, 0)
+        DYHIP_WIDE_MIX(3, 1, 5, 1, 0, 0)
+        DYHIP_WIDE_MIX(3, 2, 3, 0, 0, 0)
+        DYHIP_WIDE_PIN(2)
+        DYHIP_WIDE_FENCE
+        DYHIP_WIDE_CHAIN(4)
+        DYHIP_WIDE_ADD(3)
+        DYHIP_WIDE_MIX(4, 2, 0, 0, 0, 0)
+        DYHIP_WIDE_MIX(4, 4, 4, 0, 0, 0)
+        DYHIP_WIDE_PIN(3)
+        DYHIP_WIDE_FENCE
+        DYHIP_WIDE_CHAIN_NEXT(5, 3, e)
+        DYHIP_WIDE_ADD(4)
+        DYHIP_WIDE_MIX(5, 1, 0, 0, 0, 0)
+        DYHIP_WIDE_MIX(5, 1, 0, 1, 0, 0)
+        DYHIP_WIDE_MIX(5, 1, 5, 0, 0, 0)
+        DYHIP_WIDE_MIX(5, 1, 5, 1, 0, 0)
+        DYHIP_WIDE_MIX(5, 2, 3, 0, 0, 0)
+        DYHIP_WIDE_PIN(4)
         DYHIP_WIDE_FENCE
         // every wave's part of the next step is in LDS, and every wave holds its last fragments of this one, whose stage
         // is refilled below two steps ahead
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
         DYHIP_WIDE_FENCE
-        DYHIP_WIDE_MMA(am, bh[e])
-        DYHIP_WIDE_READ_A(al, 2, e ^ 1)
-        DYHIP_WIDE_READ_B(bh[e ^ 1], 0, e ^ 1)
+        DYHIP_WIDE_CHAIN(6)
+        DYHIP_WIDE_ADD(5)
         DYHIP_WIDE_SPLIT(0, e)
         DYHIP_WIDE_SPLIT(1, e)
-        DYHIP_WIDE_MIX(2, 3, 6, 2, 0, 0)
-        DYHIP_WIDE_MIX(2, 5, 6, 0, 2, 0)
+        DYHIP_WIDE_MIX(6, 2, 6, 0, 0, 0)
+        DYHIP_WIDE_MIX(6, 4, 10, 0, 2, 0)
+        DYHIP_WIDE_PIN(5)
         DYHIP_WIDE_FENCE
-        DYHIP_WIDE_MMA(am, bm)
+        DYHIP_WIDE_READ_B(0, e ^ 1)
+        DYHIP_WIDE_CHAIN_NEXT(7, 0, e ^ 1)
+        DYHIP_WIDE_ADD(6)
         DYHIP_WIDE_SPLIT(2, e)
         DYHIP_WIDE_SPLIT(3, e)
-        DYHIP_WIDE_MIX(3, 3, 6, 0, 0, 0)
-        DYHIP_WIDE_MIX(3, 5, 6, 0, 2, 0)
-        DYHIP_WIDE_FENCE
         DYHIP_WIDE_LOAD
-        DYHIP_WIDE_READ_A(am, 1, e ^ 1)
-        DYHIP_WIDE_MMA(ah, bm)
-        DYHIP_WIDE_MIX(4, 4, 2, 1, 0, 0)
-        DYHIP_WIDE_MIX(4, 4, 2, 0, 0, 1)
-        DYHIP_WIDE_FENCE
-        DYHIP_WIDE_READ_B(bm, 1, e ^ 1)
-        DYHIP_WIDE_MMA(ah, bl)
-        DYHIP_WIDE_MIX(5, 2, 0, 1, 0, 0)
-        DYHIP_WIDE_MIX(5, 6, 0, 0, 0, 0)
-        DYHIP_WIDE_FENCE
-        DYHIP_WIDE_MMA(ah, bh[e])
+        DYHIP_WIDE_MIX(7, 1, 6, 3, 0, 0)
+        DYHIP_WIDE_MIX(7, 1, 6, 1, 0, 0)
+        DYHIP_WIDE_MIX(7, 1, 10, 0, 2, 0)
+        DYHIP_WIDE_MIX(7, 1, 10, 1, 2, 0)
+        DYHIP_WIDE_MIX(7, 2, 10, 0, 1, 2)
+        DYHIP_WIDE_PIN(6)
         DYHIP_WIDE_FENCE
         DYHIP_WIDE_LOAD_NEXT_TILE
       }
     }
+    DYHIP_WIDE_ADD(7)
 
     // the thread index as the compiler cannot see through: the addresses below are formed here, after the loop,
     // instead of being computed ahead of it and parked in scratch memory
@@ -455,6 +511,10 @@ __global__ __launch_bounds__(kWideThreads, 1) void gemm_wide_kernel(WideArgs g) 
 #undef DYHIP_WIDE_READ_A
 #undef DYHIP_WIDE_READ_B
 #undef DYHIP_WIDE_MMA
+#undef DYHIP_WIDE_CHAIN
+#undef DYHIP_WIDE_CHAIN_NEXT
+#undef DYHIP_WIDE_PIN
+#undef DYHIP_WIDE_ADD
 #undef DYHIP_WIDE_MIX
 #undef DYHIP_WIDE_FENCE
 }
@@ -659,7 +719,7 @@ __global__ __launch_bounds__(kWideThreads, 1) void gemm_shallow_nt_kernel(Shallo
 template <bool AK, bool BKM>
 int launch_wide(dyhip_device* dev, const WideArgs& g, unsigned blocks, unsigned bit) {
   const void* fn = reinterpret_cast<const void*>(&gemm_wide_kernel<AK, BKM>);
-  if ((dev->wide_gemm_ready & (1u << bit)) == 0) {  // 128 KiB of LDS need the opt-in, once per device
+  if ((dev->wide_gemm_ready & (1u << bit)) == 0) {  // 96 KiB of LDS need the opt-in, once per device
     DYHIP_CHECK_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, int(kWideLdsBytes)));
     dev->wide_gemm_ready |= 1u << bit;
   }

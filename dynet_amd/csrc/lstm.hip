@@ -966,11 +966,11 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_nn_deep_kernel(unsigned M, 
   const unsigned l32 = lane % 32, lhi = lane / 32;
   const float bias_row = EPI == kNnAxpby ? 0.f : bias[min(rp * ROWS + threadIdx.x % ROWS, M - 1)];
   unsigned row[TILES], vcol[4];
-  stepx16 acc[TILES];
+  stepx16 acc[TILES], low[TILES];  // sums of the products of the h parts, and of the five small ones (split3.h)
 #pragma unroll
   for (int t = 0; t < TILES; ++t) {
     row[t] = min(rp * ROWS + 32 * t + l32, M - 1);
-    acc[t] = stepx16{0};
+    acc[t] = low[t] = stepx16{0};
   }
 #pragma unroll
   for (unsigned i = 0; i < 4; ++i) vcol[i] = min(ct * 32 + 8 * i + lane / 8, B - 1);  // past the batch: dropped
@@ -1028,10 +1028,11 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_nn_deep_kernel(unsigned M, 
           for (int t = 0; t < TILES; ++t)
             fa[t].from(make_float4(a[r][q][t][0], a[r][q][t][1], a[r][q][t][2], a[r][q][t][3]),
                        make_float4(a[r][q][t][4], a[r][q][t][5], a[r][q][t][6], a[r][q][t][7]));
-#define DYHIP_NN_MMA(x, y)                                                    \
-  _Pragma("unroll") for (int t = 0; t < TILES; ++t) acc[t] =                  \
-      __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[t].x, fb.y, acc[t], 0, 0, 0);
-          DYHIP_NN_MMA(l, h) DYHIP_NN_MMA(h, l) DYHIP_NN_MMA(m, m) DYHIP_NN_MMA(m, h) DYHIP_NN_MMA(h, m) DYHIP_NN_MMA(h, h)
+#define DYHIP_NN_MMA(x, y, sum)                                               \
+  _Pragma("unroll") for (int t = 0; t < TILES; ++t) sum[t] =                  \
+      __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[t].x, fb.y, sum[t], 0, 0, 0);
+          DYHIP_NN_MMA(l, h, low) DYHIP_NN_MMA(h, l, low) DYHIP_NN_MMA(m, m, low)
+          DYHIP_NN_MMA(m, h, low) DYHIP_NN_MMA(h, m, low) DYHIP_NN_MMA(h, h, acc)
 #undef DYHIP_NN_MMA
         }
         __builtin_amdgcn_wave_barrier();
@@ -1044,7 +1045,7 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_nn_deep_kernel(unsigned M, 
   for (int r = 0; r < 16; ++r) {
     const unsigned i = 8 * (r / 4) + 4 * lhi + (r % 4);
 #pragma unroll
-    for (int t = 0; t < TILES; ++t) red[(wave * ROWS + 32 * t + i) * kStepPitchR + l32] = acc[t][r];
+    for (int t = 0; t < TILES; ++t) red[(wave * ROWS + 32 * t + i) * kStepPitchR + l32] = acc[t][r] + low[t][r];
   }
   __syncthreads();
 #pragma unroll

@@ -5,10 +5,15 @@
 // the three 8-bit significands hold all 24 bits of x.  A product x*y is then formed from six of the nine bf16 products,
 //     l*h' + m*h' + m*m' + h*m' + h*l' + h*h',
 // each exact in fp32, accumulated in fp32.  Rounding to nearest leaves |m| <= 2^-8 |x| and |l| <= 2^-17 |x|, so the
-// three products left out (m*l', l*m', l*l') are below (2^-25 + 2^-25 + 2^-34) |x y|: less than the 2^-24 |x y| that
-// rounding the fp32 product once would cost.  The accumulation rounds less often than the fp32 instruction's: 16 terms
-// of the depth cost six additions into the accumulator where v_mfma_f32_32x32x2_f32 makes sixteen.  Measured against
-// fp64, the sums are as close as the fp32 instruction's or closer (the tests check both).
+// three products left out (m*l', l*m', l*l') are at most (2^-25 + 2^-25 + 2^-34) |x y| together and typically a quarter
+// of that: about the 2^-25 |x y| by which rounding an fp32 product is off at most.
+//
+// A matrix instruction rounds its accumulator once, however many of its 16 products are zero.  All six in one accumulator
+// would round a long sum six times in 16 k, where fp32 arithmetic rounds once a product that is not zero: worse than fp32
+// from half of the products zero on.  So the products h*h' have an accumulator of their own, and the five small ones,
+// whose sums are 2^-8 of it, share another (gemm_wide.hip, which has no registers for that, forms each step's sum by
+// itself).  Against fp64, K = 512, products that are not zero 100 / 25 / 10 / 1 %, in units of 1e-8:
+//   one accumulator 17 / 15 / 12 / 6.5,  two 7.7 / 5.9 / 5.2 / 4.4,  the fp32 instruction 29 / 15 / 9.8 / 4.7.
 //
 // The smallest bf16 value is 2^-133, so the parts of x hold all of it only if its last bit is at least that: |x| >= 2^-110.
 // fp32 values reach down to 2^-149 (probabilities of a confident softmax are that small), so every operand is multiplied

@@ -2140,6 +2140,21 @@ def test_gemm_split_products_keep_the_bits_of_tiny_values(dev, M, N, K, e):
         assert np.linalg.norm(y - exact) <= 0.5 * np.sqrt(K) * 2.0 ** -24 * np.linalg.norm(exact), form
 
 
+@pytest.mark.parametrize("M,N,K", SPLIT_GEMM_SHAPES + [(1000, 20, 640)])
+@pytest.mark.parametrize("density", [1.0, 0.5, 0.25, 0.1])
+def test_gemm_split_products_of_sparse_operands_are_as_close_as_fp32(dev, M, N, K, density):
+    """Zeros (of a rectifier, of dropout) take roundings from an fp32 sum.  The bound is what one rounding to nearest a
+    product that is not zero leaves of a sum of n = density * K random terms: each is off by 0.29 ulp (rms), an ulp is
+    2^-23 / 1.44 of the sum on average over its binade, and the sum's square grows like its term number, which makes
+    0.3 * sqrt(n) * 2^-24 of the whole; the one rounding of a single term (0.2 in its square) stays however small n is."""
+    rng = np.random.default_rng(M + K)
+    l, r = (f32(rng.standard_normal(s) * (rng.random(s) < np.sqrt(density))) for s in ((K, M), (N, K)))
+    exact = r.astype(np.float64) @ l.astype(np.float64)
+    bound = np.sqrt(0.2 + 0.09 * density * K) * 2.0 ** -24 * np.linalg.norm(exact)
+    for form, y in _three_forms(dev, M, N, K, l, r, np.zeros((N, M), np.float32), 0.0):
+        assert np.linalg.norm(y - exact) <= bound, form
+
+
 @pytest.mark.parametrize("M,N,K", SPLIT_GEMM_SHAPES)
 def test_gemm_split_products_keep_infinities_nans_and_huge_values(dev, M, N, K):
     """Where an operand is infinite, NaN or rounds beyond the largest bf16, its outputs are formed by plain fp32
