@@ -303,13 +303,37 @@ __global__ __launch_bounds__(64 * WAVES, 2) void gemm_direct_kernel(DirectArgs g
 #undef DYHIP_DIRECT_READ
   }
 
+  if (SPLIT) {  // this wavefront's sums, whole and to scale
+#pragma unroll
+    for (int u = 0; u < TN; ++u)
+#pragma unroll
+      for (int t = 0; t < TM; ++t) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[u][t][r] = (acc[u][t][r] + low[u][t][r]) * kSplitOut;
+        if (__builtin_expect(any_not_finite(acc[u][t]), 0)) {
+          const unsigned m = min(m0 + (AK ? 32 * t + l32 : TM * l32 + t), g.M - 1);
+          const unsigned n = min(n0 + (BKM ? 32 * u + l32 : TN * l32 + u), g.N - 1);
+          sums16 s = {};
+          unsigned fs = 0;
+          for (int sg = 0; sg < g.nseg; ++sg) {
+            const GemmSeg& q = g.seg[sg];
+            const unsigned count = (unsigned(q.K) + 15) / 16, b0 = max(w0, fs) - fs, b1 = max(min(w1, fs + count), fs) - fs;
+            add_products_fp32<AK, BKM>(s, q.A + size_t(blockIdx.z) * g.stride_a + (AK ? m * q.lda : m), q.lda,
+                                       q.B + size_t(blockIdx.z) * g.stride_b + (BKM ? n * q.ldb : n), q.ldb, 16 * b0,
+                                       min(16 * b1, unsigned(q.K)));
+            fs += count;
+          }
+          acc[u][t] = s;
+        }
+      }
+  }
   __syncthreads();
 #pragma unroll
   for (int u = 0; u < TN; ++u)
 #pragma unroll
     for (int t = 0; t < TM; ++t)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) lds[((w * TN + u) * TM + t) * 1024 + r * 64 + lane] = SPLIT ? acc[u][t][r] + low[u][t][r] : acc[u][t][r];
+      for (int r = 0; r < 16; ++r) lds[((w * TN + u) * TM + t) * 1024 + r * 64 + lane] = acc[u][t][r];
   __syncthreads();
   // wavefront w finishes 16 * TN / WAVES groups of TM outputs a lane
   float* out = g.partial != nullptr ? g.partial + size_t(blockIdx.y) * g.M * g.N : g.C + size_t(blockIdx.z) * g.stride_c;
@@ -325,24 +349,6 @@ __global__ __launch_bounds__(64 * WAVES, 2) void gemm_direct_kernel(DirectArgs g
       float v = lds[(u * TM + t) * 1024 + r * 64 + lane];
 #pragma unroll
       for (int ww = 1; ww < WAVES; ++ww) v += lds[((ww * TN + u) * TM + t) * 1024 + r * 64 + lane];
-      if (SPLIT && not_finite(v)) {
-        v = 0.f;
-        unsigned fs = 0;
-        for (int sg = 0; sg < g.nseg; ++sg) {
-          const GemmSeg& q = g.seg[sg];
-          const unsigned count = (unsigned(q.K) + 15) / 16;
-          const unsigned b0 = max(s0, fs), b1 = min(s1, fs + count);
-          if (b1 > b0) {
-            const unsigned k0 = 16 * (b0 - fs), k1 = min(unsigned(q.K), 16 * (b1 - fs));
-            const float* pa = q.A + size_t(blockIdx.z) * g.stride_a + (AK ? size_t(m) * q.lda + k0 : m + k0 * q.lda);
-            const float* pb = q.B + size_t(blockIdx.z) * g.stride_b + (BKM ? size_t(n) * q.ldb + k0 : n + k0 * q.ldb);
-            v += dot_fp32(pa, AK ? 1 : q.lda, pb, BKM ? 1 : q.ldb, k1 - k0);
-          }
-          fs += count;
-        }
-      } else if (SPLIT) {
-        v *= kSplitOut;
-      }
       float* p = out + m + size_t(n) * g.M;
       if (g.partial == nullptr) {
         if (g.epi.kind == kEpiAxpby) {

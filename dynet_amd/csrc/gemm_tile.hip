@@ -209,6 +209,30 @@ __global__ __launch_bounds__(256, 2) void gemm_tile_kernel(TileArgs g) {
 #undef DYHIP_TILE_FENCE
 #undef DYHIP_TILE_MIX
 
+  // the wavefront's sums, whole and to scale
+#pragma unroll
+  for (int u = 0; u < 2; ++u)
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[u][t][r] = (acc[u][t][r] + low[u][t][r]) * kSplitOut;
+      if (__builtin_expect(any_not_finite(acc[u][t]), 0)) {
+        const unsigned m = min(m0 + (AK ? 64 * wm + 32 * t + l32 : 4 * l32 + 2 * wm + t), g.M - 1);
+        const unsigned n = min(n0 + (BKM ? 64 * wn + 32 * u + l32 : 4 * l32 + 2 * wn + u), g.N - 1);
+        sums16 s = {};
+        unsigned first = 0;
+        for (int sg = 0; sg < g.nseg; ++sg) {
+          const GemmSeg& q = g.seg[sg];
+          const unsigned count = (unsigned(q.K) + 15) / 16, b0 = max(s0, first) - first, b1 = max(min(s1, first + count), first) - first;
+          add_products_fp32<AK, BKM>(s, q.A + size_t(blockIdx.z) * g.stride_a + (AK ? m * q.lda : m), q.lda,
+                                     q.B + size_t(blockIdx.z) * g.stride_b + (BKM ? n * q.ldb : n), q.ldb, 16 * b0,
+                                     min(16 * b1, unsigned(q.K)));
+          first += count;
+        }
+        acc[u][t] = s;
+      }
+    }
+
   // acc[u][t][r] of a lane: two rows and, for each r, two columns
   float* out = g.partial != nullptr ? g.partial + size_t(blockIdx.y) * g.M * g.N : g.C + size_t(blockIdx.z) * g.stride_c;
   const bool direct = g.partial == nullptr;
@@ -229,28 +253,10 @@ __global__ __launch_bounds__(256, 2) void gemm_tile_kernel(TileArgs g) {
     for (int u = 0; u < 2; ++u) {
       const unsigned i = 8 * (r / 4) + 4 * lhi + r % 4, n = n0 + (BKM ? 64 * wn + 32 * u + i : 4 * i + 2 * wn + u);
       if (n >= g.N) continue;
-      float v[2] = {acc[u][0][r] + low[u][0][r], acc[u][1][r] + low[u][1][r]};
+      float v[2] = {acc[u][0][r], acc[u][1][r]};
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
         if (m[t] >= g.M) continue;
-        if (not_finite(v[t])) {
-          v[t] = 0.f;
-          unsigned first = 0;
-          for (int sg = 0; sg < g.nseg; ++sg) {
-            const GemmSeg& q = g.seg[sg];
-            const unsigned count = (unsigned(q.K) + 15) / 16, b0 = max(s0, first), b1 = min(s1, first + count);
-            if (b1 > b0) {
-              const unsigned k0 = 16 * (b0 - first), k1 = min(unsigned(q.K), 16 * (b1 - first));
-              v[t] += dot_fp32(q.A + size_t(blockIdx.z) * g.stride_a + (AK ? size_t(m[t]) * q.lda + k0 : m[t] + k0 * q.lda),
-                               AK ? 1 : q.lda,
-                               q.B + size_t(blockIdx.z) * g.stride_b + (BKM ? size_t(n) * q.ldb + k0 : n + k0 * q.ldb),
-                               BKM ? 1 : q.ldb, k1 - k0);
-            }
-            first += count;
-          }
-        } else {
-          v[t] *= kSplitOut;
-        }
         if (direct) {
           v[t] += bias[t];
           if (g.epi.kind == kEpiLstmGates)

@@ -173,23 +173,40 @@ __device__ __forceinline__ unsigned out_row(unsigned wm, unsigned t, unsigned l3
   return wm * 128 + (AK ? 32 * t + l32 : 4 * l32 + t);
 }
 
-// The four outputs of group ur = 16 u + r of thread tid of a tile whose sums came out non-finite, from plain fp32
-// multiply-adds.  Nothing has been stored to them yet.
+// A wavefront's 128 x 64 sums over k-tiles kt0 .. kt1 - 1 of a tile once more, by the fp32 instruction, 32 x 32 at a time:
+// to the slot of a partial tile (this thread's first element of it, past the L2), or, with the parts of segments s0 ..
+// s1 - 1 (slot: of the first segment), through the epilogue to C.
 template <bool AK, bool BKM>
-__device__ __forceinline__ void finish_group_fp32(const WideArgs& g, unsigned m0, unsigned n0, unsigned tid, unsigned ur) {
-  const unsigned lane = tid & 63, wm = (tid >> 6) & 1, wn = tid >> 7, l32 = lane & 31, lhi = lane >> 5, r = ur % 16;
-  const unsigned n = n0 + out_column<BKM>(wn, ur / 16, 8 * (r / 4) + 4 * lhi + (r % 4));
-  if (n >= g.N) return;
+__device__ __forceinline__ void redo_sums(const WideArgs& g, unsigned tile, unsigned kt0, unsigned kt1, bool part, float* slot,
+                                          unsigned s0, unsigned s1) {
+  const unsigned wm = (threadIdx.x >> 6) & 1, wn = threadIdx.x >> 7, l32 = threadIdx.x & 31, lhi = (threadIdx.x >> 5) & 1;
+  const unsigned m0 = (tile % g.tiles_m) * kWT, n0 = (tile / g.tiles_m) * kWT;
 #pragma unroll 1
-  for (unsigned t = 0; t < 4; ++t) {
-    const unsigned m = m0 + out_row<AK>(wm, t, l32);
-    if (m >= g.M) return;
-    float x = dot_fp32(g.A + (AK ? size_t(m) * g.lda : size_t(m)), AK ? 1 : g.lda, g.B + (BKM ? size_t(n) * g.ldb : size_t(n)),
-                       BKM ? 1 : g.ldb, g.nt * kWK);
-    float* p = g.C + m + size_t(n) * g.M;
-    if (g.bias != nullptr) x += g.bias[m];
-    else if (g.beta != 0.f) x += g.beta * *p;
-    *p = x;
+  for (unsigned x = 0; x < 8; ++x) {
+    const unsigned u = x / 4, t = x % 4, m = m0 + out_row<AK>(wm, t, l32);
+    const unsigned mc = min(m, g.M - 1), nc = min(n0 + out_column<BKM>(wn, u, l32), g.N - 1);
+    sums16 s = {};
+    add_products_fp32<AK, BKM>(s, g.A + (AK ? size_t(mc) * g.lda : mc), g.lda, g.B + (BKM ? size_t(nc) * g.ldb : nc), g.ldb,
+                               kt0 * kWK, kt1 * kWK);
+    typedef __attribute__((address_space(1))) float* global_float;
+    global_float at = (global_float)(slot + size_t(16 * u) * (4 * kWideThreads) + t);
+#pragma unroll
+    for (unsigned r = 0; r < 16; ++r, at += 4 * kWideThreads) {
+      asm volatile("" : "+v"(at));  // addresses one by one
+      float v = s[r];
+      if (part) {
+        __hip_atomic_store(at, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        continue;
+      }
+      for (unsigned s2 = s0; s2 < s1; ++s2)
+        v += __hip_atomic_load(at + size_t(s2) * kSlotFloats, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      const unsigned n = n0 + out_column<BKM>(wn, u, 8 * (r / 4) + 4 * lhi + r % 4);
+      if (m >= g.M || n >= g.N) continue;
+      float* p = g.C + m + size_t(n) * g.M;
+      if (g.bias != nullptr) v += g.bias[m];
+      else if (g.beta != 0.f) v += g.beta * *p;
+      *p = v;
+    }
   }
 }
 
@@ -201,9 +218,10 @@ __global__ __launch_bounds__(kWideThreads, 1) void gemm_wide_kernel(WideArgs g) 
   const int wm = w & 1, wn = w >> 1;
   const int l32 = lane & 31, lhi = lane >> 5;
   const unsigned frag = lhi * 4096 + (l32 ^ (4 * lhi)) * 16;
-  // this lane's fragments of A and B, and its first row (below)
-  const unsigned oa = frag + wm * (AK ? 128 : 32) * 16;
-  const unsigned ob = kOperandBytes + frag + (BKM ? wn * 64 : (wn & 1) * 128 + (wn >> 1) * 32) * 16;
+  // This lane's fragments of A and B, and its first row (below).  Opaque: taken apart into what they share and constants,
+  // they would put the second stage out of reach again.
+  unsigned oa = frag + wm * (AK ? 128 : 32) * 16;
+  unsigned ob = kOperandBytes + frag + (BKM ? wn * 64 : (wn & 1) * 128 + (wn >> 1) * 32) * 16;
   constexpr unsigned ta = AK ? 512 : 1024, tb = BKM ? 512 : 1024;  // bytes between a wave's row (column) tiles
   const unsigned nt = g.nt;
 
@@ -221,7 +239,8 @@ __global__ __launch_bounds__(kWideThreads, 1) void gemm_wide_kernel(WideArgs g) 
   const float* const operand = stage_b ? g.B : g.A;
   const bool kmajor = AK == BKM ? AK : stage_b ? BKM : AK;
   const size_t step = kmajor ? 16 : size_t(16) * ld;
-  const unsigned ow = (stage_b ? kOperandBytes : 0u) + write_offset(kmajor);
+  unsigned ow = (stage_b ? kOperandBytes : 0u) + write_offset(kmajor);
+  asm volatile("" : "+v"(oa), "+v"(ob), "+v"(ow));
   const unsigned last = 2 * u1 - 1;
   unsigned load_at = 2 * u0, load_end, off[4];
   const float* load_p;
@@ -386,6 +405,22 @@ __global__ __launch_bounds__(kWideThreads, 1) void gemm_wide_kernel(WideArgs g) 
       }
     }
     DYHIP_WIDE_ADD(7)
+    // Sums to scale, and whether one is not finite: then this wavefront forms its part of them again where it would store
+    // them (redo_sums).
+    bool again;
+    {
+      float z = 0.f;
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) {
+            acc[u][t][r] *= kSplitOut;
+            z = fmaf(acc[u][t][r], 0.f, z);
+          }
+      again = __any(!(z == 0.f));
+    }
 
     // the thread index as the compiler cannot see through: the addresses below are formed here, after the loop,
     // instead of being computed ahead of it and parked in scratch memory
@@ -394,36 +429,15 @@ __global__ __launch_bounds__(kWideThreads, 1) void gemm_wide_kernel(WideArgs g) 
     // acc[u][t][r] of lane l: m = AK ? 32 t + l%32 : 4 (l%32) + t (+ 128 wm),
     // n = BKM ? 32 u + i : 2 i + u (+ 64 wn) with i = 8 (r/4) + 4 (l/32) + r%4.
     // A partial tile is stored as [u][r][thread][t]: one 128-bit access per thread and (u, r), whoever reads it.
-    if (kt0 > 0 || (kt1 < nt && !g.finish_in_kernel)) {
-      // Not the whole tile, and not this block's to finish: leave the partial tile in a slot.
-      if (g.finish_in_kernel) {
-        // past the L2, for a block on another one; the segment's flag goes up once memory has acknowledged every store
-        float* slot = g.slots + size_t(seg) * kSlotFloats + 4 * tid_e;
-#pragma unroll
-        for (int u = 0; u < 2; ++u)
-#pragma unroll
-          for (int r = 0; r < 16; ++r)
-            store_through(slot + size_t(u * 16 + r) * (4 * kWideThreads), acc[u][0][r], acc[u][1][r], acc[u][2][r],
-                          acc[u][3][r]);
-        __builtin_amdgcn_s_waitcnt(0);
-        __syncthreads();
-        if (tid_e == 0 && g.raise_flags) __hip_atomic_store(g.flags + seg, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      } else {
-        float* slot = g.slots + size_t(2 * seg + (tile == u0 / nt ? 0 : 1)) * kSlotFloats + 4 * tid_e;
-#pragma unroll
-        for (int u = 0; u < 2; ++u)
-#pragma unroll
-          for (int r = 0; r < 16; ++r)
-            *reinterpret_cast<float4*>(slot + size_t(u * 16 + r) * (4 * kWideThreads)) =
-                make_float4(acc[u][0][r], acc[u][1][r], acc[u][2][r], acc[u][3][r]);
-      }
-      continue;
-    }
+    // Not the whole tile, and not this block's to finish: it goes to a slot, past the L2 for a block on another one.
+    const bool part = kt0 > 0 || (kt1 < nt && !g.finish_in_kernel);
+    float* slot = g.slots + 4 * tid_e;
+    if (part) slot += size_t(g.finish_in_kernel ? seg : 2 * seg + (tile == u0 / nt ? 0 : 1)) * kSlotFloats;
     // This block holds the tile's first k-tiles (or all of them) and finishes the tile.  The segments that start inside
     // the tile computed their partial tiles first thing, long ago by now; the wait is bounded all the same, and a wait
     // that gives up is counted for the host to report.  Partial tiles are added in segment order.
     unsigned s_end = seg + 1;
-    if (kt1 < nt) {
+    if (!part && kt1 < nt) {
       while (s_end < segments && segment_start(s_end, g.units, segments) < ub + nt) ++s_end;
       if (tid_e == 0) {
         for (unsigned s2 = seg + 1; s2 < s_end; ++s2) {
@@ -440,13 +454,40 @@ __global__ __launch_bounds__(kWideThreads, 1) void gemm_wide_kernel(WideArgs g) 
       }
       __syncthreads();
     }
+    if (__builtin_expect(again, 0)) {
+      redo_sums<AK, BKM>(g, tile, kt0, kt1, part, slot, seg + 1, s_end);
+    } else if (part) {
+      if (g.finish_in_kernel) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+          for (int r = 0; r < 16; ++r)
+            store_through(slot + size_t(u * 16 + r) * (4 * kWideThreads), acc[u][0][r], acc[u][1][r], acc[u][2][r],
+                          acc[u][3][r]);
+      } else {
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+          for (int r = 0; r < 16; ++r)
+            *reinterpret_cast<float4*>(slot + size_t(u * 16 + r) * (4 * kWideThreads)) =
+                make_float4(acc[u][0][r], acc[u][1][r], acc[u][2][r], acc[u][3][r]);
+      }
+    }
+    if (part) {
+      if (g.finish_in_kernel) {  // the segment's flag goes up once memory has acknowledged every store
+        __builtin_amdgcn_s_waitcnt(0);
+        __syncthreads();
+        if (tid_e == 0 && g.raise_flags) __hip_atomic_store(g.flags + seg, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+      continue;
+    }
+    if (again) continue;
     const unsigned lane_e = tid_e & 63, wm_e = (tid_e >> 6) & 1, wn_e = tid_e >> 7, l32_e = lane_e & 31, lhi_e = lane_e >> 5;
     const unsigned m0 = (tile % g.tiles_m) * kWT, n0 = (tile / g.tiles_m) * kWT;
     float* out = g.C + m0 + size_t(n0) * g.M;
     const unsigned mlim = g.M - m0, nlim = g.N - n0;
     const float beta = g.bias == nullptr ? g.beta : 0.f;
     const bool add_bias = g.bias != nullptr;
-    unsigned again = 0;  // groups of four outputs left to plain fp32 arithmetic
 #pragma unroll
     for (int u = 0; u < 2; ++u)
 #pragma unroll
@@ -469,11 +510,6 @@ __global__ __launch_bounds__(kWideThreads, 1) void gemm_wide_kernel(WideArgs g) 
           const int r = r0 + q;
           const unsigned n = out_column<BKM>(wn_e, u, 8 * (r / 4) + 4 * lhi_e + (r % 4));
           if (n >= nlim) continue;
-          if (not_finite(v[q])) {
-            again |= 1u << (16 * u + r);
-            continue;
-          }
-          v[q].x *= kSplitOut; v[q].y *= kSplitOut; v[q].z *= kSplitOut; v[q].w *= kSplitOut;
           if (!AK) {
             const unsigned m = out_row<AK>(wm_e, 0, l32_e);
             if (m >= mlim) continue;
@@ -502,7 +538,6 @@ __global__ __launch_bounds__(kWideThreads, 1) void gemm_wide_kernel(WideArgs g) 
           }
         }
       }
-    for (; again != 0; again &= again - 1) finish_group_fp32<AK, BKM>(g, m0, n0, tid_e, __ffs(again) - 1);
   }
 #undef DYHIP_WIDE_TILE
 #undef DYHIP_WIDE_LOAD
@@ -550,11 +585,6 @@ __global__ __launch_bounds__(kWideThreads) void gemm_wide_fixup_kernel(WideArgs 
     }
     const unsigned n = out_column<BKM>(wn, u, 8 * (r / 4) + 4 * lhi + (r % 4));
     if (n >= nlim) continue;
-    if (not_finite(v)) {
-      finish_group_fp32<AK, BKM>(g, m0, n0, tid, ur);
-      continue;
-    }
-    v.x *= kSplitOut; v.y *= kSplitOut; v.z *= kSplitOut; v.w *= kSplitOut;
     if (!AK) {
       const unsigned m = out_row<AK>(wm, 0, l32);
       if (m >= mlim) continue;

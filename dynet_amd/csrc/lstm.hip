@@ -1040,12 +1040,29 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_nn_deep_kernel(unsigned M, 
     }
   }
 #undef DYHIP_NN_LOAD
+#pragma unroll
+  for (int t = 0; t < TILES; ++t) {  // this wavefront's sums, whole and to scale
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[t][r] = (acc[t][r] + low[t][r]) * kSplitOut;
+    if (__builtin_expect(any_not_finite(acc[t]), 0)) {
+      const unsigned n = min(ct * 32 + l32, B - 1);
+      sums16 s = {};
+      for (int which = 0; which < 2; ++which) {
+        const NnOperand& op = which == 0 ? op0 : op1;
+        const unsigned before = which == 0 ? 0 : C0;
+        const unsigned k0 = min(32 * (max(lo, before) - before), op.K), k1 = min(32 * (max(hi, before) - before), op.K);
+        add_products_fp32<true, false>(s, op.v + size_t(n) * op.ldv, op.ldv, op.W + row[t], op.ldw, k0, k1,
+                                       MASKED ? op.mask + size_t(n) * op.ldm : nullptr);
+      }
+      acc[t] = s;
+    }
+  }
   __syncthreads();  // the partial sums take the operands' place
 #pragma unroll
   for (int r = 0; r < 16; ++r) {
     const unsigned i = 8 * (r / 4) + 4 * lhi + (r % 4);
 #pragma unroll
-    for (int t = 0; t < TILES; ++t) red[(wave * ROWS + 32 * t + i) * kStepPitchR + l32] = acc[t][r] + low[t][r];
+    for (int t = 0; t < TILES; ++t) red[(wave * ROWS + 32 * t + i) * kStepPitchR + l32] = acc[t][r];
   }
   __syncthreads();
 #pragma unroll
@@ -1055,21 +1072,6 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_nn_deep_kernel(unsigned M, 
     float t = red[orow * kStepPitchR + col];
 #pragma unroll
     for (int w = 1; w < WAVES; ++w) t += red[(w * ROWS + orow) * kStepPitchR + col];
-    if (not_finite(t)) {  // formed again without the parts: see split3.h
-      t = 0.f;
-      const unsigned c0 = C * blockIdx.y / gridDim.y, c1 = C * (blockIdx.y + 1) / gridDim.y;  // this block's chunks
-      for (int which = 0; which < 2; ++which) {
-        const NnOperand& op = which == 0 ? op0 : op1;
-        const unsigned before = which == 0 ? 0 : C0;
-        const unsigned k0 = min(32 * (max(c0, before) - before), op.K), k1 = min(32 * (max(c1, before) - before), op.K);
-        const float* x = op.v + size_t(ecol) * op.ldv;
-        const float* m = MASKED ? op.mask + size_t(ecol) * op.ldm : nullptr;
-#pragma unroll 4
-        for (unsigned k = k0; k < k1; ++k) t = fmaf(op.W[erow + size_t(k) * op.ldw], MASKED ? x[k] * m[k] : x[k], t);
-      }
-    } else {
-      t *= kSplitOut;
-    }
     if (partial != nullptr) {
       partial[(size_t(blockIdx.y) * B + ecol) * M + erow] = t;
       continue;

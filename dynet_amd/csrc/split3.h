@@ -19,9 +19,14 @@
 // fp32 values reach down to 2^-149 (probabilities of a confident softmax are that small), so every operand is multiplied
 // by 2^16 on its way into the parts, exactly, and a sum by 2^-32 on its way out: all fp32 values are then split exactly,
 // subnormals included (at 2^-120, unscaled, a product was off by 4e-5, below 2^-134 it was zero).  The bf16 instructions
-// keep subnormal inputs and results.  Infinities, NaNs, operands from 2^111 on and sums from 2^96 on come out as
-// non-finite sums; the kernels form such an output again with plain fp32 multiply-adds (dot_fp32), so that infinities
-// keep their sign and huge values their value.
+// keep subnormal inputs and results.
+//
+// Infinities, NaNs, operands from 2^111 on and sums from 2^96 on come out as non-finite sums.  A wavefront that finds one
+// among its sums of a 32 x 32 tile forms that tile again over its part of the depth with the fp32 instruction, from memory
+// (add_products_fp32), so that infinities keep their sign and huge values their value.  A product full of NaNs takes two to
+// seven times as long as one of numbers: 10 000 x 4480 x 1024 0.49 -> 3.2 ms, 2051 x 2050 x 650 0.07 -> 0.18 ms, 1024 x
+// 512 x 784 16 -> 34 us (fp32 instruction alone: 0.71, 0.13 ms and 29 us; each output by itself, one multiply-add after
+// another: 97, 3.6 and 0.34 ms); one NaN in the first 1.1 ms.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -75,17 +80,95 @@ struct Split3 {
   }
 };
 
-__device__ __forceinline__ bool not_finite(float x) { return !(x - x == 0.f); }
-__device__ __forceinline__ bool not_finite(const float4& v) {
-  return !((v.x - v.x) + (v.y - v.y) + (v.z - v.z) + (v.w - v.w) == 0.f);
+typedef float sums16 __attribute__((ext_vector_type(16)));
+
+// Whether any lane holds a sum that is infinite or NaN (0 times it is not 0).
+template <typename T>
+__device__ __forceinline__ bool any_not_finite(const T& x) {
+  float z = 0.f;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) z = fmaf(x[r], 0.f, z);
+  return __any(!(z == 0.f));
 }
 
-// sum over k of a[k * step_a] * b[k * step_b], one multiply-add after another
-__device__ __forceinline__ float dot_fp32(const float* a, size_t step_a, const float* b, size_t step_b, unsigned K) {
-  float s = 0.f;
+// four values of a row, contiguous or ld apart
+template <bool KMAJOR>
+__device__ __forceinline__ float4 load4_fp32(const float* p, size_t ld) {
+  typedef float float4u __attribute__((ext_vector_type(4), aligned(4)));
+  if (KMAJOR) {
+    const float4u v = *reinterpret_cast<const float4u*>(p);
+    return make_float4(v[0], v[1], v[2], v[3]);
+  }
+  const __attribute__((address_space(1))) float* q = (const __attribute__((address_space(1))) float*)p;
+  float x[4];
+#pragma unroll
+  for (int c = 0; c < 4; ++c, q += ld) {
+    asm volatile("" : "+v"(q));  // one address at a time: the registers are full of sums
+    x[c] = *q;
+  }
+  return make_float4(x[0], x[1], x[2], x[3]);
+}
+
+// values `first` .. `first` + 3 of n, zeros from n on (read at the last one)
+template <bool KMAJOR>
+__device__ __forceinline__ float4 load4_fp32(const float* p, size_t ld, unsigned first, unsigned n) {
+  float x[4];
+#pragma unroll
+  for (unsigned c = 0; c < 4; ++c) {
+    const float v = p[min(first + c, n - 1) * (KMAJOR ? size_t(1) : ld)];
+    x[c] = first + c < n ? v : 0.f;
+  }
+  return make_float4(x[0], x[1], x[2], x[3]);
+}
+
+__device__ __forceinline__ void mma8_fp32(sums16& sum, const float4& a, const float4& b) {
+  sum = __builtin_amdgcn_mfma_f32_32x32x2f32(b.x, a.x, sum, 0, 0, 0);
+  sum = __builtin_amdgcn_mfma_f32_32x32x2f32(b.y, a.y, sum, 0, 0, 0);
+  sum = __builtin_amdgcn_mfma_f32_32x32x2f32(b.z, a.z, sum, 0, 0, 0);
+  sum = __builtin_amdgcn_mfma_f32_32x32x2f32(b.w, a.w, sum, 0, 0, 0);
+}
+
+// sum += the products of depth k0 .. k1 - 1 of a 32 x 32 tile, where a and b are this lane's (l % 32) row of the left and
+// column of the right operand; 32 k are fetched at a time.  mask: multiplies the row (stored along k, like it).
+template <bool AK, bool BKM>
+__device__ __forceinline__ void add_products_fp32(sums16& sum, const float* a, size_t lda, const float* b, size_t ldb,
+                                                  unsigned k0, unsigned k1, const float* mask = nullptr) {
+  const unsigned first = (threadIdx.x >> 3) & 4;  // lanes of the upper half take the second four of eight k
+  const size_t sa = AK ? 1 : lda, sb = BKM ? 1 : ldb;
+  a += size_t(k0) * sa;
+  b += size_t(k0) * sb;
+  if (mask != nullptr) mask += k0;
+  unsigned left = k1 > k0 ? k1 - k0 : 0;
 #pragma unroll 1
-  for (unsigned k = 0; k < K; ++k) s = fmaf(a[size_t(k) * step_a], b[size_t(k) * step_b], s);
-  return s;
+  for (; left >= 32; left -= 32) {
+    float4 x[4], y[4];
+#pragma unroll
+    for (unsigned i = 0; i < 4; ++i, a += 8 * sa, b += 8 * sb) {
+      x[i] = load4_fp32<AK>(a + first * sa, lda);
+      y[i] = load4_fp32<BKM>(b + first * sb, ldb);
+    }
+    if (mask != nullptr) {
+#pragma unroll
+      for (unsigned i = 0; i < 4; ++i, mask += 8) {
+        const float4 m = load4_fp32<true>(mask + first, 0);
+        x[i] = make_float4(x[i].x * m.x, x[i].y * m.y, x[i].z * m.z, x[i].w * m.w);
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);  // every load under way before the first is waited for
+#pragma unroll
+    for (unsigned i = 0; i < 4; ++i) mma8_fp32(sum, x[i], y[i]);
+  }
+#pragma unroll 1
+  for (; left > 0; left -= left < 8 ? left : 8, a += 8 * sa, b += 8 * sb) {
+    float4 x = load4_fp32<AK>(a, lda, first, left);
+    const float4 y = load4_fp32<BKM>(b, ldb, first, left);
+    if (mask != nullptr) {
+      const float4 m = load4_fp32<true>(mask, 0, first, left);
+      mask += 8;
+      x = make_float4(x.x * m.x, x.y * m.y, x.z * m.z, x.w * m.w);
+    }
+    mma8_fp32(sum, x, y);
+  }
 }
 
 }  // namespace dyhip

@@ -673,6 +673,9 @@ def test_lstm_cell_forward_backward(dev, I, H, B, dims, dropout, mask_full):
     (256, 256, 5, False, True), (34, 490, 33, False, True), (480, 32, 7, True, True), (650, 650, 20, True, True),
     (650, 650, 20, True, False), (62, 514, 40, True, True), (1024, 1024, 20, False, True), (1024, 1024, 128, True, True),
     (1024, 1024, 130, True, False), (30, 600, 9, True, True),
+    # more columns than those kernels take: 128 x 128 tiles and smaller ones, a split depth whose parts meet in the middle
+    # of a step's worth of the first product, first products that are not whole steps
+    (1030, 1024, 512, False, True), (1037, 1024, 300, True, True), (75, 96, 300, True, False),
 ])
 def test_gates_over_a_deep_sum(dev, I, H, B, dropout, mask_full):
     """Forward against the CPU path and fp64; dx and dh, which are added under the mask, against fp64.  Tolerances as in
@@ -704,6 +707,38 @@ def test_gates_over_a_deep_sum(dev, I, H, B, dropout, mask_full):
         dev.lstm_gates_backward([xt], [I], H, B, ht, Wxt, Wht, reft, dgt, i, gt, dpre=dpre, **kw)
         want = g0 + (d64 @ W.astype(np.float64).T) * (1.0 if m is None else m)
         assert_close(gt.numpy(), want, GRAD_RTOL, "gates bwd arg %d" % i, floor=max(1.0, float(np.sqrt(4 * H) * rms(W))))
+
+
+@pytest.mark.parametrize("I,H,B,dropout", [(650, 650, 20, False), (650, 650, 20, True), (1024, 1024, 128, True),
+                                           (1030, 1024, 512, False), (1037, 1024, 300, True), (75, 96, 300, False)])
+def test_gates_keep_infinities_nans_and_huge_values(dev, I, H, B, dropout):
+    """In either product, masked and not, over one block's depth and over several blocks': what fp32 arithmetic gives."""
+    rng = np.random.default_rng(I + H + B)
+    x, h, c_prev, Wx, Wh, b = _lstm_case(rng, I, H, B)
+    x[2, 5], x[4, I - 1], h[3, H - 2], h[1, 0] = np.inf, np.nan, -np.inf, np.nan
+    Wx[8, 30], Wh[11, 20] = 3.4e38, 3.4e38
+    x[:, 8] *= 1e-3
+    h[:, 11] *= 1e-3
+    mx = mh = None
+    kw = {}
+    if dropout:
+        mx, mh = f32(rng.integers(0, 2, (B, I)) * 2.0), f32(rng.integers(0, 2, (B, H)) * 2.0)
+        mx[2, 5], mh[3, H - 2] = 2.0, 0.0  # an infinity kept, and one dropped: NaN
+        kw = dict(mask_x=dev.tensor(mx), mask_x_bd=B, mask_h=dev.tensor(mh), mask_h_bd=B)
+    fx = dev.empty((B, 4 * H))
+    dev.lstm_gates_forward([dev.tensor(x)], [I], H, B, dev.tensor(h), dev.tensor(Wx), dev.tensor(Wh), dev.tensor(b), fx, **kw)
+    with np.errstate(all="ignore"):
+        want, _, _ = _lstm_exact_step(x, h, c_prev, Wx, Wh, b, mx, mh)
+    got = fx.numpy()[:, 3 * H:]  # the tanh gate: the sigmoids clamp what they are given
+    want = want[:, 3 * H:]
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.isnan(want).any()
+    fin = np.isfinite(want)
+    assert_close(got[fin], want[fin], FWD_RTOL, "g", floor=max(1.0, float(np.sqrt(I + H) * rms(c_prev * 0.1))))
+    rows = np.ones(B, bool)
+    rows[1:5] = False  # of the other gates the rows without infinities and NaNs
+    with np.errstate(all="ignore"):
+        full, _, _ = _lstm_exact_step(x[rows], h[rows], c_prev[rows], Wx, Wh, b, *(None if m is None else m[rows] for m in (mx, mh)))
+    assert_close(fx.numpy()[rows], full, FWD_RTOL, "gates", floor=max(1.0, float(np.sqrt(I + H) * 0.1)))
 
 
 # One timestep for up to 16 columns: a depth that gives some wavefronts nothing (H = 128 and nothing else: the kernel for
@@ -2177,6 +2212,56 @@ def test_gemm_split_products_keep_infinities_nans_and_huge_values(dev, M, N, K):
         assert_close(y[fin], want[fin], FWD_RTOL, form, floor=np.sqrt(K))
         col = np.isfinite(want[:, 20])
         assert_close(y[col, 20], want[col, 20], FWD_RTOL, form + ": the column of the huge value")
+
+
+# 128 x 128 tiles, 64 x 64, 64 x 32 and 32 x 32 with the item in the grid, ragged
+@pytest.mark.parametrize("M,N,K,B", [(260, 390, 100, 40), (300, 260, 150, 64), (70, 90, 200, 30), (33, 41, 133, 50)])
+def test_gemm_strided_batched_of_ordinary_size(dev, M, N, K, B):
+    """The three forms against fp64, with infinities, NaNs and huge values in some items."""
+    rng = np.random.default_rng(M + N + K + B)
+    l, r, y0 = (f32(rng.standard_normal(s)) for s in ((B, K, M), (B, N, K), (B, N, M)))
+    l[7, 5, 7], r[7, 9, K - 3], l[B - 1, 40, 20], r[B - 1, 3, 5], l[B // 2, 11, 20] = np.inf, -np.inf, np.nan, np.nan, 3.4e38
+    r[B // 2, :, 11] *= 1e-3
+    with np.errstate(all="ignore"):
+        want = r.astype(np.float64) @ l.astype(np.float64) + y0
+    for tl, tr in ((0, 0), (1, 0), (0, 1)):
+        lt = dev.tensor(f32(l.transpose(0, 2, 1)) if tl else l)
+        rt = dev.tensor(f32(r.transpose(0, 2, 1)) if tr else r)
+        yt = dev.tensor(y0)
+        dev.gemm_strided_batched(tl, tr, M, N, K, lt, M * K, rt, N * K, 1.0, yt, M * N, B)
+        y = yt.numpy()
+        assert np.array_equal(np.isnan(y), np.isnan(want)), (tl, tr)
+        inf = np.isinf(want)
+        assert inf.any() and np.array_equal(np.isinf(y), inf) and np.array_equal(y[inf], want[inf].astype(np.float32))
+        fin = np.isfinite(want)
+        fin[B // 2, :, 20] = False
+        assert_close(y[fin], want[fin], FWD_RTOL, "finite outputs", floor=np.sqrt(K))
+        assert_close(y[B // 2, :, 20], want[B // 2, :, 20], FWD_RTOL, "the column of the huge value")
+        for w in lib_pools():
+            dev.free_pool(w)
+
+
+@pytest.mark.parametrize("form,M,N,K", [("nn", 4352, 4096, 512), ("tn", 1024, 1024, 8192), ("nt", 2051, 2050, 650),
+                                        ("nn", 1024, 512, 784)])
+def test_gemm_of_nans_takes_a_few_times_as_long_as_of_numbers(dev, form, M, N, K):
+    """A training step whose activations have become NaN: 2 to 7 times (3.3 to 4.5 times the fp32 instruction's time); 20 to
+    200 times when each output is formed by itself, one product after another."""
+    rng = np.random.default_rng(M)
+    l, r, y = dev.tensor(f32(rng.standard_normal((K, M)))), dev.tensor(f32(rng.standard_normal((N, K)))), dev.empty((N, M))
+    nans = dev.empty((N, K))
+    dev.constant(nans, float("nan"))
+
+    def best(op):
+        times = []
+        for _ in range(4):
+            dev.timer_start()
+            getattr(dev, "gemm_" + form)(M, N, K, l, op, 0.0, y)
+            times.append(dev.timer_stop())
+        return min(times)
+
+    of_nans = best(nans)
+    assert np.isnan(y.numpy()).all()
+    assert of_nans <= 14 * best(r)
 
 
 # Edges of the tiles of ordinary products: fewer than four rows (or columns) in the last tile or in the whole matrix, groups
