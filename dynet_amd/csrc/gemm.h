@@ -91,7 +91,8 @@ int gemm_slices_sum(dyhip_device* dev, size_t M, size_t N, unsigned splits, cons
 
 // gemm_small.hip: one-launch products for operands of a few hundred KB, any layout, single or strided-batched, with
 // the axpby or the bias epilogue.
-bool gemm_small_eligible(const dyhip_device* dev, size_t M, size_t N, size_t K, const GemmEpiParams& epi, unsigned batch);
+bool gemm_small_eligible(const dyhip_device* dev, bool a_kmajor, bool b_kmajor, size_t M, size_t N, size_t K,
+                         const GemmEpiParams& epi, unsigned batch);
 int gemm_small_run(dyhip_device* dev, bool a_kmajor, bool b_kmajor, size_t M, size_t N, const GemmSeg& s, float* C,
                    const GemmEpiParams& epi, const GemmBatch* batch);
 

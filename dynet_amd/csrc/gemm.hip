@@ -71,7 +71,7 @@ struct MidConfig {
 //                                           measured at
 constexpr MidConfig kMidConfigs[] = {
     {1, 1, 4, 3, 4.6, {5.8, 10.3, 15.0}},   // 1024 x 512 x 784: 11.8, x 2048: 24.1
-    {1, 1, 8, 2, 4.6, {5.5, 10.5, 0.0}},    // 50 x 512 x 1024 in 8 parts: 8.1 with the sum of the parts
+    {1, 1, 8, 1, 4.6, {5.5, 0.0, 0.0}},     // 50 x 512 x 1024 in 8 parts: 8.1 with the sum of the parts
     {2, 1, 4, 2, 4.9, {9.1, 17.8, 0.0}},    // 1024 x 512 x 2048: 23.9; 1024 x 1024 x 512: 14.1
     {2, 1, 8, 1, 4.9, {8.2, 0.0, 0.0}},     // 1024 x 512 x 1024: 13.0, x 4096: 38.2
     {2, 2, 4, 2, 5.5, {14.5, 31.0, 0.0}},   // 4096 x 256 x 4480: 69.3; 2048 x 2240 x 512: 47.0
@@ -971,7 +971,7 @@ int gemm_run(dyhip_device* dev, bool a_kmajor, bool b_kmajor, size_t M, size_t N
     DYHIP_REQUIRE(batch->stride_c >= M * N, "batch items of the GEMM output overlap");
   }
   if (nseg == 1 && !to_caller && C != nullptr && segs[0].A != nullptr && segs[0].B != nullptr &&
-      gemm_small_eligible(dev, M, N, segs[0].K, epi, batch ? batch->count : 1))
+      gemm_small_eligible(dev, a_kmajor, b_kmajor, M, N, segs[0].K, epi, batch ? batch->count : 1))
     return gemm_small_run(dev, a_kmajor, b_kmajor, M, N, segs[0], C, epi, batch);
   size_t K = 0;
   for (int s = 0; s < nseg; ++s) {

@@ -50,17 +50,19 @@ struct DirectOperand {
   Off off[KMAJOR ? L : 1];
   unsigned K, rows;              // depth; rows inside the matrix from the tile's first
   // Groups of four rows past the matrix edge are moved to its last four rows; one that straddles the edge is shifted back
-  // into place on its way to LDS.  few: fewer than four rows, every load is checked (uniform).
-  unsigned shift;
+  // into place on its way to LDS.  back: rows before the tile that its only group then starts at.  few: the matrix has fewer
+  // than four rows, every load is checked (uniform).
+  unsigned shift, back;
   bool straddles, few;
 
   __device__ __forceinline__ void init(const float* p, size_t ld_, unsigned K_, unsigned mn0, unsigned MN, unsigned lane) {
     ld = ld_;
     K = K_;
     rows = MN - mn0;
-    base = p + (KMAJOR ? size_t(mn0) * ld : size_t(mn0));
     straddles = !KMAJOR && rows < 32 * T && rows % 4 != 0;
-    few = !KMAJOR && rows < 4;
+    few = !KMAJOR && rows < 4 && mn0 == 0;
+    back = !KMAJOR && rows < 4 && mn0 > 0 ? 4 - rows : 0;
+    base = p + (KMAJOR ? size_t(mn0) * ld : size_t(mn0 - back));
     shift = 0;
     if (KMAJOR) {
 #pragma unroll
@@ -68,7 +70,7 @@ struct DirectOperand {
     } else {
       const unsigned r0 = 4 * (lane % (8 * T)), moved = min(r0, rows >= 4 ? rows - 4 : 0u);
       off[0] = 4 * (Off(lane / (8 * T)) * Off(ld) + moved);
-      shift = min(r0 - moved, 3u);  // (3: a group wholly past the edge, whatever it holds)
+      shift = min(r0 - moved + back, 3u);  // (3: a group wholly past the edge, whatever it holds)
     }
   }
   __device__ __forceinline__ void load(float4u (&v)[L], unsigned step) const {
@@ -89,7 +91,7 @@ struct DirectOperand {
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
         const unsigned r = min(KMAJOR ? r0 : r0 + c, rows - 1), k = KMAJOR ? k0 + c : k0;
-        const float x = base[KMAJOR ? size_t(r) * ld + min(k, K - 1) : size_t(min(k, K - 1)) * ld + r];
+        const float x = base[KMAJOR ? size_t(r) * ld + min(k, K - 1) : size_t(min(k, K - 1)) * ld + back + r];
         v[i][c] = k < K ? x : 0.f;
       }
     }

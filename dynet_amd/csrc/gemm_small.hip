@@ -69,8 +69,10 @@ __device__ __forceinline__ void small_fetch(const float* __restrict__ p, size_t 
 
 constexpr int kSmallGroups = 4;  // groups of eight depth indices a stage: 32 indices, 16 values of each operand a lane
 
-// KW: wavefronts that split the depth of one tile (8 or 4; the block has KW wavefronts), or 1: four wavefronts, a tile
-// each.  The next stage's loads are issued before the current stage's matrix-core steps.
+// KW: wavefronts that split the depth of one tile (8 or 4; the block has KW wavefronts), the next stage's loads issued
+// before the current stage's matrix-core steps; or 1: four wavefronts, a tile each, one or two stages straight through, in
+// 48 registers instead of 114: eight wavefronts a SIMD instead of four (6464 x 1251 x 9: 20.5 -> 16.6 us, 5280 x 908 x 64
+// 17.5 -> 14.9; with all of a stage's loads under way before the first product, in 64 registers, 20.9 for the former).
 template <int AVEC, int BVEC, int KW>
 __global__ __launch_bounds__(KW == 1 ? 256 : 64 * KW) void gemm_small_kernel(SmallGemmArgs g) {
   __shared__ float red[KW > 1 ? KW * 16 * 64 : 1];
@@ -102,7 +104,14 @@ __global__ __launch_bounds__(KW == 1 ? 256 : 64 * KW) void gemm_small_kernel(Sma
     }
   };
   fetch(a0, b0, kbeg);
-  for (unsigned k0 = kbeg; k0 < kend; k0 += 16 * T) {
+  if (KW == 1) {
+    steps(a0, b0, kbeg);
+    if (kend > kbeg + 8 * T) {  // uniform
+      fetch(a1, b1, kbeg + 8 * T);
+      steps(a1, b1, kbeg + 8 * T);
+    }
+  }
+  for (unsigned k0 = kbeg; KW > 1 && k0 < kend; k0 += 16 * T) {
     fetch(a1, b1, k0 + 8 * T);
     steps(a0, b0, k0);
     fetch(a0, b0, k0 + 16 * T);
@@ -147,21 +156,30 @@ static int small_depth_waves(size_t K, size_t tiles, size_t cus) {
   return K >= 512 && tiles <= 2 * cus ? 8 : 4;
 }
 
-// Which products come here instead of gemm_direct.hip (measured on 17 shapes in the three layouts).  A wavefront's depth
-// costs one memory round trip per stage of 32 indices, hidden only by other blocks on the CU, and the fp32 matrix
-// instruction: good for one stage (512 x 300 x 100: 3.8 against 4.6 us), for two of them on few tiles (256 x 256 x 256:
-// 4.9 against 4.8..5.2; 512 x 512 x 512: 10.0 / 8.5 / 6.5 against 7.1 / 7.6 / 6.8) or on more than two one-wavefront tiles
-// per CU (2000 x 500 x 40: 5.7 against 7.1; 1024 x 512 x 50, two: 5.5..6.0 against 5.0..5.2).
-bool gemm_small_eligible(const dyhip_device* dev, size_t M, size_t N, size_t K, const GemmEpiParams& epi, unsigned batch) {
+// Which products come here instead of gemm_direct.hip and gemm_tile.hip (measured on 500 shapes in the three layouts).  A
+// wavefront's depth costs one memory round trip per stage of 32 indices, hidden only by other blocks on the CU, and the
+// fp32 matrix instruction.  A depth of one stage: always, the time is that of the output (3703 x 4288 x 28: 25 us against
+// 40 and more; 224 x 362 x 11 times 439 items 55 against 91; 1536 x 3654 x 2 12 against 19).  Deeper: one stage a wavefront
+// (512 x 300 x 100: 3.8 against 4.6 us), two of them on few tiles (256 x 256 x 256: 4.9 against 4.8..5.2; 512 x 512 x 512:
+// 10.0 / 8.5 / 6.5 against 7.1 / 7.6 / 6.8) or on more than two one-wavefront tiles per CU (2000 x 500 x 40: 5.7 against
+// 7.1; 1024 x 512 x 50, two: 5.5..6.0 against 5.0..5.2; 5856 x 1536 x 64 23.9 against 32.9; but as l^T*r off the 16-byte
+// grid, 2480 x 2080 x 49, 28.4 against 20.8), three for one to three rows or columns stored along them, whose steps are all
+// checked ones there (2 x 5888 x 288: 6.7 against 8.7; 64 x 1 x 353 times 131 items 8.2 against 11; four: 2 x 217 x 800
+// 10.3 against 7.9).
+bool gemm_small_eligible(const dyhip_device* dev, bool a_kmajor, bool b_kmajor, size_t M, size_t N, size_t K,
+                         const GemmEpiParams& epi, unsigned batch) {
   if (epi.kind != kEpiAxpby && !(epi.kind == kEpiBias && epi.bias != nullptr)) return false;
-  if (M == 0 || N == 0 || K == 0 || M > (size_t(1) << 20) || N > (size_t(1) << 20) || K > 65536 || batch > 65535u) return false;
+  if (M == 0 || N == 0 || K == 0 || N > (size_t(1) << 20) || K > 65536 || batch > 65535u) return false;
+  if (K <= 8 * kSmallGroups && M <= (size_t(1) << 30)) return true;
+  if (M > (size_t(1) << 20)) return false;
   const size_t cus = dev->num_cus > 0 ? size_t(dev->num_cus) : 256;
   const size_t tiles = cdiv<size_t>(M, 32) * cdiv<size_t>(N, 32) * (batch > 0 ? batch : 1);
   const size_t work = tiles * cdiv<size_t>(K, 32);  // in units of one tile x one stage
-  if (tiles > 16 * cus || work > 64 * cus) return false;
   const int waves = small_depth_waves(K, tiles, cus);
+  if (waves == 1 && tiles > 2 * cus && (K % 4 == 0 || !a_kmajor)) return true;
+  if (tiles > 16 * cus || work > 64 * cus) return false;
   const size_t stages = cdiv<size_t>(cdiv<size_t>(K, waves), 8 * kSmallGroups);
-  return stages <= 1 || (stages <= 2 && (tiles < cus || (waves == 1 && tiles > 2 * cus)));
+  return stages <= 1 || (stages <= 2 && (tiles < cus || (waves == 1 && tiles > 2 * cus))) || (stages <= 3 && ((!a_kmajor && M < 4) || (!b_kmajor && N < 4)));
 }
 
 int gemm_small_run(dyhip_device* dev, bool a_kmajor, bool b_kmajor, size_t M, size_t N, const GemmSeg& s, float* C,
@@ -198,9 +216,9 @@ int gemm_small_run(dyhip_device* dev, bool a_kmajor, bool b_kmajor, size_t M, si
   const dim3 grid(kwaves > 1 ? tm : cdiv<unsigned>(tm, 4), tn, items);
 #define DYHIP_SMALL_KW(AV, BV)                                                                                       \
   do {                                                                                                               \
-    if (kwaves == 8) hipLaunchKernelGGL((gemm_small_kernel<AV, BV, 8>), grid, dim3(512), 0, dev->stream, g);         \
-    else if (kwaves == 4) hipLaunchKernelGGL((gemm_small_kernel<AV, BV, 4>), grid, dim3(256), 0, dev->stream, g);    \
-    else hipLaunchKernelGGL((gemm_small_kernel<AV, BV, 1>), grid, dim3(256), 0, dev->stream, g);                     \
+    if (kwaves == 8) hipLaunchKernelGGL((gemm_small_kernel<AV, BV, 8>), grid, dim3(512), 0, dev->stream, g);                \
+    else if (kwaves == 4) hipLaunchKernelGGL((gemm_small_kernel<AV, BV, 4>), grid, dim3(256), 0, dev->stream, g);           \
+    else hipLaunchKernelGGL((gemm_small_kernel<AV, BV, 1>), grid, dim3(256), 0, dev->stream, g);                            \
   } while (0)
 #define DYHIP_SMALL_B(AV)                     \
   do {                                        \

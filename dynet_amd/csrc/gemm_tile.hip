@@ -54,10 +54,11 @@ __global__ __launch_bounds__(256, 2) void gemm_tile_kernel(TileArgs g) {
   const bool kmajor = AK == BKM ? AK : stage_b ? BKM : AK;
   const unsigned w2 = w & 1, mn0 = stage_b ? n0 : m0, rows = (stage_b ? g.N : g.M) - mn0;
   // First of a lane's rows, and its k inside a step.  Groups of four rows that reach past the matrix edge are moved to its
-  // last four, and written to those rows' slots (by several lanes then, with the same values).
-  const unsigned row0 = kmajor ? 16 * w2 + lane / 4 : min(4 * (lane % 32), rows >= 4 ? rows - 4 : 0u);
+  // last four, and written to those rows' slots (by several lanes then, with the same values); rows before the tile, where
+  // fewer than four are left, to slots past the edge.
+  const unsigned row0 = kmajor ? 16 * w2 + lane / 4 : rows >= 4 ? min(4 * (lane % 32), rows - 4) : mn0 > 0 ? rows - 4 : 0u;
   const unsigned quarter = kmajor ? lane % 4 : 2 * w2 + lane / 32, half = quarter / 2;
-  const bool few = !kmajor && rows < 4;
+  const bool few = !kmajor && rows < 4 && mn0 == 0;
   unsigned load_at = s0, load_end = 0, load_k = 0, Kseg = 0;  // next step; end of its segment; its k; the segment's depth
   size_t ld = 0, off[4];
   const float* op = nullptr;  // the segment's operand at the tile's first row
@@ -78,7 +79,7 @@ __global__ __launch_bounds__(256, 2) void gemm_tile_kernel(TileArgs g) {
          (kmajor ? size_t(mn0) * ld : size_t(mn0));                                                      \
     load_k = (load_at - first_) * 16;                                                                    \
     _Pragma("unroll") for (int j_ = 0; j_ < 4; ++j_) off[j_] =                                           \
-        kmajor ? size_t(min(row0 + 32 * j_, rows - 1)) * ld + 4 * quarter : row0 + size_t(4 * quarter + j_) * ld; \
+        kmajor ? size_t(min(row0 + 32 * j_, rows - 1)) * ld + 4 * quarter : size_t(ptrdiff_t(int(row0))) + size_t(4 * quarter + j_) * ld; \
   }
   float4u raw[4];
   // loads past the block's last step repeat it
@@ -108,7 +109,7 @@ __global__ __launch_bounds__(256, 2) void gemm_tile_kernel(TileArgs g) {
   ob[0] = kTileOperand + frag + wn * 1024;
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
-    const unsigned row = row0 + (kmajor ? 32 * j : j), slot = kmajor ? row : 32 * (row % 4) + row / 4;
+    const unsigned row = (row0 + (kmajor ? 32 * j : j)) % kTileT, slot = kmajor ? row : 32 * (row % 4) + row / 4;
     ow[j] = (stage_b ? kTileOperand : 0u) + half * 2048 + (slot ^ (4 * half)) * 16 + (quarter % 2) * 8;
   }
   oa[1] = oa[0] + kTileStage;
@@ -148,6 +149,14 @@ __global__ __launch_bounds__(256, 2) void gemm_tile_kernel(TileArgs g) {
       for (int r = 0; r < 16; ++r) acc[u][t][r] = low[u][t][r] = 0.f;
 
   if (s0 < s1) {
+    if (!kmajor && rows < kTileT) {
+      // Slots past the edge are never written.  Their outputs are dropped, but must not look like sums that are not finite:
+      // zeros in this wavefront's half of them.
+#pragma unroll
+      for (unsigned x = 0; x < 12; ++x)
+        *reinterpret_cast<uint4*>(lds + (stage_b ? kTileOperand : 0u) + half * 2048 + x / 6 * kTileStage + x % 6 / 2 * kTilePlane +
+                                  x % 2 * 1024 + lane * 16) = make_uint4(0, 0, 0, 0);
+    }
     DYHIP_TILE_SEG
     DYHIP_TILE_LOAD
 #pragma unroll

@@ -2241,6 +2241,40 @@ def test_gemm_strided_batched_of_ordinary_size(dev, M, N, K, B):
             dev.free_pool(w)
 
 
+def _best_time(dev, call, runs=5):
+    times = []
+    for _ in range(runs):
+        dev.timer_start()
+        for _ in range(4):
+            call()
+        times.append(dev.timer_stop())
+    return min(times)
+
+
+@pytest.mark.parametrize("M,N,K,B", [(3703, 4288, 28, 1), (224, 362, 11, 439), (1536, 3654, 2, 1), (8070, 1238, 24, 1)])
+def test_shallow_products_take_the_time_of_their_output(dev, M, N, K, B):
+    """A depth of at most 32: against filling the output (2 times its time; 4 to 6 times with a block a 32 x 32 tile)."""
+    l, r, y = dev.empty((B, K, M)), dev.empty((B, N, K)), dev.empty((B, N, M))
+    dev.constant(l, 0.5)
+    dev.constant(r, 2.0)
+    fill = _best_time(dev, lambda: dev.constant(y, 0.0))
+    product = _best_time(dev, lambda: dev.gemm_strided_batched(0, 0, M, N, K, l, M * K, r, N * K, 0.0, y, M * N, B))
+    assert (y.numpy() == K).all()
+    assert product <= 3.5 * fill
+
+
+def test_ragged_tiles_take_no_longer_than_whole_ones(dev):
+    """128 x 128 tiles: what a block holds past the matrix edge must not send it the way of infinities and NaNs."""
+    K = 672
+    times = []
+    for M, N in ((2336, 1472), (2432, 1536)):
+        l, r, y = dev.empty((K, M)), dev.empty((N, K)), dev.empty((N, M))
+        dev.constant(l, 0.5)
+        dev.constant(r, 2.0)
+        times.append(_best_time(dev, lambda: dev.gemm_nt(M, N, K, l, r, 0.0, y)))
+    assert times[0] <= 1.5 * times[1]
+
+
 @pytest.mark.parametrize("form,M,N,K", [("nn", 4352, 4096, 512), ("tn", 1024, 1024, 8192), ("nt", 2051, 2050, 650),
                                         ("nn", 1024, 512, 784)])
 def test_gemm_of_nans_takes_a_few_times_as_long_as_of_numbers(dev, form, M, N, K):
