@@ -3,14 +3,20 @@
 // alignment: everything between the streaming kernels for a few rows or columns and the 256 x 256-tile kernel.
 //
 // A block owns a tile of 32*TM x 32*TN outputs; its wavefronts split the depth, each multiplies the whole tile over its
-// part, and they meet in LDS once, at the end.  Operands go from memory (the L2s, mostly) straight into the registers
-// that feed the matrix cores: no LDS stage, no barrier in the loop.  fp32 in and out, on the bf16 matrix cores with every
-// operand as three bf16 values (split3.h); depths below 32 on the fp32 instruction, whose error is the smaller there.
+// part, and they meet in LDS once, at the end: no barrier in the loop.  fp32 in and out, on the bf16 matrix cores with every
+// operand as three bf16 values (split3.h); depths below 32, which only a batch of more than 65 535 items, slices for another
+// kernel and gates of a handful of inputs bring here, on the fp32 instruction in one form.
 //
-// Fragment of a 16-deep step: lane 32*lhi + l32 holds k = 8*lhi .. 8*lhi + 7 of row (column) l32: two 128-bit loads where
-// the operand is contiguous along k (dword-aligned is enough), eight 32-bit loads over 32 neighbouring lanes each where
-// it is contiguous along its rows.  Two steps are in flight.  Rows past the matrix are read at a clamped row and their
-// outputs dropped; a depth that is not a multiple of 16 ends in a step of clamped, zeroed loads.
+// Step of 16 k: 128-bit loads (dword-aligned is enough) in the order of memory, written to a piece of LDS that is the
+// wavefront's own, read from there as fragments (lane 32*lhi + l32 holds k = 8*lhi .. 8*lhi + 7 of row l32), split in
+// registers.  Four steps of loads are in flight and a step crosses LDS under the products of the one before it; with 2 x 2
+// tiles, whose accumulators and fragments fill the registers, one, and it is read when its fragments are formed (1024^3
+// 20.8 -> 22.2 us, against 26.4 with the sums of a step by themselves, which spilled).  Rows past the matrix are read at a
+// clamped row and their outputs dropped; a depth that is not a multiple of 16 ends in a step of clamped, zeroed loads.
+//
+// What bounds it: the latency of a step's way through memory, LDS and the split, with one to three wavefronts a SIMD to
+// cover it.  us in a graph, fp32 instruction in 128-wide tiles -> here: 1024 x 512 x 784 l*r 22.3 -> 13.5, 1024 x 784 x 512
+// l*r^T 24.2 -> 14.9, 1024^3 33.6 -> 22.4.
 #include <algorithm>
 #include <type_traits>
 

@@ -942,8 +942,8 @@ __global__ __launch_bounds__(256) void skinny_nn_kernel(unsigned M, unsigned H, 
 
 // The same product for depths of kNnDeep and more, on the bf16 matrix cores (split3.h).  At a small batch the kernel
 // above has fewer blocks than the GPU has CUs (82 at H = 650), and a wavefront walks a quarter of the depth in rounds of
-// loads that nothing hides.  Here the depths of both products, laid end to end in chunks of 32 k, are dealt to sixteen
-// (eight with 64 rows) wavefronts; each has its next chunk in flight.  v comes in whole 128-byte lines, eight columns an
+// loads that nothing hides.  Here the depths of both products, laid end to end in chunks of 32 k, are dealt to eight
+// wavefronts; each has its next chunk in flight.  v comes in whole 128-byte lines, eight columns an
 // instruction, and goes through a wavefront's own piece of LDS into fragments: read in fragment order, 32 columns x 32
 // bytes an instruction, its line lookups alone took as long as the product.
 // MASKED: v is multiplied by its dropout mask on the way in, which saves the launches that would form the products.
@@ -1096,12 +1096,12 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_nn_deep_kernel(unsigned M, 
 // 25.7 us).  Not for a block that would walk more than 2 MB of weights alone (a few rows over a very long depth), nor
 // for odd depths (v's fragments are 128-bit loads along k, or two 64-bit ones).
 //
-// skinny_nn_deep_kernel from a depth of 512 (I = H = 256, B = 20: 5.8 -> 5.6, where its gain ends) while its blocks are
-// one round of the CUs (us in a graph, before and after): gates forward, I = H = 650, B = 20 with dropout 16.3 -> 11.4
-// (three launches, now two: three blocks share the depth), I = H = 1024, B = 64 14.8 -> 14.1, B = 128 23.4 -> 21.6,
-// I = H = 512, B = 32 8.6 -> 8.0; affine 1024 x 64 x 1024 8.3 -> 7.7, 2000 x 20 x 4096 23.4 -> 14.3 (four blocks share
-// the depth), 10 000 x 32 x 1024 14.8 -> 14.6.  More blocks than CUs lose: 10 000 x 64 x 512 18.6 -> 19.0.  Bound by what
-// a CU can have in flight towards the Infinity Cache (20-25 GB/s of weights a CU): only more CUs a weight help.
+// skinny_nn_deep_kernel from a depth of 512 while its blocks are one round of the CUs, where it takes the masks or several
+// blocks share the depth (us in a graph, before and after): gates forward, I = H = 650, B = 20 with dropout 16.0 -> 11.6
+// (three launches, now two: three blocks share the depth), B = 40 18.7 -> 16.4, I = H = 1024, B = 20 13.8 -> 12.6; affine
+// 2000 x 20 x 4096 23.3 -> 14.6 (four blocks).  Without either the kernel above is as fast or faster: I = H = 1024, B = 64
+// 14.6 against 15.3, B = 128 23.3 against 23.4; 10 000 x 32 x 1024 14.8 against 15.4.  Bound by what a CU can have in flight
+// towards the Infinity Cache (20-25 GB/s of weights a CU): only more CUs a weight help.
 constexpr size_t kNnDeep = 512;
 
 int skinny_nn_gemm(dyhip_device* dev, size_t M, size_t N, int nseg, const GemmSeg* segs, float* C, const GemmEpiParams& epi,
@@ -1134,13 +1134,17 @@ int skinny_nn_gemm(dyhip_device* dev, size_t M, size_t N, int nseg, const GemmSe
                                  : NnOperand{segs[0].A, segs[0].B, 0u, segs[0].lda, segs[0].ldb, m0.p, m0.ld};
   const dim3 grid(cdiv<unsigned>(unsigned(M), 32 * tiles) * ct), block(256);
   const float beta = kind == kNnAxpby ? epi.beta : 0.f;
+  // Few blocks: the depth over several of them, whose slices a second launch adds up.  The host pays for that launch too, so
+  // only where it is worth much, or where the masks have saved two.
+  unsigned splits = 0;  // 0: not that kernel
   if (Kt >= kNnDeep && segs[0].K >= 32 && segs[nseg - 1].K >= 32 && grid.x <= cus) {
-    // Few blocks: the depth over several of them, whose slices a second launch adds up.  The host pays for that launch
-    // too, so only where it is worth much, or where the masks have saved two.
+    splits = 1;
     const size_t least = masks != nullptr ? 384 : 1024;
-    unsigned splits = 1;
     while (grid.x * (splits + 1) <= cus && Kt / (splits + 1) >= least) ++splits;
     if (dev->gemm_ws == nullptr || dev->gemm_ws_bytes < sizeof(float) * M * N * splits) splits = 1;
+    if (splits == 1 && masks == nullptr) splits = 0;
+  }
+  if (splits > 0) {
     float* const partial = splits > 1 ? static_cast<float*>(dev->gemm_ws) : nullptr;
 #define DYHIP_NN_DEEP(T, E, MK)                                                                                          \
   hipLaunchKernelGGL((skinny_nn_deep_kernel<T, 8, E, MK>), dim3(grid.x, splits), dim3(512), 0, dev->stream, unsigned(M), epi.H, \

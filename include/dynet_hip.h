@@ -233,7 +233,7 @@ int dyhip_layer_norm_backward(dyhip_device* dev, size_t n, unsigned bd, const fl
 int dyhip_layer_norm_backward_static(dyhip_device* dev, size_t n, unsigned bd, const float* x, const float* g,
                                      const float* dEdf, float* dx, float* dg, float* db);
 
-/* ---- GEMM shim: dynet/matrix-multiply.h, fp32 in / fp32 accumulate on MFMA.
+/* ---- GEMM shim: dynet/matrix-multiply.h, fp32 in / fp32 accumulate on the matrix cores.
  * The device-pointer acc_scalar of the reference (kSCALAR_ONE / kSCALAR_ZERO)
  * becomes the by-value beta. ---------------------------------------------- */
 /* MatrixMultiply (:16-37): y[MxN] = beta*y + l[MxK] * r[KxN] */
@@ -245,7 +245,7 @@ int dyhip_gemm_nt_acc(dyhip_device* dev, size_t M, size_t N, size_t K, const flo
 /* Which kernel the three calls above take for a problem with packed leading dimensions and 16-byte aligned
  * operands: *wide_tiles = 1 when the 256 x 256-tile kernel takes the whole product (large outputs with enough
  * depth per CU), 2 when it takes the leading columns that form full rounds of one tile per CU and the rest runs
- * as a product of its own, 0 for the 128-wide kernel or the fragment-order product.  trans_l / trans_r as in
+ * as a product of its own, 0 for any other kernel.  trans_l / trans_r as in
  * dyhip_gemm_strided_batched.  No counterpart in the reference (cuBLAS picks its kernels silently); for tests
  * and tuning. */
 int dyhip_gemm_uses_wide_tiles(dyhip_device* dev, int trans_l, int trans_r, size_t M, size_t N, size_t K, int* wide_tiles);

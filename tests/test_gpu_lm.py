@@ -144,7 +144,7 @@ def test_lm_dropout_inside_a_captured_step_draws_new_masks_on_every_replay(dev):
 @pytest.fixture(scope="module")
 def wide_case():
     """The LM configuration's layer widths (E = 256, H = 1024, two layers, B = 128: the sizes that select the
-    production kernels - 128-wide GEMM tiles, the single-launch timestep, split-K recurrent products) with a
+    production kernels - large GEMM tiles, the single-launch timestep, split-K recurrent products) with a
     vocabulary and a sequence length small enough for one CPU core: the oracle step takes ~10 s, once."""
     V, E, H, L, B, T = 300, 256, 1024, 2, 128, 3
     rng = np.random.default_rng(23)

@@ -205,7 +205,7 @@ def test_gemm_nn_mid(dev, M, N, K):
 
 # Large outputs go to the 256 x 256-tile kernel, which deals the k-tiles of all tiles to the CUs in equal segments:
 # (a) fewer tiles than CUs: every tile spans several segments, whose partial tiles a second kernel adds; ragged edges
-# and a depth that is not a multiple of 32 (the rest of the depth is added by the 128-wide kernel); (b), (c) a little
+# and a depth that is not a multiple of 32 (the rest of the depth is added by a product of its own); (b), (c) a little
 # more than one tile, and about two shallow tiles, per CU: a cut tile is finished inside the kernel; (d) a transposed
 # left operand whose row count is not a multiple of 4.
 # Checked against the fp64 product of the same fp32 inputs (the oracle's triple loop is the same sum, too slow here).
@@ -777,7 +777,7 @@ def test_step_of_a_few_columns(dev, I, H, B):
     assert np.array_equal(hp_out.numpy()[cols], want_hp.numpy()[cols])
 
 
-@pytest.mark.parametrize("M,N,K", [(333, 9, 2100), (70, 33, 514), (1000, 20, 640)])
+@pytest.mark.parametrize("M,N,K", [(333, 9, 2100), (70, 33, 514), (70, 33, 2050), (1000, 20, 640)])
 def test_deep_sums_of_a_small_batch_keep_infinities_and_nans(dev, M, N, K):
     """The affine layer where operands are infinite, NaN or next to FLT_MAX: what fp32 arithmetic gives."""
     rng = np.random.default_rng(M)
@@ -2163,7 +2163,7 @@ def test_gemm_split_products_have_fp32_precision_over_the_exponent_range(dev, M,
         assert np.linalg.norm(err) <= 0.5 * np.sqrt(K) * 2.0 ** -24 * np.linalg.norm(exact), form
 
 
-@pytest.mark.parametrize("M,N,K", SPLIT_GEMM_SHAPES + [(1000, 20, 640)])  # the last: the deep sum of a small batch
+@pytest.mark.parametrize("M,N,K", SPLIT_GEMM_SHAPES + [(333, 9, 2100)])  # the last: the deep sum of a small batch
 @pytest.mark.parametrize("e", [-112, -126, -140])
 def test_gemm_split_products_keep_the_bits_of_tiny_values(dev, M, N, K, e):
     """Operands of the size 2^e, subnormals at 2^-140, times large ones: products of ordinary size, to the same bound as
@@ -2175,7 +2175,7 @@ def test_gemm_split_products_keep_the_bits_of_tiny_values(dev, M, N, K, e):
         assert np.linalg.norm(y - exact) <= 0.5 * np.sqrt(K) * 2.0 ** -24 * np.linalg.norm(exact), form
 
 
-@pytest.mark.parametrize("M,N,K", SPLIT_GEMM_SHAPES + [(1000, 20, 640)])
+@pytest.mark.parametrize("M,N,K", SPLIT_GEMM_SHAPES + [(333, 9, 2100)])
 @pytest.mark.parametrize("density", [1.0, 0.5, 0.25, 0.1])
 def test_gemm_split_products_of_sparse_operands_are_as_close_as_fp32(dev, M, N, K, density):
     """Zeros (of a rectifier, of dropout) take roundings from an fp32 sum.  The bound is what one rounding to nearest a
@@ -2188,6 +2188,24 @@ def test_gemm_split_products_of_sparse_operands_are_as_close_as_fp32(dev, M, N, 
     bound = np.sqrt(0.2 + 0.09 * density * K) * 2.0 ** -24 * np.linalg.norm(exact)
     for form, y in _three_forms(dev, M, N, K, l, r, np.zeros((N, M), np.float32), 0.0):
         assert np.linalg.norm(y - exact) <= bound, form
+
+
+# the 256 x 256-tile kernel, 128 x 128 tiles, smaller ones, the deep sum of a small batch
+@pytest.mark.parametrize("M,N,K", [(4096, 4096, 512), (2304, 2176, 96), (300, 260, 256), (1000, 40, 2048)])
+def test_gemm_splits_every_value_exactly(dev, M, N, K):
+    """Times a matrix with one 1 a column: the parts of a value add up to it, bit for bit.  Random bit patterns, subnormals
+    among them, below 2^110 (larger ones may be left to the fp32 instruction)."""
+    rng = np.random.default_rng(M)
+    bits = rng.integers(0, 237 << 23, (K, M), dtype=np.uint32)
+    bits[::5] %= np.uint32(40 << 23)  # a fifth below 2^-87, a fortieth of that subnormal
+    bits |= rng.integers(0, 2, (K, M), dtype=np.uint32) << np.uint32(31)
+    l = bits.view(np.float32)
+    pick = rng.integers(0, K, N)
+    r = np.zeros((N, K), np.float32)
+    r[np.arange(N), pick] = 1.0
+    assert (np.abs(l[pick]) < 2.0 ** -126).any()
+    for form, y in _three_forms(dev, M, N, K, l, r, np.zeros((N, M), np.float32), 0.0):
+        assert np.array_equal(y, l[pick]), form
 
 
 @pytest.mark.parametrize("M,N,K", SPLIT_GEMM_SHAPES)
