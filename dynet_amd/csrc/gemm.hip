@@ -4,7 +4,7 @@
 //   * a right operand of 5 to 256 columns, small outputs with deep sums: the fragment-order products of lstm.hip;
 //   * at most four (nine to 32) columns, a depth of at most 32, at most 32 rows: the kernels below, which stream the large
 //     operand once;
-//   * operands of a few hundred KB: gemm_small.hip;
+//   * operands of a few hundred KB, and depths of at most 32 (64 with many tiles): gemm_small.hip;
 //   * everything else: 128 x 128 tiles (gemm_tile.hip) or smaller ones (gemm_direct.hip), chosen with a split of the depth
 //     by the cost model plan_mid.
 // Where the depth is split over blocks each writes its slice to a workspace and a second kernel adds the slices in

@@ -809,8 +809,9 @@ size_t gemm_wide_whole_rounds_columns(const dyhip_device* dev, bool a_kmajor, bo
   const size_t cus = dev->num_cus > 0 ? size_t(dev->num_cus) : 256;
   const size_t tiles_m = cdiv<size_t>(M, kWT), tiles = tiles_m * cdiv<size_t>(N, kWT);
   const size_t direct = tiles / cus * cus;
-  // From a depth of 768 on one sequence of k-tiles over all tiles is the faster one (4096 x 4480: K = 512 111 against
-  // 117 us, K = 1024 206 against 189 us, K = 2048 372 against 342 us).
+  // From a depth of 768 on one sequence of k-tiles over all tiles is as fast or faster (l*r, apart against one sequence:
+  // 4096 x 4480 K = 512 121 against 135 us, 768 176 and 176, 1024 222 against 219; 8192 x 2304 K = 512 130 against 137,
+  // 768 182 against 179, 1024 234 against 221, 2048 441 against 407).
   if (K >= 768 || direct == 0 || direct == tiles || direct % tiles_m != 0 || tiles - direct > cus / 4) return 0;
   const size_t cols = direct / tiles_m * kWT;
   return cols < N && gemm_wide_eligible(dev, a_kmajor, b_kmajor, M, cols, K, A, lda, B, ldb, C) ? cols : 0;
