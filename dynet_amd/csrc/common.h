@@ -73,6 +73,8 @@ struct dyhip_device {
   bool gemm_flags_used;      // a launch since the last host synchronisation may have counted a wait that gave up
   unsigned gemm_spin_limit;  // polls before a block's wait for another block's partial tile gives up
   int gemm_raise_flags;      // 0 only in tests of the give-up path: producers leave their flags down
+  unsigned sequence_ready;   // lstm_sequence.hip: kernels whose dynamic-LDS limit has been raised on this device
+  unsigned sequence_blocks;  // 0; else, in tests, the most blocks an LSTM sequence is launched with
   hipEvent_t ev_start, ev_stop;
   dyhip_device* parent;                // non-null for a forked queue: pools, scalars and allocator belong to the parent
   std::vector<hipEvent_t> sync_events; // ring of events recorded on this queue for dyhip_device_wait

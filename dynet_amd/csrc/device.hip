@@ -181,7 +181,7 @@ static int gemm_giveups_of_queue(dyhip_device* q, unsigned* gave_up) {
 }
 
 // Called by every entry point that has just synchronised dev's stream and hands results to the host: turns waits
-// that gave up inside a 256 x 256-tile GEMM (on this queue, or on a queue forked from it: a graph launched here may
+// that gave up inside a 256 x 256-tile GEMM or an LSTM sequence (on this queue, or on a queue forked from it: a graph launched here may
 // hold products recorded there) into an error.
 int dyhip::gemm_check_giveups(dyhip_device* dev) {
   unsigned total = 0, n = 0;
@@ -194,8 +194,8 @@ int dyhip::gemm_check_giveups(dyhip_device* dev) {
     total += n;
   }
   if (total != 0)
-    return fail(DYHIP_ERR_RUNTIME, "GEMM: %u blocks gave up waiting for a partial tile; the products since the last "
-                                   "synchronisation are incomplete", total);
+    return fail(DYHIP_ERR_RUNTIME, "GEMM or LSTM sequence: %u blocks gave up waiting for another block; the results since "
+                                   "the last synchronisation are incomplete", total);
   return DYHIP_OK;
 }
 
@@ -342,6 +342,8 @@ int dyhip_device_create(int ordinal, const size_t pool_mb[4], dyhip_device** out
   dev->gemm_ws = nullptr;
   dev->gemm_ws_bytes = 0;
   dev->wide_gemm_ready = 0;
+  dev->sequence_ready = 0;
+  dev->sequence_blocks = 0;
   dev->gemm_flags = nullptr;
   dev->gemm_flags_used = false;
   dev->ln_scratch = nullptr;
@@ -623,11 +625,11 @@ int dyhip_graph_launch(dyhip_device* dev, dyhip_graph* graph) {
   DYHIP_CHECK_DEV(dev);
   DYHIP_REQUIRE(graph != nullptr, "null graph handle");
   DYHIP_CHECK_HIP(hipGraphLaunch(graph->exec, dev->stream));
-  // a recorded large GEMM runs again with every replay, on this queue or on one forked from it: the next
-  // synchronisation looks at their give-up counters
-  if (dev->wide_gemm_ready != 0) dev->gemm_flags_used = true;
+  // a recorded large GEMM or LSTM sequence runs again with every replay, on this queue or on one forked from it: the
+  // next synchronisation looks at their give-up counters
+  if (dev->wide_gemm_ready != 0 || dev->sequence_ready != 0) dev->gemm_flags_used = true;
   for (dyhip_device* f : dev->forks)
-    if (f->wide_gemm_ready != 0) f->gemm_flags_used = true;
+    if (f->wide_gemm_ready != 0 || f->sequence_ready != 0) f->gemm_flags_used = true;
   return DYHIP_OK;
 }
 

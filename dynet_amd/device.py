@@ -448,6 +448,24 @@ class Device:
         _check(cdll.dyhip_lstm_cell_forward(self.handle, _u(H), _u(B), _p(xproj), _p(b), _vp(rec), _u(splits),
                                             _p(c_tm1), _i(logistic_mode), _p(gates), _p(c), _p(h)))
 
+    def lstm_sequence_workspace(self, H, B, T):
+        """Bytes of scratch that a layer's timesteps in one launch need; 0 where the sizes are not supported."""
+        n = _sz(0)
+        _check(cdll.dyhip_lstm_sequence_workspace(self.handle, _u(H), _u(B), _u(T), C.byref(n)))
+        return n.value
+
+    def lstm_sequence_forward(self, H, B, T, Wh, xproj, b, gates, c, h, ws, ws_bytes, mask_h=None,
+                              logistic_mode=lib.LOGISTIC_PACKET):
+        _check(cdll.dyhip_lstm_sequence_forward(self.handle, _u(H), _u(B), _u(T), _p(Wh), _p(mask_h), _p(xproj), _p(b),
+                                                _i(logistic_mode), _p(gates), _p(c), _p(h), _vp(ws), _sz(ws_bytes)))
+
+    def lstm_sequence_backward(self, H, B, T, Wh, gates, c, dh, dpre, ws, ws_bytes, mask_h=None):
+        _check(cdll.dyhip_lstm_sequence_backward(self.handle, _u(H), _u(B), _u(T), _p(Wh), _p(mask_h), _p(gates), _p(c),
+                                                 _p(dh), _p(dpre), _vp(ws), _sz(ws_bytes)))
+
+    def set_sequence_blocks(self, blocks):
+        _check(cdll.dyhip_device_set_sequence_blocks(self.handle, _u(blocks)))
+
     def lstm_step_supported(self, H, B):
         ok = C.c_int(0)
         _check(cdll.dyhip_lstm_step_supported(self.handle, _u(H), _u(B), C.byref(ok)))

@@ -19,7 +19,9 @@ What differs from DyNet's node-at-a-time execution (results agree to fp32 roundi
   * ``path="fused"`` (default) runs layer by layer: one GEMM forms Wx*x for all timesteps, a timestep is then
     the recurrent GEMM Wh*h plus one cell kernel (gates + c + h); backward mirrors it, and dx, dWx, dWh, db are
     GEMMs/reductions over all timesteps;
-  * a timestep of the fused path is one kernel forward (recurrent product + cell update) and one backward (Wh^T *
+  * all timesteps of a layer are one kernel each way where the sizes allow (``sequence``; not with overlap=True or an
+    explicit ``single_launch``);
+  * else a timestep of the fused path is one kernel forward (recurrent product + cell update) and one backward (Wh^T *
     dpre of the step above + cell backward), both reading their operands from packed copies in matrix-core
     fragment order that the previous timestep's kernel wrote (``single_launch``, where the sizes allow);
   * with ``overlap=True`` the fused path cuts the time axis into chunks and runs the layers as a pipeline on one
@@ -122,20 +124,29 @@ class LstmLM:
             self.gath_x = dev.empty((T, B, max(E, H)), pool=DE)
             self.gath_h = dev.empty((T, B, H), pool=DE)
         self.d_pre = [dev.empty((T, B, 4 * H), pool=DE) for _ in range(L)]  # overwritten, never accumulated into
+        # all timesteps of a layer as one launch each way where the sizes allow; the layers take turns with its scratch
+        # (a launch that takes about 20 us before its second timestep, then at H = 1024, B = 128 4.5 us a timestep less than a
+        # launch each; at H = 128, where that is 0.2 forward and 0.8 backward, from 16 timesteps on)
+        long_enough = T >= (16 if H == 128 else 5)
+        nseq = dev.lstm_sequence_workspace(H, B, T) if (path == "fused" and long_enough and not self.overlap
+                                                        and single_launch is None) else 0
+        self.sequence = nseq > 0
+        self.seq_ws, self.seq_bytes = dev.workspace(nseq)
         fb, bb = dev.lstm_cell_workspace(H, B)
         self.rec_f_bytes, self.rec_b_bytes = fb, bb
-        self.rec_f = [dev.workspace(fb)[0] for _ in range(L)]  # one per layer: layers run side by side
-        self.rec_b = [dev.workspace(bb)[0] for _ in range(L)]
+        self.rec_f = [dev.workspace(fb)[0] for _ in range(L)] if not self.sequence else []  # one per layer: layers run side by side
+        self.rec_b = [dev.workspace(bb)[0] for _ in range(L)] if not self.sequence else []
         # forward timesteps as one kernel each (recurrent product + cell update) where the size allows
         ok = path == "fused" and dev.lstm_step_supported(H, B)
         self.single_launch = ok if single_launch is None else (bool(single_launch) and ok)
-        self.Wh_packed = [dev.empty((4 * H * H,), pool=PS) for _ in range(L)] if self.single_launch else []
-        self.WhT_packed = [dev.empty((4 * H * H,), pool=PS) for _ in range(L)] if self.single_launch else []
+        packed = self.single_launch and not self.sequence
+        self.Wh_packed = [dev.empty((4 * H * H,), pool=PS) for _ in range(L)] if packed else []
+        self.WhT_packed = [dev.empty((4 * H * H,), pool=PS) for _ in range(L)] if packed else []
         # packed copies of h and of dpre for the next timestep's recurrent product, two per layer used in turn
-        nh = dev.lstm_packed_state_floats(H, B) if self.single_launch else 0
-        nd = dev.lstm_packed_state16_floats(4 * H, B) if self.single_launch else 0
-        self.h_packed = [[dev.empty((nh,), pool=FXS) for _ in range(2)] for _ in range(L)] if self.single_launch else []
-        self.dpre_packed = [[dev.empty((nd,), pool=DE) for _ in range(2)] for _ in range(L)] if self.single_launch else []
+        nh = dev.lstm_packed_state_floats(H, B) if packed else 0
+        nd = dev.lstm_packed_state16_floats(4 * H, B) if packed else 0
+        self.h_packed = [[dev.empty((nh,), pool=FXS) for _ in range(2)] for _ in range(L)] if packed else []
+        self.dpre_packed = [[dev.empty((nd,), pool=DE) for _ in range(2)] for _ in range(L)] if packed else []
         # queue l runs layer l; queue 0 is the device itself
         self.queues = [dev] + ([dev.fork() for _ in range(L - 1)] if self.overlap else [])
         self.plan, self.plan_ws, self.plan_ws_bytes = dev.lookup_plan_buffers(N, V)
@@ -244,7 +255,7 @@ class LstmLM:
 
     def _forward_layers_fused(self):
         d, E, H, L, B, T, N = self.dev, self.E, self.H, self.L, self.B, self.T, self.N
-        if self.single_launch:  # the weights moved in the last update
+        if self.single_launch and not self.sequence:  # the weights moved in the last update
             for l in range(L):
                 d.lstm_pack_recurrent(H, self.p[f"Wh{l}"], self.Wh_packed[l])
                 d.lstm_pack_recurrent_transposed16(H, self.p[f"Wh{l}"], self.WhT_packed[l])
@@ -254,8 +265,13 @@ class LstmLM:
                     self._mask_inputs(d, l)
                 x, d_in = self._x_of(l)
                 d.gemm_nn(4 * H, N, d_in, self.p[f"Wx{l}"], x, 0.0, self.gates[l])  # Wx*x of every timestep
-                self._cell_steps_forward(d, l, 0, T)
-                if self.use_dropout and self.single_launch and T > 1:  # for dWh: h (.) mask_h of every timestep
+                if self.sequence:
+                    d.lstm_sequence_forward(H, B, T, self.p[f"Wh{l}"], self.gates[l], self.p[f"b{l}"], self.gates[l],
+                                            self.c[l], self.h[l], self.seq_ws, self.seq_bytes,
+                                            mask_h=self.mask_h[l] if self.use_dropout else None)
+                else:
+                    self._cell_steps_forward(d, l, 0, T)
+                if self.use_dropout and (self.sequence or self.single_launch) and T > 1:  # for dWh: h (.) mask_h of every timestep
                     d.cmult_forward(B * H, T, 1, self.h[l], self.mask_h[l], self.hm[l])
             return
         # pipeline over time chunks: queue l runs layer l, one chunk behind queue l-1
@@ -369,7 +385,11 @@ class LstmLM:
         self._rec_b_n = [0] * L
         if not self.overlap:
             for l in reversed(range(L)):
-                self._cell_steps_backward(d, l, 0, T)
+                if self.sequence:
+                    d.lstm_sequence_backward(H, B, T, self.p[f"Wh{l}"], self.gates[l], self.c[l], self.d_h[l], self.d_pre[l],
+                                             self.seq_ws, self.seq_bytes, mask_h=self.mask_h[l] if self.use_dropout else None)
+                else:
+                    self._cell_steps_backward(d, l, 0, T)
                 d_in, dx = (H, self.d_h[l - 1]) if l > 0 else (E, self.d_emb)
                 d.gemm_tn(d_in, N, 4 * H, self.p[f"Wx{l}"], self.d_pre[l], 0.0, dx)
                 if self.use_dropout:  # the gradient reaches the layer's input through mask_x

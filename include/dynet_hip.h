@@ -67,6 +67,9 @@ int dyhip_device_sync(dyhip_device* dev);
  * spin_limit = 0 every consumer gives up at once while every kernel still runs to its end: the host-driven test of
  * the error path.  Applies to products issued afterwards on this queue.  No counterpart in the reference. */
 int dyhip_device_set_gemm_handoff(dyhip_device* dev, unsigned spin_limit, int raise_flags);
+/* For tests: the most blocks that an LSTM sequence (dyhip_lstm_sequence_forward / _backward) is launched with, as if the
+ * others had not found a place on the GPU yet; 0 (the default): one for each tile. */
+int dyhip_device_set_sequence_blocks(dyhip_device* dev, unsigned blocks);
 int dyhip_device_ordinal(const dyhip_device* dev, int* ordinal);
 int dyhip_device_stream(dyhip_device* dev, void** hip_stream);
 int dyhip_device_pool(dyhip_device* dev, int which, dyhip_pool** pool);
@@ -392,6 +395,20 @@ int dyhip_lstm_step_backward_packed(dyhip_device* dev, unsigned H, unsigned B, c
                                     const float* dpre_next_packed16, const float* gates, const float* c,
                                     const float* c_tm1, const float* dh, const float* dc, float* dpre, float* dc_tm1,
                                     float* dpre_packed16);
+/* All T timesteps of a layer in ONE launch (no counterpart in the reference: the loop of dynet/lstm.cc:1044-1080 over its
+ * three nodes), from the zero initial state.  xproj: Wx * x of every timestep, T x B columns of 4H (may be gates);
+ * mask_h: the recurrent dropout mask (H x B) or null; gates, c, h, dh, dpre: T x B columns.  The backward takes dh, the
+ * gradient that reaches every h_t from outside the recurrence, and writes dpre of every timestep.  Wh is read as it lies.
+ * dyhip_lstm_sequence_workspace: bytes that either call needs, on a 256-byte boundary; 0 where the sizes are not
+ * supported (H beyond 1024, more tiles of units x columns than CUs): the single timesteps cover those.  Calls on queues
+ * that overlap need a workspace each.  Same results as the timesteps up to fp32 summation order; a dpre of 2^111 or more
+ * counts as infinite in the recurrent product. */
+int dyhip_lstm_sequence_workspace(dyhip_device* dev, unsigned H, unsigned B, unsigned T, size_t* bytes);
+int dyhip_lstm_sequence_forward(dyhip_device* dev, unsigned H, unsigned B, unsigned T, const float* Wh, const float* mask_h,
+                                const float* xproj, const float* b, int logistic_mode, float* gates, float* c, float* h,
+                                void* ws, size_t ws_bytes);
+int dyhip_lstm_sequence_backward(dyhip_device* dev, unsigned H, unsigned B, unsigned T, const float* Wh, const float* mask_h,
+                                 const float* gates, const float* c, const float* dh, float* dpre, void* ws, size_t ws_bytes);
 /* The two single-launch timesteps with the recurrent dropout mask of CompactVanillaLSTMBuilder (dynet/lstm.cc:964-982:
  * one mask per layer and sequence, H x B, already scaled by 1 / retention; the node applies it as h_tm1 (.) mask_h,
  * dynet/nodes-lstm.cc:178-198, and hands the gradient back through it, :448-470).  Forward: h is written plain,
