@@ -120,8 +120,8 @@ __global__ __launch_bounds__(256, 2) void gemm_tile_kernel(TileArgs g) {
 #define DYHIP_TILE_SPLIT(j, stage)                                                                       \
   {                                                                                                      \
     uint2 h_, m_, l_;                                                                                    \
-    split3_pair(kmajor ? raw[j][0] : raw[0][j], kmajor ? raw[j][1] : raw[1][j], h_.x, m_.x, l_.x);       \
-    split3_pair(kmajor ? raw[j][2] : raw[2][j], kmajor ? raw[j][3] : raw[3][j], h_.y, m_.y, l_.y);       \
+    split3_pair_beside_products(kmajor ? raw[j][0] : raw[0][j], kmajor ? raw[j][1] : raw[1][j], h_.x, m_.x, l_.x);       \
+    split3_pair_beside_products(kmajor ? raw[j][2] : raw[2][j], kmajor ? raw[j][3] : raw[3][j], h_.y, m_.y, l_.y);       \
     char* d_ = lds + ow[j] + (stage) * kTileStage;                                                            \
     *reinterpret_cast<uint2*>(d_) = h_;                                                                  \
     *reinterpret_cast<uint2*>(d_ + kTilePlane) = m_;                                                     \

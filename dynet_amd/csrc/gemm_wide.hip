@@ -9,11 +9,11 @@
 // 4480 x 1024) at a shader clock that falls to 1.9 GHz; a third stage in LDS, which takes the two wavefronts of a SIMD out
 // of step, changed nothing.  Measured, random operands, against v_mfma_f32_32x32x2_f32 in the same tiling (94 % busy,
 // 157 TFLOP/s at most):
-//   10000 x 4480 x 1024 l*r     708 -> 486 us (130 -> 189 TFLOP/s)   1024 x 4480 x 10000 l^T*r   712 -> 488 us
-//   10000 x 1024 x 4480 l*r^T   688 -> 457 us (133 -> 201)            4096 x 1024 x 4480 l*r^T    285 -> 194 us
+//   10000 x 4480 x 1024 l*r     708 -> 473 us (130 -> 194 TFLOP/s)   1024 x 4480 x 10000 l^T*r   712 -> 478 us
+//   10000 x 1024 x 4480 l*r^T   688 -> 448 us (133 -> 205)            4096 x 1024 x 4480 l*r^T    285 -> 192 us
 //
 // Step of 16 k.  Operands are fetched as fp32 into registers (four 128-bit loads a thread), split there and written to
-// LDS as three bf16 planes: splitting in the block re-does the work for every tile that shares an operand, but 72 vector
+// LDS as three bf16 planes: splitting in the block re-does the work for every tile that shares an operand, but 104 vector
 // instructions a wave and step hide under 48 MFMAs, where a pass of its own over the operands would move 10 bytes per
 // element (450 MB for a 10000 x 4480 operand).  LDS holds two stages of 48 KiB; fragments are read as 128 bits a lane.
 //
@@ -124,8 +124,8 @@ __device__ __forceinline__ void split_row(bool kmajor, const float4 (&v)[4], int
 #pragma unroll
   for (int k = 0; k < 4; ++k) x[k] = kmajor ? component(v[j], k) : component(v[k], j);
   uint2 h, m, l;
-  split3_pair(x[0], x[1], h.x, m.x, l.x);
-  split3_pair(x[2], x[3], h.y, m.y, l.y);
+  split3_pair_beside_products(x[0], x[1], h.x, m.x, l.x);
+  split3_pair_beside_products(x[2], x[3], h.y, m.y, l.y);
   *reinterpret_cast<uint2*>(dst + 1024 * j) = h;
   *reinterpret_cast<uint2*>(dst + 1024 * j + kPlaneBytes) = m;
   *reinterpret_cast<uint2*>(dst + 1024 * j + 2 * kPlaneBytes) = l;
