@@ -1372,6 +1372,54 @@ __global__ __launch_bounds__(256) void gemm_tn_thin_kernel(unsigned M, unsigned 
   }
 }
 
+// One column of B for each item of a strided batch (the scores of an attention over a batch and their gradient): a
+// wavefront owns COLS columns of A, their whole depth, and B's entries in registers for all of them; up to 4 x COLS
+// 128-bit loads of A in flight a lane and nothing to meet for but the wavefront's own sums.  The kernel above multiplies
+// four columns of B for one and meets in LDS.
+template <int COLS>
+__global__ __launch_bounds__(256) void gemm_tn_vector_kernel(unsigned M, unsigned K4, const float* __restrict__ A, size_t lda,
+                                                             const float* __restrict__ B, float beta, float* __restrict__ C,
+                                                             size_t stride_a, size_t stride_b, size_t stride_c) {
+  const unsigned lane = threadIdx.x & 63, i0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * COLS;
+  if (i0 >= M) return;  // wave-uniform, no barrier below
+  A += size_t(blockIdx.y) * stride_a;
+  const float4* b4 = reinterpret_cast<const float4*>(B + size_t(blockIdx.y) * stride_b);
+  C += size_t(blockIdx.y) * stride_c;
+  const float4* a4[COLS];
+  float acc[COLS][4];  // four short sums, added in pairs: no longer a chain than the block form
+#pragma unroll
+  for (int c = 0; c < COLS; ++c) {
+    a4[c] = reinterpret_cast<const float4*>(A + size_t(min(i0 + c, M - 1)) * lda);  // columns past the end: not stored
+#pragma unroll
+    for (int u = 0; u < 4; ++u) acc[c][u] = 0.f;
+  }
+  for (unsigned k0 = 0; k0 < K4; k0 += 256) {
+    float4 a[COLS][4], b[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const unsigned k = k0 + 64 * u + lane, kc = min(k, K4 - 1);
+      b[u] = b4[kc];
+      if (k >= K4) b[u] = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+      for (int c = 0; c < COLS; ++c) a[c][u] = a4[c][kc];
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int c = 0; c < COLS; ++c) {
+        acc[c][u] = fmaf(a[c][u].x, b[u].x, acc[c][u]);
+        acc[c][u] = fmaf(a[c][u].y, b[u].y, acc[c][u]);
+        acc[c][u] = fmaf(a[c][u].z, b[u].z, acc[c][u]);
+        acc[c][u] = fmaf(a[c][u].w, b[u].w, acc[c][u]);
+      }
+  }
+#pragma unroll
+  for (int c = 0; c < COLS; ++c) {
+    const float t = wave_sum((acc[c][0] + acc[c][1]) + (acc[c][2] + acc[c][3]));
+    if (lane == 0 && i0 + c < M) C[i0 + c] = beta != 0.f ? beta * C[i0 + c] + t : t;
+  }
+}
+
 // ---- C[M x N] = beta * C + A^T B for 5..256 columns of B (in tiles of 32) on the matrix cores, the operands as they lie --
 // A's columns (the depth contiguous) are fetched by coalesced 128-bit loads, 32 depth indices of 32 columns a
 // wavefront at a time (128-byte runs), and turned into matrix-core fragments through a wavefront's own LDS tile:
@@ -1528,6 +1576,15 @@ static int thin_tn_run(dyhip_device* dev, size_t M, size_t N, size_t K, const fl
                        size_t ldb, float beta, float* C, const GemmBatch* batch = nullptr) {
   const unsigned items = batch != nullptr && batch->count > 1 ? batch->count : 1;
   const size_t sa = items > 1 ? batch->stride_a : 0, sb = items > 1 ? batch->stride_b : 0, sc = items > 1 ? batch->stride_c : 0;
+  // one column, enough of them for a thousand wavefronts (35 x 1 x 1024 in 128 items 4.8 -> 3.2 us, 35 x 1 x 256 4.1 -> 3.2,
+  // 12 x 1 x 1024 in 64 items 3.0 either way; one column of A a wavefront 3.3, three 3.2, streaming loads 3.2-3.8)
+  if (N == 1 && items > 1 && M * items >= 2048) {
+    const dim3 vgrid(static_cast<unsigned>(cdiv<size_t>(M, 8)), items);
+    hipLaunchKernelGGL((gemm_tn_vector_kernel<2>), vgrid, dim3(256), 0, dev->stream, static_cast<unsigned>(M),
+                       static_cast<unsigned>(K / 4), A, lda, B, beta, C, sa, sb, sc);
+    DYHIP_CHECK_LAUNCH();
+    return DYHIP_OK;
+  }
   const int cols = M * items > 4096 ? 4 : M * items > 512 ? 2 : 1;
   const dim3 grid(static_cast<unsigned>(cdiv<size_t>(M, cols)), items), block(256);
 #define DYHIP_THIN_TN_C(NP, CC)                                                                                 \
