@@ -86,22 +86,40 @@ __global__ __launch_bounds__(256) void sgd_scaled_kernel(size_t n4, size_t n, fl
 
 // The entries of a lookup plan (lookup.hip): one 16-byte record per grouped position, .x = id (ids >= vocab replaced
 // by vocab), .z = entries of its run before it (0 at the head of a run).
-// One block per grouped position; only the first entry of each run of equal ids acts.
-__global__ __launch_bounds__(128) void sgd_rows_kernel(unsigned n, const uint4* __restrict__ entries,
-                                                       unsigned dim, unsigned vocab, float* __restrict__ values,
-                                                       float* __restrict__ grads, float lr, float wd,
-                                                       const float* __restrict__ gscale) {
-  const unsigned k = blockIdx.x;
+// A wavefront per grouped position, four to a block; only the first entry of each run of equal ids acts.  V is float4 where
+// rows are whole 16-byte groups: a lane then has four loads in flight, two of the row and two of its gradient.
+// Memory work: 16 384 ids of which 4109 differ, rows of 512 floats, 34 MB: 11.2 -> 9.2 us (a block of two wavefronts a
+// position, one float a lane and step, before).
+__device__ __forceinline__ float stepped(float p, float g, float s) { return p - g * s; }
+__device__ __forceinline__ float4 stepped(const float4& p, const float4& g, float s) {
+  return make_float4(p.x - g.x * s, p.y - g.y * s, p.z - g.z * s, p.w - g.w * s);
+}
+
+template <class V>
+__global__ __launch_bounds__(256) void sgd_rows_kernel(unsigned n, const uint4* __restrict__ entries, unsigned dimv,
+                                                       unsigned vocab, V* __restrict__ values, V* __restrict__ grads,
+                                                       float lr, float wd, const float* __restrict__ gscale) {
+  const unsigned k = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + threadIdx.x / 64), lane = threadIdx.x % 64;
+  if (k >= n) return;
   const uint4 e = entries[k];
   const unsigned id = e.x;
   if (id >= vocab || e.z != 0) return;
   const float gs = *gscale;
   const float s = lr * gs / wd;
-  float* pv = values + size_t(id) * dim;
-  float* pg = grads + size_t(id) * dim;
-  for (unsigned j = threadIdx.x; j < dim; j += 128) {
-    if (gs != 0.f) pv[j] -= pg[j] * s;
-    pg[j] = 0.f;
+  V* pv = values + size_t(id) * dimv;
+  V* pg = grads + size_t(id) * dimv;
+  for (unsigned j0 = 0; j0 < dimv; j0 += 128) {
+    const unsigned j = j0 + lane, last = dimv - 1;
+    const bool in0 = j < dimv, in1 = j + 64 < dimv;
+    const V p0 = pv[min(j, last)], g0 = pg[min(j, last)], p1 = pv[min(j + 64, last)], g1 = pg[min(j + 64, last)];
+    if (in0) {
+      if (gs != 0.f) pv[j] = stepped(p0, g0, s);
+      pg[j] = V{};
+    }
+    if (in1) {
+      if (gs != 0.f) pv[j + 64] = stepped(p1, g1, s);
+      pg[j + 64] = V{};
+    }
   }
 }
 
@@ -183,8 +201,14 @@ int dyhip_sgd_update_rows(dyhip_device* dev, unsigned n_ids, const void* plan, s
   if (n_ids == 0 || dim == 0) return DYHIP_OK;
   DYHIP_REQUIRE(plan && values && grads && gscale, "null pointer");
   DYHIP_REQUIRE(wd != 0.f && dim < (size_t(1) << 31), "bad weight decay scale or dimension");
-  hipLaunchKernelGGL(sgd_rows_kernel, dim3(n_ids), dim3(128), 0, dev->stream, n_ids,
-                     static_cast<const uint4*>(plan), (unsigned)dim, vocab, values, grads, lr, wd, gscale);
+  const dim3 grid(cdiv<unsigned>(n_ids, 4)), block(256);
+  const uint4* entries = static_cast<const uint4*>(plan);
+  if (dim % 4 == 0 && aligned16(values) && aligned16(grads))
+    hipLaunchKernelGGL(sgd_rows_kernel<float4>, grid, block, 0, dev->stream, n_ids, entries, unsigned(dim / 4), vocab,
+                       reinterpret_cast<float4*>(values), reinterpret_cast<float4*>(grads), lr, wd, gscale);
+  else
+    hipLaunchKernelGGL(sgd_rows_kernel<float>, grid, block, 0, dev->stream, n_ids, entries, unsigned(dim), vocab, values, grads,
+                       lr, wd, gscale);
   DYHIP_CHECK_LAUNCH();
   return DYHIP_OK;
 }
