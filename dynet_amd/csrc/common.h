@@ -87,6 +87,19 @@ struct dyhip_device {
 };
 
 namespace dyhip {
+// Host integers that travel in a kernel's argument block, which is copied when the kernel is launched: the caller's memory is
+// free when the call returns, without a staging copy and a wait for it (a call with 1 to 512 indices 20 -> 6.5 us).
+template <unsigned N>
+struct HostWords {
+  unsigned v[N];
+};
+constexpr unsigned kFewHostWords = 64, kHostWords = 960;  // a block holds 4 KiB; most calls name a handful
+// misc.hip: dst[0..n) = src[0..n) that way, in pieces of kHostWords.  Refused, as the wait was, while the queue is captured: a
+// graph would repeat the values of the capture.
+int put_host_words(dyhip_device* dev, unsigned* dst, const unsigned* src, unsigned n);
+int refuse_while_capturing(dyhip_device* dev);
+constexpr unsigned kPutHostWordsMost = 2 * kHostWords;  // beyond, the copy and the wait take no longer (2048: 20 us either way)
+
 // reduce.hip: looks up, on the current device, the address of the static scratch array (once per device handle)
 int ln_static_scratch_setup(dyhip_device* dev);
 // device.hip: after a host synchronisation of dev's stream, reports waits that gave up inside a large GEMM

@@ -100,6 +100,25 @@ __global__ __launch_bounds__(kLkThreads) void lookup_gather_kernel(unsigned n_id
   }
 }
 
+// The same for ids that come with the launch (validated on the host), a few hundred at most: decoding, a short sentence.
+// It writes them to ids_dev as well, which the backward pass reads.
+template <unsigned N, class V, bool SCALE>
+__global__ __launch_bounds__(kLkThreads) void lookup_gather_host_kernel(HostWords<N> ids, unsigned n_ids, unsigned dimv, unsigned tpr,
+                                                                        unsigned* __restrict__ ids_dev,
+                                                                        const V* __restrict__ table, float mult,
+                                                                        V* __restrict__ fx) {
+  const unsigned groups = kLkThreads / tpr;
+  const unsigned grp = threadIdx.x / tpr, t = threadIdx.x - grp * tpr;
+  const unsigned row = blockIdx.x * groups + grp;
+  if (grp >= groups || row >= n_ids) return;
+  const unsigned id = ids.v[row];
+  if (t == 0) ids_dev[row] = id;
+  for (unsigned c = t; c < dimv; c += tpr) {
+    const V v = table[size_t(id) * dimv + c];
+    fx[size_t(row) * dimv + c] = SCALE ? vscale(v, mult) : v;
+  }
+}
+
 // ---- the plan: ids grouped by value ------------------------------------------------
 // plan = [entries | arrivals | status], each part padded to 256 bytes.  Entry k of the grouped order is one
 // 16-byte record, so that a consumer's first (and only) dependent load per entry is a single 128-bit access:
@@ -1189,6 +1208,22 @@ static int reduce_planned(dyhip_device* dev, unsigned n, const void* plan, size_
   return DYHIP_OK;
 }
 
+template <unsigned N>
+static void gather_host(dyhip_device* dev, unsigned n, const unsigned* ids_host, unsigned* ids_dev, bool vec, unsigned dimv,
+                        unsigned tpr, const float* table, float mult, float* fx) {
+  HostWords<N> ids;
+  std::copy(ids_host, ids_host + n, ids.v);
+  const dim3 grid(cdiv<unsigned>(n, kLkThreads / tpr)), block(kLkThreads);
+#define DYHIP_GATHER_HOST(V, SCALE)                                                                                       \
+  hipLaunchKernelGGL((lookup_gather_host_kernel<N, V, SCALE>), grid, block, 0, dev->stream, ids, n, dimv, tpr, ids_dev,    \
+                     reinterpret_cast<const V*>(table), mult, reinterpret_cast<V*>(fx))
+  if (vec && mult == 1.0f) DYHIP_GATHER_HOST(float4, false);
+  else if (vec) DYHIP_GATHER_HOST(float4, true);
+  else if (mult == 1.0f) DYHIP_GATHER_HOST(float, false);
+  else DYHIP_GATHER_HOST(float, true);
+#undef DYHIP_GATHER_HOST
+}
+
 }  // namespace dyhip
 
 using namespace dyhip;
@@ -1205,12 +1240,23 @@ int dyhip_lookup_forward(dyhip_device* dev, unsigned n_ids, const unsigned* ids_
     for (unsigned b = 0; b < n_ids; ++b)
       DYHIP_REQUIRE(ids_host[b] < vocab, "Out-of-bounds attempt to access index %u for LookupParameter of size %u",
                     ids_host[b], vocab);
-    DYHIP_CHECK_HIP(hipMemcpyAsync(ids_dev, ids_host, sizeof(unsigned) * n_ids, hipMemcpyHostToDevice, dev->stream));
-    DYHIP_CHECK_HIP(hipStreamSynchronize(dev->stream));  // ids_host may be released by the caller on return
   }
   const bool vec = dim % 4 == 0 && aligned16(table) && aligned16(fx);
   const unsigned dimv = static_cast<unsigned>(vec ? dim / 4 : dim);
   const unsigned tpr = threads_per_row(dimv);
+  if (ids_host != nullptr && n_ids <= kHostWords) {
+    DYHIP_CHECK_STATUS(refuse_while_capturing(dev));
+    if (n_ids <= kFewHostWords) gather_host<kFewHostWords>(dev, n_ids, ids_host, ids_dev, vec, dimv, tpr, table, mult, fx);
+    else gather_host<kHostWords>(dev, n_ids, ids_host, ids_dev, vec, dimv, tpr, table, mult, fx);
+    DYHIP_CHECK_LAUNCH();
+    return DYHIP_OK;
+  }
+  if (ids_host != nullptr && n_ids <= kPutHostWordsMost) {
+    DYHIP_CHECK_STATUS(put_host_words(dev, ids_dev, ids_host, n_ids));
+  } else if (ids_host != nullptr) {
+    DYHIP_CHECK_HIP(hipMemcpyAsync(ids_dev, ids_host, sizeof(unsigned) * n_ids, hipMemcpyHostToDevice, dev->stream));
+    DYHIP_CHECK_HIP(hipStreamSynchronize(dev->stream));  // ids_host may be released by the caller on return
+  }
   const unsigned rows_per_block = (kLkThreads / tpr) * kGatherRowsUnroll;
   const dim3 grid(cdiv<unsigned>(n_ids, rows_per_block)), block(kLkThreads);
   // the table is read through the caches (hot rows repeat); the output is streamed when large

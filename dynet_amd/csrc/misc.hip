@@ -7,6 +7,8 @@
 // sequence (id % num_seqs), so neighbouring lanes touch different sequences; here
 // blockIdx.y is the sequence and lanes walk consecutive floats of it, with
 // 128-bit accesses when both sides are 16-byte aligned.
+#include <algorithm>
+
 #include "common.h"
 
 namespace dyhip {
@@ -114,6 +116,38 @@ __global__ __launch_bounds__(kThreads) void gather_segments_kernel(GatherArgs a,
          i < e; i += kThreads)
       pt[i] = ps[i];
   }
+}
+
+template <unsigned N>
+__global__ __launch_bounds__(kThreads) void put_words_kernel(HostWords<N> a, unsigned n, unsigned* __restrict__ dst) {
+  const unsigned i = blockIdx.x * kThreads + threadIdx.x;
+  if (i < n) dst[i] = a.v[i];
+}
+
+int refuse_while_capturing(dyhip_device* dev) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  DYHIP_CHECK_HIP(hipStreamIsCapturing(dev->stream, &status));
+  if (status != hipStreamCaptureStatusNone)
+    return fail(DYHIP_ERR_RUNTIME, "host indices cannot be recorded into a graph: stage them on the device");
+  return DYHIP_OK;
+}
+
+template <unsigned N>
+static void put_words(dyhip_device* dev, unsigned* dst, const unsigned* src, unsigned n) {
+  HostWords<N> a;
+  std::copy(src, src + n, a.v);
+  hipLaunchKernelGGL(put_words_kernel<N>, dim3(cdiv<unsigned>(n, kThreads)), dim3(kThreads), 0, dev->stream, a, n, dst);
+}
+
+int put_host_words(dyhip_device* dev, unsigned* dst, const unsigned* src, unsigned n) {
+  DYHIP_CHECK_STATUS(refuse_while_capturing(dev));
+  for (unsigned first = 0; first < n; first += kHostWords) {
+    const unsigned count = n - first < kHostWords ? n - first : kHostWords;
+    if (count <= kFewHostWords) put_words<kFewHostWords>(dev, dst + first, src + first, count);
+    else put_words<kHostWords>(dev, dst + first, src + first, count);
+  }
+  DYHIP_CHECK_LAUNCH();
+  return DYHIP_OK;
 }
 
 // stage 1: per-block partial of sum g^2 ; stage 2: one block adds the partials in order

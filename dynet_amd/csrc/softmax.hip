@@ -1242,9 +1242,12 @@ int dyhip_pnls_forward(dyhip_device* dev, size_t rows, unsigned bd, const float*
   float* z = static_cast<float*>(aux);
   float* m = z + bd;
   unsigned* ids_dev = reinterpret_cast<unsigned*>(m + bd);
-  // pageable source: the copy has been staged by the time the call returns
-  DYHIP_CHECK_HIP(hipMemcpyAsync(ids_dev, ids.data(), sizeof(unsigned) * bd, hipMemcpyHostToDevice, dev->stream));
-  DYHIP_CHECK_HIP(hipStreamSynchronize(dev->stream));
+  if (bd <= kPutHostWordsMost) {
+    DYHIP_CHECK_STATUS(put_host_words(dev, ids_dev, ids.data(), bd));
+  } else {  // pageable source, read until the copy is done
+    DYHIP_CHECK_HIP(hipMemcpyAsync(ids_dev, ids.data(), sizeof(unsigned) * bd, hipMemcpyHostToDevice, dev->stream));
+    DYHIP_CHECK_HIP(hipStreamSynchronize(dev->stream));
+  }
   return launch_lse(dev, rows, bd, x, m, z, ids_dev, fx);
 }
 
