@@ -829,16 +829,24 @@ struct NnOperand {
 };
 enum { kNnGates = 0, kNnBias = 1, kNnAxpby = 2 };
 
+// A block's row tile.  Blocks go to the XCDs round robin.  Where M is no multiple of 32 two row tiles share a 128-byte line
+// of every k, and with tiles dealt round two L2s fetch it: each XCD takes `each` consecutive row tiles instead (a tile past
+// the last one is computed on the last row and dropped).  us in a graph, dealt round and consecutive: 10 000 x 64 x 1024
+// 28.5 and 26.0, 50 000 x 32 x 1024 55.3 and 51.4, 2600 x 64 x 1300 14.4 and 11.5, 9000 x 32 x 650 13.3 and 12.4, 10 000 x
+// 32 x 1024 15.0 and 14.8.  M a multiple of 32: 16 384 x 32 x 1024 15.6 and 16.4, 12 000 x 32 x 1024 14.4 and 14.9.
+__device__ __forceinline__ unsigned nn_row_tile(unsigned each) {
+  return each == 0 ? blockIdx.x : blockIdx.x % 8 * each + blockIdx.x / 8;
+}
+
 // TILES = 1: a block owns 32 rows (twice the blocks and half the matrix-core steps a wavefront: the smallest
 // baseline cell, 16 blocks of 64 rows, 8.0 us; 5.6 us with 32 of 32)
 template <int TILES, int EPI, int B_BYTES>
-__global__ __launch_bounds__(256) void skinny_nn_kernel(unsigned M, unsigned H, unsigned B, NnOperand op0, NnOperand op1,
+__global__ __launch_bounds__(256) void skinny_nn_kernel(unsigned each, unsigned M, unsigned H, unsigned B, NnOperand op0, NnOperand op1,
                                                         const float* __restrict__ bias, float beta, int mode,
                                                         float* __restrict__ fx) {
   constexpr unsigned ROWS = 32 * TILES;
   __shared__ float red[4 * ROWS * kStepPitchR];
-  const unsigned RP = (M + ROWS - 1) / ROWS;  // rows past the end are computed on the last row and dropped
-  const unsigned rp = blockIdx.x % RP, ct = blockIdx.x / RP;
+  const unsigned rp = nn_row_tile(each), ct = blockIdx.y;  // rows past the end are computed on the last row and dropped
   const unsigned wave = threadIdx.x / 64, lane = threadIdx.x % 64;
   const unsigned l32 = lane % 32, lhi = lane / 32;
   stepx16 acc0 = {0}, acc1 = {0};
@@ -953,15 +961,14 @@ typedef float stepx4u __attribute__((ext_vector_type(4), aligned(4)));
 constexpr unsigned kNnPitch = 36;  // 32 k and four floats of padding: fragment reads of 16 columns cover all banks
 
 template <int TILES, int WAVES, int EPI, bool MASKED>
-__global__ __launch_bounds__(64 * WAVES) void skinny_nn_deep_kernel(unsigned M, unsigned H, unsigned B, NnOperand op0,
+__global__ __launch_bounds__(64 * WAVES) void skinny_nn_deep_kernel(unsigned each, unsigned M, unsigned H, unsigned B, NnOperand op0,
                                                                     NnOperand op1, const float* __restrict__ bias,
                                                                     float beta, int mode, float* __restrict__ fx,
                                                                     float* __restrict__ partial) {
   constexpr unsigned ROWS = 32 * TILES;
   constexpr unsigned LDS = WAVES * 32 * (kNnPitch > TILES * kStepPitchR ? kNnPitch : TILES * kStepPitchR);
   __shared__ __attribute__((aligned(16))) float red[LDS];
-  const unsigned RP = (M + ROWS - 1) / ROWS;  // rows past the end are computed on the last row and dropped
-  const unsigned rp = blockIdx.x % RP, ct = blockIdx.x / RP;
+  const unsigned rp = nn_row_tile(each), ct = blockIdx.y;  // rows past the end are computed on the last row and dropped
   const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64;
   const unsigned l32 = lane % 32, lhi = lane / 32;
   const float bias_row = EPI == kNnAxpby ? 0.f : bias[min(rp * ROWS + threadIdx.x % ROWS, M - 1)];
@@ -975,7 +982,7 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_nn_deep_kernel(unsigned M, 
 #pragma unroll
   for (unsigned i = 0; i < 4; ++i) vcol[i] = min(ct * 32 + 8 * i + lane / 8, B - 1);  // past the batch: dropped
   const unsigned C0 = (op0.K + 31) / 32, C = C0 + (op1.K + 31) / 32;
-  const unsigned part = blockIdx.y * WAVES + wave, parts = gridDim.y * WAVES;
+  const unsigned part = blockIdx.z * WAVES + wave, parts = gridDim.z * WAVES;
   const unsigned lo = C * part / parts, hi = C * (part + 1) / parts;
   float* const mine = red + wave * 32 * kNnPitch;
 
@@ -1073,7 +1080,7 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_nn_deep_kernel(unsigned M, 
 #pragma unroll
     for (int w = 1; w < WAVES; ++w) t += red[(w * ROWS + orow) * kStepPitchR + col];
     if (partial != nullptr) {
-      partial[(size_t(blockIdx.y) * B + ecol) * M + erow] = t;
+      partial[(size_t(blockIdx.z) * B + ecol) * M + erow] = t;
       continue;
     }
     float* out = fx + size_t(ecol) * M + erow;
@@ -1132,22 +1139,26 @@ int skinny_nn_gemm(dyhip_device* dev, size_t M, size_t N, int nseg, const GemmSe
   const NnOperand op0{segs[0].A, segs[0].B, unsigned(segs[0].K), segs[0].lda, segs[0].ldb, m0.p, m0.ld};
   const NnOperand op1 = nseg > 1 ? NnOperand{segs[1].A, segs[1].B, unsigned(segs[1].K), segs[1].lda, segs[1].ldb, m1.p, m1.ld}
                                  : NnOperand{segs[0].A, segs[0].B, 0u, segs[0].lda, segs[0].ldb, m0.p, m0.ld};
-  const dim3 grid(cdiv<unsigned>(unsigned(M), 32 * tiles) * ct), block(256);
+  const unsigned rt = cdiv<unsigned>(unsigned(M), 32 * tiles), blocks = rt * ct;
+  // consecutive row tiles of an XCD, 0: dealt round (also where the padding to 8 XCDs would cost a round of the CUs)
+  unsigned each = M % 32 == 0 ? 0 : (rt + 7) / 8;
+  if (cdiv(8 * each * ct, cus) > cdiv(blocks, cus)) each = 0;
+  const dim3 grid(each == 0 ? rt : 8 * each, ct), block(256);
   const float beta = kind == kNnAxpby ? epi.beta : 0.f;
   // Few blocks: the depth over several of them, whose slices a second launch adds up.  The host pays for that launch too, so
   // only where it is worth much, or where the masks have saved two.
   unsigned splits = 0;  // 0: not that kernel
-  if (Kt >= kNnDeep && segs[0].K >= 32 && segs[nseg - 1].K >= 32 && grid.x <= cus) {
+  if (Kt >= kNnDeep && segs[0].K >= 32 && segs[nseg - 1].K >= 32 && blocks <= cus) {
     splits = 1;
     const size_t least = masks != nullptr ? 384 : 1024;
-    while (grid.x * (splits + 1) <= cus && Kt / (splits + 1) >= least) ++splits;
+    while (blocks * (splits + 1) <= cus && Kt / (splits + 1) >= least) ++splits;
     if (dev->gemm_ws == nullptr || dev->gemm_ws_bytes < sizeof(float) * M * N * splits) splits = 1;
     if (splits == 1 && masks == nullptr) splits = 0;
   }
   if (splits > 0) {
     float* const partial = splits > 1 ? static_cast<float*>(dev->gemm_ws) : nullptr;
 #define DYHIP_NN_DEEP(T, E, MK)                                                                                          \
-  hipLaunchKernelGGL((skinny_nn_deep_kernel<T, 8, E, MK>), dim3(grid.x, splits), dim3(512), 0, dev->stream, unsigned(M), epi.H, \
+  hipLaunchKernelGGL((skinny_nn_deep_kernel<T, 8, E, MK>), dim3(grid.x, ct, splits), dim3(512), 0, dev->stream, each, unsigned(M), epi.H, \
                      unsigned(N), op0, op1, epi.bias, beta, epi.logistic_mode, C, partial)
 #define DYHIP_NN_DEEP_T(T)                                             \
   do {                                                                 \
@@ -1166,7 +1177,7 @@ int skinny_nn_gemm(dyhip_device* dev, size_t M, size_t N, int nseg, const GemmSe
   }
   if (masks != nullptr) return DYHIP_OK;
 #define DYHIP_SKINNY_NN_B(T, E, BB)                                                                                 \
-  hipLaunchKernelGGL((skinny_nn_kernel<T, E, BB>), grid, block, 0, dev->stream, unsigned(M), epi.H, unsigned(N), op0, op1, \
+  hipLaunchKernelGGL((skinny_nn_kernel<T, E, BB>), grid, block, 0, dev->stream, each, unsigned(M), epi.H, unsigned(N), op0, op1, \
                      epi.bias, beta, epi.logistic_mode, C)
 #define DYHIP_SKINNY_NN(T, E)        \
   do {                               \
