@@ -41,6 +41,10 @@ struct MemAllocator {
 
 }  // namespace dyhip
 
+namespace dyhip {
+struct Mailbox;  // device.hip
+}
+
 // One growable bump-allocated region set: a list of blocks, allocation only
 // from the newest block, consolidation on free().
 struct dyhip_pool {
@@ -83,6 +87,7 @@ struct dyhip_device {
   uint64_t* rng_state;                 // device: {Philox key, next counter}; one per queue, see random.hip
   uint32_t rng_stream;                 // third counter word: 0 for the device, 1.. for its forked queues
   uint32_t forks_made;                 // forked queues created so far (numbers their random streams)
+  dyhip::Mailbox* mailbox;             // small results on their way to the host; one per queue
   void* ln_scratch;                    // this GPU's copy of the static scratch array of dyhip_layer_norm_backward_static
 };
 
@@ -102,8 +107,8 @@ constexpr unsigned kPutHostWordsMost = 2 * kHostWords;  // beyond, the copy and 
 
 // reduce.hip: looks up, on the current device, the address of the static scratch array (once per device handle)
 int ln_static_scratch_setup(dyhip_device* dev);
-// device.hip: after a host synchronisation of dev's stream, reports waits that gave up inside a large GEMM
-int gemm_check_giveups(dyhip_device* dev);
+// device.hip: waits for dev's stream and reports waits that gave up inside a large GEMM or an LSTM sequence
+int sync_and_check_giveups(dyhip_device* dev);
 }  // namespace dyhip
 
 struct dyhip_graph {

@@ -10,6 +10,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <mutex>
 
 #include "common.h"
 
@@ -167,30 +168,110 @@ static int gemm_flags_setup(dyhip_device* dev) {
   return gemm_flags_clear(dev);
 }
 
-// One queue's give-up counter; the queue's stream has been synchronised.
-static int gemm_giveups_of_queue(dyhip_device* q, unsigned* gave_up) {
+// ---- small results on their way to the host -----------------------------------------------------------------------------
+// A copy to pageable memory is a blit into the runtime's staging memory, a wait for it and a copy out of that, and the counter of
+// blocks that gave up waiting cost another one after each product of 256 x 256 tiles or LSTM sequence.  Up to kMailWords words
+// are written to page-locked memory by a kernel of one block instead, the counter beside them, before the one wait.  A small kernel
+// and 4 bytes of its result 25.3 -> 16.8 us, 16 KiB 25.6 -> 18.2 (the wait alone: 13); the counter 19 us a wait.  Beyond, bytes
+// that are not whole words and memory that is not this GPU's go through the copy.
+constexpr unsigned kMailWords = 4096, kMailThreads = 1024;
+
+struct dyhip::Mailbox {
+  std::mutex in_use;  // from the launch until the words have been taken out
+  unsigned* words;    // kMailWords, and the counter
+};
+
+static Mailbox* mailbox_new() {
+  void* p = nullptr;
+  if (hipHostMalloc(&p, (kMailWords + 1) * sizeof(unsigned), hipHostMallocDefault) != hipSuccess) return nullptr;
+  Mailbox* m = new Mailbox;
+  m->words = static_cast<unsigned*>(p);
+  return m;
+}
+
+static void mailbox_delete(Mailbox* m) {
+  if (m == nullptr) return;
+  (void)hipHostFree(m->words);
+  delete m;
+}
+
+__global__ __launch_bounds__(kMailThreads) void mail_kernel(const unsigned* __restrict__ src, unsigned n,
+                                                            const unsigned* __restrict__ counter, unsigned* __restrict__ words) {
+  unsigned v[kMailWords / kMailThreads];
+#pragma unroll
+  for (unsigned u = 0; u < kMailWords / kMailThreads; ++u) {
+    const unsigned i = threadIdx.x + u * blockDim.x;
+    if (i < n) v[u] = src[i];
+  }
+#pragma unroll
+  for (unsigned u = 0; u < kMailWords / kMailThreads; ++u) {
+    const unsigned i = threadIdx.x + u * blockDim.x;
+    if (i < n) words[i] = v[u];
+  }
+  if (counter != nullptr && threadIdx.x == 0) words[kMailWords] = *counter;
+}
+
+// Whether kernels of this thread's current device may be launched on the queue now (a copy may be issued from any device, and
+// reports a capture itself).
+static bool mail_possible(const dyhip_device* q) {
+  int current = -1;
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  return q->mailbox != nullptr && hipGetDevice(&current) == hipSuccess && current == q->ordinal &&
+         hipStreamIsCapturing(q->stream, &status) == hipSuccess && status == hipStreamCaptureStatusNone;
+}
+
+// Whether a kernel on the queue may read nbytes at src in words: wholly inside an allocation in this GPU's memory.
+static bool mail_can_read(const dyhip_device* q, const void* src, size_t nbytes) {
+  if (nbytes > kMailWords * sizeof(unsigned) || nbytes % 4 != 0 || (reinterpret_cast<uintptr_t>(src) & 3u) != 0) return false;
+  hipPointerAttribute_t at;
+  hipDeviceptr_t base = nullptr;
+  size_t size = 0;
+  if (hipPointerGetAttributes(&at, src) != hipSuccess ||
+      hipMemGetAddressRange(&base, &size, const_cast<void*>(src)) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  const size_t before = static_cast<const char*>(src) - static_cast<const char*>(base);
+  return at.type == hipMemoryTypeDevice && at.device == q->ordinal && before <= size && nbytes <= size - before;
+}
+
+// Waits for a queue.  With the wait come nbytes at src (mail_can_read; 0: none) and the number of blocks that gave up waiting for
+// another one since the last such call.
+static int queue_wait(dyhip_device* q, void* dst, const void* src, size_t nbytes, unsigned* gave_up) {
   *gave_up = 0;
-  if (!q->gemm_flags_used || q->gemm_flags == nullptr) return DYHIP_OK;
+  const unsigned* counter = q->gemm_flags_used && q->gemm_flags != nullptr ? q->gemm_flags + kGemmFlagWords - 1 : nullptr;
+  if (nbytes == 0 && (counter == nullptr || !mail_possible(q))) {
+    DYHIP_CHECK_HIP(hipStreamSynchronize(q->stream));
+    if (counter == nullptr) return DYHIP_OK;
+    DYHIP_CHECK_HIP(hipMemcpyAsync(gave_up, counter, sizeof(unsigned), hipMemcpyDeviceToHost, q->stream));
+    DYHIP_CHECK_HIP(hipStreamSynchronize(q->stream));
+  } else {
+    std::lock_guard<std::mutex> lock(q->mailbox->in_use);
+    const unsigned n = static_cast<unsigned>(nbytes / sizeof(unsigned));
+    hipLaunchKernelGGL(mail_kernel, dim3(1), dim3(n <= 256 ? 64 : kMailThreads), 0, q->stream, static_cast<const unsigned*>(src),
+                       n, counter, q->mailbox->words);
+    DYHIP_CHECK_LAUNCH();
+    DYHIP_CHECK_HIP(hipStreamSynchronize(q->stream));
+    if (nbytes > 0) std::memcpy(dst, q->mailbox->words, nbytes);
+    if (counter == nullptr) return DYHIP_OK;
+    *gave_up = q->mailbox->words[kMailWords];
+  }
   q->gemm_flags_used = false;
-  DYHIP_CHECK_HIP(hipMemcpyAsync(gave_up, q->gemm_flags + kGemmFlagWords - 1, sizeof(unsigned), hipMemcpyDeviceToHost,
-                                 q->stream));
-  DYHIP_CHECK_HIP(hipStreamSynchronize(q->stream));
   // a waiter that gave up cleared a flag that its late producer raised afterwards: start the next launch clean
   if (*gave_up != 0) DYHIP_CHECK_STATUS(gemm_flags_clear(q));
   return DYHIP_OK;
 }
 
-// Called by every entry point that has just synchronised dev's stream and hands results to the host: turns waits
+// Behind every entry point that synchronises dev's stream and hands results to the host: turns waits
 // that gave up inside a 256 x 256-tile GEMM or an LSTM sequence (on this queue, or on a queue forked from it: a graph launched here may
 // hold products recorded there) into an error.
-int dyhip::gemm_check_giveups(dyhip_device* dev) {
+static int wait_and_check(dyhip_device* dev, void* dst, const void* src, size_t nbytes) {
   unsigned total = 0, n = 0;
-  DYHIP_CHECK_STATUS(gemm_giveups_of_queue(dev, &n));
+  DYHIP_CHECK_STATUS(queue_wait(dev, dst, src, nbytes, &n));
   total += n;
   for (dyhip_device* f : dev->forks) {
     if (!f->gemm_flags_used) continue;
-    DYHIP_CHECK_HIP(hipStreamSynchronize(f->stream));
-    DYHIP_CHECK_STATUS(gemm_giveups_of_queue(f, &n));
+    DYHIP_CHECK_STATUS(queue_wait(f, nullptr, nullptr, 0, &n));
     total += n;
   }
   if (total != 0)
@@ -198,6 +279,8 @@ int dyhip::gemm_check_giveups(dyhip_device* dev) {
                                    "the last synchronisation are incomplete", total);
   return DYHIP_OK;
 }
+
+int dyhip::sync_and_check_giveups(dyhip_device* dev) { return wait_and_check(dev, nullptr, nullptr, 0); }
 
 extern "C" {
 
@@ -347,6 +430,7 @@ int dyhip_device_create(int ordinal, const size_t pool_mb[4], dyhip_device** out
   dev->gemm_flags = nullptr;
   dev->gemm_flags_used = false;
   dev->ln_scratch = nullptr;
+  dev->mailbox = nullptr;
   dev->stream_threshold = size_t(8) << 20;
   hipError_t e = hipStreamCreateWithFlags(&dev->stream, hipStreamNonBlocking);
   if (e != hipSuccess) {
@@ -373,6 +457,10 @@ int dyhip_device_create(int ordinal, const size_t pool_mb[4], dyhip_device** out
   if (st == DYHIP_OK) {
     dev->rng_state = static_cast<uint64_t*>(dev->alloc->malloc(256));
     if (dev->rng_state == nullptr) st = fail(DYHIP_ERR_OUT_OF_MEMORY, "failed to allocate the random generator state");
+  }
+  if (st == DYHIP_OK) {
+    dev->mailbox = mailbox_new();
+    if (dev->mailbox == nullptr) st = fail(DYHIP_ERR_OUT_OF_MEMORY, "failed to allocate page-locked memory for small results");
   }
   if (st == DYHIP_OK) st = dyhip_reset_rng(dev, 0);
   if (st == DYHIP_OK) st = ln_static_scratch_setup(dev);  // this device is current (hipSetDevice above)
@@ -402,6 +490,7 @@ int dyhip_device_fork(dyhip_device* parent, dyhip_device** out) {
   dev->sync_next = 0;
   dev->gemm_ws = nullptr;
   dev->rng_state = nullptr;
+  dev->mailbox = nullptr;
   hipError_t e = hipStreamCreateWithFlags(&dev->stream, hipStreamNonBlocking);
   if (e != hipSuccess) {
     delete dev;
@@ -414,7 +503,8 @@ int dyhip_device_fork(dyhip_device* parent, dyhip_device** out) {
   dev->gemm_ws = parent->alloc->malloc(dev->gemm_ws_bytes + kGemmFlagWords * sizeof(unsigned));
   dev->rng_state = static_cast<uint64_t*>(parent->alloc->malloc(256));
   dev->rng_stream = ++parent->forks_made;
-  if (dev->gemm_ws == nullptr || dev->rng_state == nullptr) {
+  dev->mailbox = mailbox_new();
+  if (dev->gemm_ws == nullptr || dev->rng_state == nullptr || dev->mailbox == nullptr) {
     dyhip_device_destroy(dev);
     return fail(DYHIP_ERR_OUT_OF_MEMORY, "failed to allocate the workspace of the forked queue");
   }
@@ -470,6 +560,7 @@ int dyhip_device_destroy(dyhip_device* dev) {
       }
     if (dev->gemm_ws) dev->alloc->free(dev->gemm_ws);
     if (dev->rng_state) dev->alloc->free(dev->rng_state);
+    mailbox_delete(dev->mailbox);
     (void)hipEventDestroy(dev->ev_start);
     (void)hipEventDestroy(dev->ev_stop);
     (void)hipStreamDestroy(dev->stream);
@@ -482,6 +573,7 @@ int dyhip_device_destroy(dyhip_device* dev) {
   if (dev->scalars) dev->alloc->free(dev->scalars);
   if (dev->rng_state) dev->alloc->free(dev->rng_state);
   if (dev->gemm_ws) dev->alloc->free(dev->gemm_ws);
+  mailbox_delete(dev->mailbox);
   delete dev->alloc;
   (void)hipEventDestroy(dev->ev_start);
   (void)hipEventDestroy(dev->ev_stop);
@@ -492,8 +584,7 @@ int dyhip_device_destroy(dyhip_device* dev) {
 
 int dyhip_device_sync(dyhip_device* dev) {
   DYHIP_CHECK_DEV(dev);
-  DYHIP_CHECK_HIP(hipStreamSynchronize(dev->stream));
-  return gemm_check_giveups(dev);
+  return sync_and_check_giveups(dev);
 }
 
 int dyhip_device_set_gemm_handoff(dyhip_device* dev, unsigned spin_limit, int raise_flags) {
@@ -573,9 +664,10 @@ int dyhip_memcpy_d2h(dyhip_device* dev, void* dst_host, const void* src, size_t 
   DYHIP_CHECK_DEV(dev);
   if (nbytes == 0) return DYHIP_OK;
   DYHIP_REQUIRE(dst_host != nullptr && src != nullptr, "null pointer in d2h copy");
+  // with the check for waits that gave up: the bytes may be the output of a product that is incomplete
+  if (mail_possible(dev) && mail_can_read(dev, src, nbytes)) return wait_and_check(dev, dst_host, src, nbytes);
   DYHIP_CHECK_HIP(hipMemcpyAsync(dst_host, src, nbytes, hipMemcpyDeviceToHost, dev->stream));
-  DYHIP_CHECK_HIP(hipStreamSynchronize(dev->stream));
-  return gemm_check_giveups(dev);  // the bytes may be the output of a product that is incomplete
+  return sync_and_check_giveups(dev);
 }
 
 int dyhip_memcpy_d2d(dyhip_device* dev, void* dst, const void* src, size_t nbytes) {

@@ -1305,9 +1305,7 @@ int dyhip_lookup_plan_invalid_ids(dyhip_device* dev, unsigned n_ids, const void*
   DYHIP_REQUIRE(plan != nullptr, "null pointer in lookup plan");
   Plan w;
   plan_parts(plan, n_ids, &w);
-  DYHIP_CHECK_HIP(hipMemcpyAsync(count, w.status, sizeof(unsigned), hipMemcpyDeviceToHost, dev->stream));
-  DYHIP_CHECK_HIP(hipStreamSynchronize(dev->stream));
-  return gemm_check_giveups(dev);
+  return dyhip_memcpy_d2h(dev, count, w.status, sizeof(unsigned));
 }
 
 int dyhip_lookup_accumulate_grads_planned_workspace(unsigned n_ids, size_t dim, size_t* ws_bytes) {

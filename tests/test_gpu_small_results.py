@@ -1,0 +1,52 @@
+"""Results on their way to the host: by a kernel into page-locked memory up to 16 KiB of whole words, by a copy otherwise."""
+import threading
+
+import numpy as np
+import pytest
+
+from dynet_amd import DevTensor
+from dynet_amd.device import PinnedArray
+from tests.util import f32
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("offset", [0, 1, 4, 12])  # bytes
+@pytest.mark.parametrize("nbytes", [1, 4, 6, 252, 256, 260, 1024, 4092, 16380, 16384, 16388, 20001])  # 64 threads, 1024; copies
+def test_every_byte_comes_back_and_none_beside_it(dev, nbytes, offset):
+    x = np.random.default_rng(nbytes).integers(0, 256, 20480).astype(np.uint8)
+    whole = dev.empty(x.size // 4, np.uint32)
+    whole.set(x.view(np.uint32))
+    src = DevTensor(dev, whole.ptr + offset, (nbytes,), np.uint8)
+    assert np.array_equal(src.numpy(), x[offset:offset + nbytes])
+
+
+def test_results_of_several_threads_and_queues(dev):
+    """Each thread reads its own tensor over and over, two of them through a queue of their own."""
+    xs = [f32(np.full(1 + 1000 * k, k + 0.5)) for k in range(4)]
+    ts = [dev.tensor(x) for x in xs]
+    dev.sync()
+    forks = [dev.fork(), dev.fork()]
+    wrong = []
+
+    def read(k):
+        t = ts[k] if k < 2 else DevTensor(forks[k - 2], ts[k].ptr, ts[k].shape, np.float32)
+        for _ in range(200):
+            if not np.array_equal(t.numpy(), xs[k]):
+                wrong.append(k)
+
+    threads = [threading.Thread(target=read, args=(k,)) for k in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for f in forks:
+        f.close()
+    assert not wrong
+
+
+def test_a_source_outside_the_gpus_memory_is_copied(dev):
+    staging = PinnedArray((8,))
+    staging.array[:] = np.arange(8)
+    assert np.array_equal(DevTensor(dev, staging.ptr, (8,), np.float32).numpy(), np.arange(8, dtype=np.float32))
+    staging.close()
