@@ -7,6 +7,7 @@
 // newest block overflows, consolidation into one block of the total capacity
 // on free(), zero-fill at block creation, used()/set_used() only meaningful
 // while there is a single block.
+#include <chrono>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -171,21 +172,24 @@ static int gemm_flags_setup(dyhip_device* dev) {
 // ---- small results on their way to the host -----------------------------------------------------------------------------
 // A copy to pageable memory is a blit into the runtime's staging memory, a wait for it and a copy out of that, and the counter of
 // blocks that gave up waiting cost another one after each product of 256 x 256 tiles or LSTM sequence.  Up to kMailWords words
-// are written to page-locked memory by a kernel of one block instead, the counter beside them, before the one wait.  A small kernel
-// and 4 bytes of its result 25.3 -> 16.8 us, 16 KiB 25.6 -> 18.2 (the wait alone: 13); the counter 19 us a wait.  Beyond, bytes
-// that are not whole words and memory that is not this GPU's go through the copy.
+// are written to page-locked memory by a kernel of one block instead, the counter beside them and then the launch's ticket, which
+// the host polls: a wait through the runtime takes 4.5 us longer (a marker behind the kernel, and its signal).  A small kernel and
+// 4 bytes of its result 25.3 -> 12.1 us, 16 KiB 25.9 -> 17.5 (kernel and runtime's wait alone: 13); the counter 19 us a wait.
+// Beyond, bytes that are not whole words and memory that is not this GPU's go through the copy.
 constexpr unsigned kMailWords = 4096, kMailThreads = 1024;
 
 struct dyhip::Mailbox {
   std::mutex in_use;  // from the launch until the words have been taken out
-  unsigned* words;    // kMailWords, and the counter
+  unsigned* words;    // kMailWords, the counter, and the ticket of the last launch whose words are all there
+  unsigned ticket;
 };
 
 static Mailbox* mailbox_new() {
   void* p = nullptr;
-  if (hipHostMalloc(&p, (kMailWords + 1) * sizeof(unsigned), hipHostMallocDefault) != hipSuccess) return nullptr;
+  if (hipHostMalloc(&p, (kMailWords + 2) * sizeof(unsigned), hipHostMallocDefault) != hipSuccess) return nullptr;
   Mailbox* m = new Mailbox;
   m->words = static_cast<unsigned*>(p);
+  m->words[kMailWords + 1] = m->ticket = 0;
   return m;
 }
 
@@ -196,7 +200,8 @@ static void mailbox_delete(Mailbox* m) {
 }
 
 __global__ __launch_bounds__(kMailThreads) void mail_kernel(const unsigned* __restrict__ src, unsigned n,
-                                                            const unsigned* __restrict__ counter, unsigned* __restrict__ words) {
+                                                            const unsigned* __restrict__ counter, unsigned* __restrict__ words,
+                                                            unsigned ticket) {
   unsigned v[kMailWords / kMailThreads];
 #pragma unroll
   for (unsigned u = 0; u < kMailWords / kMailThreads; ++u) {
@@ -209,6 +214,9 @@ __global__ __launch_bounds__(kMailThreads) void mail_kernel(const unsigned* __re
     if (i < n) words[i] = v[u];
   }
   if (counter != nullptr && threadIdx.x == 0) words[kMailWords] = *counter;
+  __threadfence_system();
+  __syncthreads();
+  if (threadIdx.x == 0) __hip_atomic_store(words + kMailWords + 1, ticket, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // Whether kernels of this thread's current device may be launched on the queue now (a copy may be issued from any device, and
@@ -235,6 +243,20 @@ static bool mail_can_read(const dyhip_device* q, const void* src, size_t nbytes)
   return at.type == hipMemoryTypeDevice && at.device == q->ordinal && before <= size && nbytes <= size - before;
 }
 
+// Whether the words of the last launch are there within 200 us; the caller waits through the runtime if not, and for every 256th
+// launch, so that the runtime sees launches end too.
+static bool mail_arrives(const Mailbox* m) {
+  if (m->ticket % 256 == 0) return false;
+  const auto end = std::chrono::steady_clock::now() + std::chrono::microseconds(200);
+  do {
+    for (int i = 0; i < 64; ++i) {
+      if (__atomic_load_n(m->words + kMailWords + 1, __ATOMIC_ACQUIRE) == m->ticket) return true;
+      __builtin_ia32_pause();
+    }
+  } while (std::chrono::steady_clock::now() < end);
+  return false;
+}
+
 // Waits for a queue.  With the wait come nbytes at src (mail_can_read; 0: none) and the number of blocks that gave up waiting for
 // another one since the last such call.
 static int queue_wait(dyhip_device* q, void* dst, const void* src, size_t nbytes, unsigned* gave_up) {
@@ -249,9 +271,9 @@ static int queue_wait(dyhip_device* q, void* dst, const void* src, size_t nbytes
     std::lock_guard<std::mutex> lock(q->mailbox->in_use);
     const unsigned n = static_cast<unsigned>(nbytes / sizeof(unsigned));
     hipLaunchKernelGGL(mail_kernel, dim3(1), dim3(n <= 256 ? 64 : kMailThreads), 0, q->stream, static_cast<const unsigned*>(src),
-                       n, counter, q->mailbox->words);
+                       n, counter, q->mailbox->words, ++q->mailbox->ticket);
     DYHIP_CHECK_LAUNCH();
-    DYHIP_CHECK_HIP(hipStreamSynchronize(q->stream));
+    if (!mail_arrives(q->mailbox)) DYHIP_CHECK_HIP(hipStreamSynchronize(q->stream));
     if (nbytes > 0) std::memcpy(dst, q->mailbox->words, nbytes);
     if (counter == nullptr) return DYHIP_OK;
     *gave_up = q->mailbox->words[kMailWords];

@@ -45,6 +45,14 @@ def test_results_of_several_threads_and_queues(dev):
     assert not wrong
 
 
+@pytest.mark.parametrize("n", [1, 256, 300, 4096])
+def test_each_result_is_that_of_the_kernel_before(dev, n):
+    x = dev.empty(n)
+    for k in range(600):  # past the launches that are waited for through the runtime
+        dev.constant(x, k + 0.25)
+        assert np.all(x.numpy() == k + 0.25)
+
+
 def test_a_source_outside_the_gpus_memory_is_copied(dev):
     staging = PinnedArray((8,))
     staging.array[:] = np.arange(8)
