@@ -736,10 +736,9 @@ def lstm_lm(steps, warmup=12, use_graph=True):
                       "clip_threshold": 5.0, "init": "Glorot (lookup: embedding dim only), LSTM biases 0",
                       "ids": "Zipf(1.1)"},
            "tokens_per_step": T * B, "gemm_flop_per_step": flops,
-           "fused_path_schedule": "one device queue, layer by layer; a forward timestep is one kernel (recurrent "
-                                  "product + cell update) and so is a backward one (Wh^T dpre of the step above + "
-                                  "cell backward), operands handed from timestep to timestep in matrix-core "
-                                  "fragment order",
+           "fused_path_schedule": "one device queue, layer by layer; all timesteps of a layer are one kernel forward "
+                                  "(recurrent product + cell update) and one backward (Wh^T dpre of the step above + "
+                                  "cell backward), the recurrent weights kept on chip",
            "node_path_schedule": "the three fused LSTM nodes per layer and timestep, every backward argument its own "
                                  "call; the gates nodes' backward calls for Wx, Wh and b record their operands and the "
                                  "T recorded products of a parameter are formed as one product over the gathered "
