@@ -11,6 +11,7 @@
 // (max, sum of exp(x - max)) pair over its 128-bit slices, pairs are merged by
 // wave butterfly and then across waves through LDS.  Backward is one
 // elementwise read-modify-write pass with the one-hot subtraction folded in.
+#include <algorithm>
 #include <cmath>
 #include <vector>
 
@@ -57,13 +58,35 @@ __device__ __forceinline__ MaxSum ms_merge(const MaxSum a, const MaxSum b) {
   return r;
 }
 
-// One block per batch element.  Writes m[b], z[b]; if ids != nullptr also
+// Where the picked positions of PickNegLogSoftmax come from: device memory (null: nothing is picked), or with the launch, up to
+// kHostWords of them, and then they are written to device memory too, for the backward pass.  A kernel of its own that put them
+// there waited for the argument block in host memory before the columns could be read; here that wait lies under them (zero, forward
+// and backward of 50 000 x 512 82.2 -> 80.2 us, a classifier's training step over 512 labels 165.6 -> 163.8).
+struct DeviceIds {
+  const unsigned* ids;
+  __device__ __forceinline__ bool any() const { return ids != nullptr; }
+  __device__ __forceinline__ unsigned take(unsigned b) const { return ids[b]; }
+  int place(dyhip_device*, unsigned) const { return DYHIP_OK; }
+};
+template <unsigned N>
+struct HostIds {
+  HostWords<N> words;
+  unsigned* ids;
+  __device__ __forceinline__ bool any() const { return true; }
+  __device__ __forceinline__ unsigned take(unsigned b) const {  // by one thread for each b
+    const unsigned id = words.v[b];
+    ids[b] = id;
+    return id;
+  }
+  int place(dyhip_device* dev, unsigned n) const { return put_host_words(dev, ids, words.v, n); }
+};
+
+// One block per batch element.  Writes m[b], z[b]; if there are ids also
 // fx[b] = z[b] - x[ids[b]] (the pick of PickNegLogSoftmax).
-template <bool VEC, bool NT>
+template <bool NT, class Ids>
 __global__ __launch_bounds__(kLseThreads) void lse_cols_kernel(size_t rows, const float* __restrict__ x,
                                                                float* __restrict__ m_out, float* __restrict__ z_out,
-                                                               const unsigned* __restrict__ ids,
-                                                               float* __restrict__ fx) {
+                                                               Ids ids, float* __restrict__ fx) {
   __shared__ float lm[kLseWaves], ls[kLseWaves];
   const unsigned b = blockIdx.x;
   const float* px = x + size_t(b) * rows;
@@ -72,40 +95,36 @@ __global__ __launch_bounds__(kLseThreads) void lse_cols_kernel(size_t rows, cons
   a.s = 0.f;
   // the picked logit is fetched up front so that its two dependent loads overlap the streaming pass
   float picked = 0.f;
-  if (ids != nullptr && threadIdx.x == 0) picked = x[ids[b]];
-  if (VEC) {
-    // A column starts wherever b * rows falls: up to three leading elements bring it to a 16-byte boundary, the body
-    // runs in 128-bit groups, up to three elements trail (taken by the last threads of the block).  With rows a
-    // multiple of four and an aligned x there is only the body.
-    const size_t head = min(size_t((4u - unsigned((reinterpret_cast<uintptr_t>(px) >> 2) & 3u)) & 3u), rows);
-    const size_t n4 = (rows - head) >> 2;
-    if (threadIdx.x < head) ms_push1(a, px[threadIdx.x]);
-    {
-      const size_t e = head + (n4 << 2) + (kLseThreads - 1 - threadIdx.x);
-      if (e < rows) ms_push1(a, px[e]);
-    }
-    const float4* p4 = reinterpret_cast<const float4*>(px + head);
-    size_t i = threadIdx.x;
-    // eight independent 128-bit loads in flight per thread before the first exp
-    for (; i + 7 * kLseThreads < n4; i += 8 * kLseThreads) {
-      float4 v[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) v[u] = ldg4<NT>(p4 + i + u * kLseThreads);
-#pragma unroll
-      for (int u = 0; u < 8; ++u) ms_push4(a, v[u]);
-    }
-    for (; i + 3 * kLseThreads < n4; i += 4 * kLseThreads) {
-      const float4 v0 = ldg4<NT>(p4 + i), v1 = ldg4<NT>(p4 + i + kLseThreads),
-                   v2 = ldg4<NT>(p4 + i + 2 * kLseThreads), v3 = ldg4<NT>(p4 + i + 3 * kLseThreads);
-      ms_push4(a, v0);
-      ms_push4(a, v1);
-      ms_push4(a, v2);
-      ms_push4(a, v3);
-    }
-    for (; i < n4; i += kLseThreads) ms_push4(a, ldg4<NT>(p4 + i));
-  } else {
-    for (size_t i = threadIdx.x; i < rows; i += kLseThreads) ms_push1(a, px[i]);
+  if (ids.any() && threadIdx.x == 0) picked = x[ids.take(b)];
+  // A column starts wherever b * rows falls: up to three leading elements bring it to a 16-byte boundary, the body
+  // runs in 128-bit groups, up to three elements trail (taken by the last threads of the block).  With rows a
+  // multiple of four and an aligned x there is only the body.
+  const size_t head = min(size_t((4u - unsigned((reinterpret_cast<uintptr_t>(px) >> 2) & 3u)) & 3u), rows);
+  const size_t n4 = (rows - head) >> 2;
+  if (threadIdx.x < head) ms_push1(a, px[threadIdx.x]);
+  {
+    const size_t e = head + (n4 << 2) + (kLseThreads - 1 - threadIdx.x);
+    if (e < rows) ms_push1(a, px[e]);
   }
+  const float4* p4 = reinterpret_cast<const float4*>(px + head);
+  size_t i = threadIdx.x;
+  // eight independent 128-bit loads in flight per thread before the first exp
+  for (; i + 7 * kLseThreads < n4; i += 8 * kLseThreads) {
+    float4 v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) v[u] = ldg4<NT>(p4 + i + u * kLseThreads);
+#pragma unroll
+    for (int u = 0; u < 8; ++u) ms_push4(a, v[u]);
+  }
+  for (; i + 3 * kLseThreads < n4; i += 4 * kLseThreads) {
+    const float4 v0 = ldg4<NT>(p4 + i), v1 = ldg4<NT>(p4 + i + kLseThreads),
+                 v2 = ldg4<NT>(p4 + i + 2 * kLseThreads), v3 = ldg4<NT>(p4 + i + 3 * kLseThreads);
+    ms_push4(a, v0);
+    ms_push4(a, v1);
+    ms_push4(a, v2);
+    ms_push4(a, v3);
+  }
+  for (; i < n4; i += kLseThreads) ms_push4(a, ldg4<NT>(p4 + i));
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) {
     MaxSum o;
@@ -137,7 +156,7 @@ __global__ __launch_bounds__(kLseThreads) void lse_cols_kernel(size_t rows, cons
       if (empty) t.m = -INFINITY;
       m_out[b] = t.m;
       z_out[b] = z;
-      if (ids != nullptr) fx[b] = z - picked;
+      if (ids.any()) fx[b] = z - picked;
     }
   }
 }
@@ -145,16 +164,16 @@ __global__ __launch_bounds__(kLseThreads) void lse_cols_kernel(size_t rows, cons
 // Short columns (rows <= 64 * U): one wavefront per column, four columns per block, every load of a column in flight
 // at once.  A 1024-thread block per column of 33 rows (a tagger's label set over a large batch) is 1023 idle threads
 // and a barrier per column: 337 us for 100 000 columns against 8 us here.
-template <int U>
+template <int U, class Ids>
 __global__ __launch_bounds__(256) void lse_cols_wave_kernel(unsigned rows, unsigned bd, const float* __restrict__ x,
                                                             float* __restrict__ m_out, float* __restrict__ z_out,
-                                                            const unsigned* __restrict__ ids, float* __restrict__ fx) {
+                                                            Ids ids, float* __restrict__ fx) {
   const unsigned b = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (b >= bd) return;  // whole wavefronts leave; the kernel has no barrier
   const int lane = threadIdx.x & 63;
   const float* px = x + size_t(b) * rows;
   float picked = 0.f;
-  if (ids != nullptr && lane == 0) picked = x[ids[b]];
+  if (ids.any() && lane == 0) picked = x[ids.take(b)];
   float v[U];
 #pragma unroll
   for (int u = 0; u < U; ++u) {
@@ -179,7 +198,7 @@ __global__ __launch_bounds__(256) void lse_cols_wave_kernel(unsigned rows, unsig
     const float z = empty ? NAN : logf(a.s) + a.m;
     m_out[b] = empty ? -INFINITY : a.m;
     z_out[b] = z;
-    if (ids != nullptr) fx[b] = z - picked;
+    if (ids.any()) fx[b] = z - picked;
   }
 }
 
@@ -187,14 +206,15 @@ __global__ __launch_bounds__(256) void lse_cols_wave_kernel(unsigned rows, unsig
 // wavefront per column the six merge steps of the butterfly, two exp each, cost more than the column's own terms:
 // 23 us for 100 000 columns of 33 rows, vector-instruction bound).  A wavefront reads 64 neighbouring columns, i.e.
 // one contiguous span, line by line through its L1.
+template <class Ids>
 __global__ __launch_bounds__(256) void lse_cols_thread_kernel(unsigned rows, unsigned bd, const float* __restrict__ x,
                                                               float* __restrict__ m_out, float* __restrict__ z_out,
-                                                              const unsigned* __restrict__ ids, float* __restrict__ fx) {
+                                                              Ids ids, float* __restrict__ fx) {
   const unsigned b = blockIdx.x * 256 + threadIdx.x;
   if (b >= bd) return;
   const float* px = x + size_t(b) * rows;
   float picked = 0.f;
-  if (ids != nullptr) picked = x[ids[b]];
+  if (ids.any()) picked = x[ids.take(b)];
   MaxSum a;
   a.m = kLseStartMax;
   a.s = 0.f;
@@ -211,7 +231,7 @@ __global__ __launch_bounds__(256) void lse_cols_thread_kernel(unsigned rows, uns
   const float z = empty ? NAN : logf(a.s) + a.m;
   m_out[b] = empty ? -INFINITY : a.m;
   z_out[b] = z;
-  if (ids != nullptr) fx[b] = z - picked;
+  if (ids.any()) fx[b] = z - picked;
 }
 
 // The backward pass over short columns, one wavefront per column as above.
@@ -707,14 +727,15 @@ static void launch_argmax_cols(dyhip_device* dev, size_t rows, unsigned bd, cons
 int batch_reduce(dyhip_device* dev, size_t n, unsigned bd, const float* in0, const float* in1, float* out,
                  bool accumulate, void* ws, size_t ws_bytes);
 
-static int launch_lse(dyhip_device* dev, size_t rows, unsigned bd, const float* x, float* m, float* z,
-                      const unsigned* ids, float* fx) {
+template <class Ids>
+static int launch_lse(dyhip_device* dev, size_t rows, unsigned bd, const float* x, float* m, float* z, const Ids& ids,
+                      float* fx) {
   if (rows <= kLseWaveMaxRows) {
     const dim3 grid(cdiv<unsigned>(bd, 4)), block(256);
     const unsigned r = static_cast<unsigned>(rows);
-#define DYHIP_LSE_WAVE(U) hipLaunchKernelGGL(lse_cols_wave_kernel<U>, grid, block, 0, dev->stream, r, bd, x, m, z, ids, fx)
+#define DYHIP_LSE_WAVE(U) hipLaunchKernelGGL((lse_cols_wave_kernel<U, Ids>), grid, block, 0, dev->stream, r, bd, x, m, z, ids, fx)
     if (r <= 64)
-      hipLaunchKernelGGL(lse_cols_thread_kernel, dim3(cdiv<unsigned>(bd, 256)), block, 0, dev->stream, r, bd, x, m, z, ids, fx);
+      hipLaunchKernelGGL(lse_cols_thread_kernel<Ids>, dim3(cdiv<unsigned>(bd, 256)), block, 0, dev->stream, r, bd, x, m, z, ids, fx);
     else if (r <= 128) DYHIP_LSE_WAVE(2);
     else if (r <= 256) DYHIP_LSE_WAVE(4);
     else DYHIP_LSE_WAVE(8);
@@ -724,23 +745,30 @@ static int launch_lse(dyhip_device* dev, size_t rows, unsigned bd, const float* 
   }
   unsigned chunks = 0;
   if (col_chunked(dev, rows, bd, &chunks)) {
+    DYHIP_CHECK_STATUS(ids.place(dev, bd));
     float* part = static_cast<float*>(dev->gemm_ws);
     hipLaunchKernelGGL(col_chunk_kernel<0>, dim3(chunks, bd), dim3(256), 0, dev->stream, rows, x, nullptr, part);
-    hipLaunchKernelGGL(col_finish_kernel<0>, dim3(bd), dim3(64), 0, dev->stream, rows, chunks, part, x, ids, m, z, fx,
+    hipLaunchKernelGGL(col_finish_kernel<0>, dim3(bd), dim3(64), 0, dev->stream, rows, chunks, part, x, ids.ids, m, z, fx,
                        nullptr);
     DYHIP_CHECK_LAUNCH();
     return DYHIP_OK;
   }
-  const bool vec = true;  // any column: its ends are peeled off around a body of 128-bit groups
-  const bool stream = rows * size_t(bd) * sizeof(float) >= dev->stream_threshold;
-  if (vec && stream)
-    hipLaunchKernelGGL((lse_cols_kernel<true, true>), dim3(bd), dim3(kLseThreads), 0, dev->stream, rows, x, m, z, ids, fx);
-  else if (vec)
-    hipLaunchKernelGGL((lse_cols_kernel<true, false>), dim3(bd), dim3(kLseThreads), 0, dev->stream, rows, x, m, z, ids, fx);
+  if (rows * size_t(bd) * sizeof(float) >= dev->stream_threshold)
+    hipLaunchKernelGGL((lse_cols_kernel<true, Ids>), dim3(bd), dim3(kLseThreads), 0, dev->stream, rows, x, m, z, ids, fx);
   else
-    hipLaunchKernelGGL((lse_cols_kernel<false, false>), dim3(bd), dim3(kLseThreads), 0, dev->stream, rows, x, m, z, ids, fx);
+    hipLaunchKernelGGL((lse_cols_kernel<false, Ids>), dim3(bd), dim3(kLseThreads), 0, dev->stream, rows, x, m, z, ids, fx);
   DYHIP_CHECK_LAUNCH();
   return DYHIP_OK;
+}
+
+template <unsigned N>
+static int launch_lse_host(dyhip_device* dev, size_t rows, unsigned bd, const float* x, float* m, float* z,
+                           const unsigned* ids_host, unsigned* ids_dev, float* fx) {
+  DYHIP_CHECK_STATUS(refuse_while_capturing(dev));
+  HostIds<N> ids;
+  std::copy(ids_host, ids_host + bd, ids.words.v);
+  ids.ids = ids_dev;
+  return launch_lse(dev, rows, bd, x, m, z, ids, fx);
 }
 
 // ---- Softmax / LogSoftmax over dim 0 ---------------------------------------------------
@@ -1277,7 +1305,7 @@ int dyhip_logsumexp_cols(dyhip_device* dev, size_t rows, unsigned bd, const floa
   DYHIP_CHECK_DEV(dev);
   DYHIP_REQUIRE(rows >= 1 && x && m && z, "logsumexp needs a non-empty tensor");
   if (bd == 0) return DYHIP_OK;
-  return launch_lse(dev, rows, bd, x, m, z, nullptr, nullptr);
+  return launch_lse(dev, rows, bd, x, m, z, DeviceIds{nullptr}, nullptr);
 }
 
 int dyhip_pnls_forward(dyhip_device* dev, size_t rows, unsigned bd, const float* x, const unsigned* labels_host,
@@ -1296,13 +1324,15 @@ int dyhip_pnls_forward(dyhip_device* dev, size_t rows, unsigned bd, const float*
   float* z = static_cast<float*>(aux);
   float* m = z + bd;
   unsigned* ids_dev = reinterpret_cast<unsigned*>(m + bd);
+  if (bd <= kFewHostWords) return launch_lse_host<kFewHostWords>(dev, rows, bd, x, m, z, ids.data(), ids_dev, fx);
+  if (bd <= kHostWords) return launch_lse_host<kHostWords>(dev, rows, bd, x, m, z, ids.data(), ids_dev, fx);
   if (bd <= kPutHostWordsMost) {
     DYHIP_CHECK_STATUS(put_host_words(dev, ids_dev, ids.data(), bd));
   } else {  // pageable source, read until the copy is done
     DYHIP_CHECK_HIP(hipMemcpyAsync(ids_dev, ids.data(), sizeof(unsigned) * bd, hipMemcpyHostToDevice, dev->stream));
     DYHIP_CHECK_HIP(hipStreamSynchronize(dev->stream));
   }
-  return launch_lse(dev, rows, bd, x, m, z, ids_dev, fx);
+  return launch_lse(dev, rows, bd, x, m, z, DeviceIds{ids_dev}, fx);
 }
 
 int dyhip_pnls_forward_staged(dyhip_device* dev, size_t rows, unsigned bd, const float* x, void* aux, float* fx) {
@@ -1311,7 +1341,7 @@ int dyhip_pnls_forward_staged(dyhip_device* dev, size_t rows, unsigned bd, const
   if (bd == 0) return DYHIP_OK;
   float* z = static_cast<float*>(aux);
   float* m = z + bd;
-  return launch_lse(dev, rows, bd, x, m, z, reinterpret_cast<const unsigned*>(m + bd), fx);
+  return launch_lse(dev, rows, bd, x, m, z, DeviceIds{reinterpret_cast<const unsigned*>(m + bd)}, fx);
 }
 
 int dyhip_pnls_backward(dyhip_device* dev, size_t rows, unsigned bd, const float* x, const void* aux,
@@ -1418,7 +1448,7 @@ int dyhip_softmax_forward(dyhip_device* dev, size_t rows, unsigned cols, const f
     DYHIP_CHECK_LAUNCH();
     return DYHIP_OK;
   }
-  DYHIP_CHECK_STATUS(launch_lse(dev, rows, cols, x, m, z, nullptr, nullptr));
+  DYHIP_CHECK_STATUS(launch_lse(dev, rows, cols, x, m, z, DeviceIds{nullptr}, nullptr));
   return launch_col_apply<0>(dev, rows, cols, x, nullptr, m, z, fx);
 }
 
@@ -1462,7 +1492,7 @@ int dyhip_logsumexp_dim_forward(dyhip_device* dev, size_t rows, size_t cols, uns
   if (bd == 0) return DYHIP_OK;
   if (dim == 0) {
     DYHIP_REQUIRE(cols * size_t(bd) <= 0xffffffffu, "too many columns");
-    return launch_lse(dev, rows, static_cast<unsigned>(cols * bd), x, m, fx, nullptr, nullptr);
+    return launch_lse(dev, rows, static_cast<unsigned>(cols * bd), x, m, fx, DeviceIds{nullptr}, nullptr);
   }
   return launch_rowwise<0>(dev, rows, cols, bd, x, nullptr, m, fx);
 }
@@ -1492,7 +1522,7 @@ int dyhip_log_softmax_forward(dyhip_device* dev, size_t rows, unsigned cols, con
     DYHIP_CHECK_LAUNCH();
     return DYHIP_OK;
   }
-  DYHIP_CHECK_STATUS(launch_lse(dev, rows, cols, x, m, z, nullptr, nullptr));
+  DYHIP_CHECK_STATUS(launch_lse(dev, rows, cols, x, m, z, DeviceIds{nullptr}, nullptr));
   return launch_col_apply<1>(dev, rows, cols, x, nullptr, z, nullptr, fx);
 }
 

@@ -36,6 +36,28 @@ def test_pnls_of_host_labels(dev, n):
     assert np.max(np.abs(fx.numpy() - exact)) <= 8 * 2.0 ** -23 + 33 * 2.0 ** -24
 
 
+@pytest.mark.parametrize("rows,n", [(r, n) for r in (1, 64, 65, 512, 513, 4099) for n in (1, 64, 65, 960)]
+                         + [(65536, 1), (70001, 64), (65537, 65)])
+def test_pnls_of_host_labels_over_every_kernel_of_the_columns(dev, rows, n):
+    """The labels reach the loss and, through the auxiliary memory, the gradient; up to 64 columns of 65 536 rows are cut."""
+    rng = np.random.default_rng(n + rows)
+    x = rng.standard_normal((n, rows)).astype(np.float32)
+    labels = rng.integers(0, rows, n).astype(np.uint32)
+    xt, aux, fx = dev.tensor(x), dev.empty((3 * n,)), dev.empty((n,))
+    dy, dx = dev.tensor(np.ones(n, np.float32)), dev.tensor(np.zeros((n, rows), np.float32))
+    dev.pnls_forward(rows, n, xt, labels, aux, fx)
+    dev.pnls_backward(rows, n, xt, aux, dy, dx)
+    x64, at = x.astype(np.float64), np.arange(n)
+    z = np.log(np.exp(x64).sum(1))
+    # logarithm and difference of values below 16, each rounded once; a term of the sum goes through up to 32 sums and merges
+    bound = 16 * 2.0 ** -23 + 64 * 2.0 ** -24
+    assert np.max(np.abs(fx.numpy() - (z - x64[at, labels]))) <= bound
+    want = np.exp(x64 - z[:, None])
+    want[at, labels] -= 1.0
+    # z as above and x - z rounded below 16, under an exponential of at most one
+    assert np.max(np.abs(dx.numpy() - want)) <= 2 * bound
+
+
 def test_host_indices_are_not_recorded_into_a_graph(dev):
     tt, idd, fx = dev.tensor(np.ones((4, 8), np.float32)), dev.empty((3,), np.uint32), dev.empty((3, 8))
     aux, loss = dev.empty((9,)), dev.empty((3,))
