@@ -74,7 +74,7 @@ struct dyhip_device {
   size_t gemm_ws_bytes;
   unsigned wide_gemm_ready;  // gemm_wide.hip: kernels whose dynamic-LDS limit has been raised on this device
   unsigned* gemm_flags;      // gemm_wide.hip: kGemmFlagWords words behind gemm_ws that no other kernel touches, zero between launches
-  bool gemm_flags_used;      // a launch since the last host synchronisation may have counted a wait that gave up
+  bool gemm_flags_used;      // a launch since the last host synchronisation may have counted a wait that gave up (mark_gemm_flags_used)
   unsigned gemm_spin_limit;  // polls before a block's wait for another block's partial tile gives up
   int gemm_raise_flags;      // 0 only in tests of the give-up path: producers leave their flags down
   unsigned sequence_ready;   // lstm_sequence.hip: kernels whose dynamic-LDS limit has been raised on this device
@@ -107,6 +107,10 @@ constexpr unsigned kPutHostWordsMost = 2 * kHostWords;  // beyond, the copy and 
 
 // reduce.hip: looks up, on the current device, the address of the static scratch array (once per device handle)
 int ln_static_scratch_setup(dyhip_device* dev);
+// After a launch that may count a wait that gave up: the queue's next wait looks at the counter.  (Before the launch, another
+// thread's wait could take the mark down and read the counter too early.)
+inline void mark_gemm_flags_used(dyhip_device* dev) { __atomic_store_n(&dev->gemm_flags_used, true, __ATOMIC_RELEASE); }
+inline bool gemm_flags_marked(const dyhip_device* dev) { return __atomic_load_n(&dev->gemm_flags_used, __ATOMIC_ACQUIRE); }
 // device.hip: waits for dev's stream and reports waits that gave up inside a large GEMM or an LSTM sequence
 int sync_and_check_giveups(dyhip_device* dev);
 }  // namespace dyhip

@@ -156,8 +156,8 @@ using namespace dyhip;
 // are told, and start out zero.
 // The fill runs on the queue's own stream (a non-blocking stream is not ordered against the null stream) and has
 // finished when the call returns.
-static int gemm_flags_clear(dyhip_device* dev) {
-  DYHIP_CHECK_HIP(hipMemsetAsync(dev->gemm_flags, 0, kGemmFlagWords * sizeof(unsigned), dev->stream));
+static int gemm_flags_clear(dyhip_device* dev, unsigned words) {
+  DYHIP_CHECK_HIP(hipMemsetAsync(dev->gemm_flags, 0, words * sizeof(unsigned), dev->stream));
   DYHIP_CHECK_HIP(hipStreamSynchronize(dev->stream));
   return DYHIP_OK;
 }
@@ -166,7 +166,7 @@ static int gemm_flags_setup(dyhip_device* dev) {
   dev->gemm_flags = reinterpret_cast<unsigned*>(static_cast<char*>(dev->gemm_ws) + dev->gemm_ws_bytes);
   dev->gemm_spin_limit = 1u << 22;  // polls about a microsecond apart: seconds
   dev->gemm_raise_flags = 1;
-  return gemm_flags_clear(dev);
+  return gemm_flags_clear(dev, kGemmFlagWords);
 }
 
 // ---- small results on their way to the host -----------------------------------------------------------------------------
@@ -182,6 +182,7 @@ struct dyhip::Mailbox {
   std::mutex in_use;  // from the launch until the words have been taken out
   unsigned* words;    // kMailWords, the counter, and the ticket of the last launch whose words are all there
   unsigned ticket;
+  unsigned reported;  // of the queue's give-up counter
 };
 
 static Mailbox* mailbox_new() {
@@ -189,7 +190,7 @@ static Mailbox* mailbox_new() {
   if (hipHostMalloc(&p, (kMailWords + 2) * sizeof(unsigned), hipHostMallocDefault) != hipSuccess) return nullptr;
   Mailbox* m = new Mailbox;
   m->words = static_cast<unsigned*>(p);
-  m->words[kMailWords + 1] = m->ticket = 0;
+  m->words[kMailWords + 1] = m->ticket = m->reported = 0;
   return m;
 }
 
@@ -257,30 +258,49 @@ static bool mail_arrives(const Mailbox* m) {
   return false;
 }
 
-// Waits for a queue.  With the wait come nbytes at src (mail_can_read; 0: none) and the number of blocks that gave up waiting for
-// another one since the last such call.
-static int queue_wait(dyhip_device* q, void* dst, const void* src, size_t nbytes, unsigned* gave_up) {
-  *gave_up = 0;
-  const unsigned* counter = q->gemm_flags_used && q->gemm_flags != nullptr ? q->gemm_flags + kGemmFlagWords - 1 : nullptr;
+// Waits for a queue; with the wait come nbytes at src (mail_can_read; 0: none) and, where asked for, the give-up counter.
+static int wait_with_words(dyhip_device* q, void* dst, const void* src, size_t nbytes, const unsigned* counter, unsigned* count) {
   if (nbytes == 0 && (counter == nullptr || !mail_possible(q))) {
     DYHIP_CHECK_HIP(hipStreamSynchronize(q->stream));
     if (counter == nullptr) return DYHIP_OK;
-    DYHIP_CHECK_HIP(hipMemcpyAsync(gave_up, counter, sizeof(unsigned), hipMemcpyDeviceToHost, q->stream));
+    DYHIP_CHECK_HIP(hipMemcpyAsync(count, counter, sizeof(unsigned), hipMemcpyDeviceToHost, q->stream));
     DYHIP_CHECK_HIP(hipStreamSynchronize(q->stream));
-  } else {
-    std::lock_guard<std::mutex> lock(q->mailbox->in_use);
-    const unsigned n = static_cast<unsigned>(nbytes / sizeof(unsigned));
-    hipLaunchKernelGGL(mail_kernel, dim3(1), dim3(n <= 256 ? 64 : kMailThreads), 0, q->stream, static_cast<const unsigned*>(src),
-                       n, counter, q->mailbox->words, ++q->mailbox->ticket);
-    DYHIP_CHECK_LAUNCH();
-    if (!mail_arrives(q->mailbox)) DYHIP_CHECK_HIP(hipStreamSynchronize(q->stream));
-    if (nbytes > 0) std::memcpy(dst, q->mailbox->words, nbytes);
-    if (counter == nullptr) return DYHIP_OK;
-    *gave_up = q->mailbox->words[kMailWords];
+    return DYHIP_OK;
   }
-  q->gemm_flags_used = false;
+  const unsigned n = static_cast<unsigned>(nbytes / sizeof(unsigned));
+  hipLaunchKernelGGL(mail_kernel, dim3(1), dim3(n <= 256 ? 64 : kMailThreads), 0, q->stream, static_cast<const unsigned*>(src),
+                     n, counter, q->mailbox->words, ++q->mailbox->ticket);
+  DYHIP_CHECK_LAUNCH();
+  if (!mail_arrives(q->mailbox)) DYHIP_CHECK_HIP(hipStreamSynchronize(q->stream));
+  if (nbytes > 0) std::memcpy(dst, q->mailbox->words, nbytes);
+  if (counter != nullptr) *count = q->mailbox->words[kMailWords];
+  return DYHIP_OK;
+}
+
+// Waits for a queue.  With the wait come nbytes at src (mail_can_read; 0: none) and the number of blocks that gave up waiting for
+// another one and have not been reported yet.
+// Threads may wait for and launch on one queue at the same time.  The mark of a launch that may give up is taken down before
+// the counter is read, and put there after the launch (mark_gemm_flags_used): a launch behind the read leaves it up for the
+// next wait.  The counter itself only ever grows, so that what such a launch adds while this wait clears the flags counts too.
+static int queue_wait(dyhip_device* q, void* dst, const void* src, size_t nbytes, unsigned* gave_up) {
+  *gave_up = 0;
+  if (nbytes == 0 && (q->gemm_flags == nullptr || !gemm_flags_marked(q))) {
+    DYHIP_CHECK_HIP(hipStreamSynchronize(q->stream));
+    return DYHIP_OK;
+  }
+  std::lock_guard<std::mutex> lock(q->mailbox->in_use);
+  const bool marked = q->gemm_flags != nullptr && __atomic_exchange_n(&q->gemm_flags_used, false, __ATOMIC_ACQ_REL);
+  unsigned count = 0;
+  const int st = wait_with_words(q, dst, src, nbytes, marked ? q->gemm_flags + kGemmFlagWords - 1 : nullptr, &count);
+  if (st != DYHIP_OK) {
+    if (marked) mark_gemm_flags_used(q);
+    return st;
+  }
+  if (!marked) return DYHIP_OK;
+  *gave_up = count - q->mailbox->reported;
+  q->mailbox->reported = count;
   // a waiter that gave up cleared a flag that its late producer raised afterwards: start the next launch clean
-  if (*gave_up != 0) DYHIP_CHECK_STATUS(gemm_flags_clear(q));
+  if (*gave_up != 0) DYHIP_CHECK_STATUS(gemm_flags_clear(q, kGemmFlagWords - 1));
   return DYHIP_OK;
 }
 
@@ -292,7 +312,7 @@ static int wait_and_check(dyhip_device* dev, void* dst, const void* src, size_t 
   DYHIP_CHECK_STATUS(queue_wait(dev, dst, src, nbytes, &n));
   total += n;
   for (dyhip_device* f : dev->forks) {
-    if (!f->gemm_flags_used) continue;
+    if (!gemm_flags_marked(f)) continue;
     DYHIP_CHECK_STATUS(queue_wait(f, nullptr, nullptr, 0, &n));
     total += n;
   }
@@ -741,9 +761,9 @@ int dyhip_graph_launch(dyhip_device* dev, dyhip_graph* graph) {
   DYHIP_CHECK_HIP(hipGraphLaunch(graph->exec, dev->stream));
   // a recorded large GEMM or LSTM sequence runs again with every replay, on this queue or on one forked from it: the
   // next synchronisation looks at their give-up counters
-  if (dev->wide_gemm_ready != 0 || dev->sequence_ready != 0) dev->gemm_flags_used = true;
+  if (dev->wide_gemm_ready != 0 || dev->sequence_ready != 0) mark_gemm_flags_used(dev);
   for (dyhip_device* f : dev->forks)
-    if (f->wide_gemm_ready != 0 || f->sequence_ready != 0) f->gemm_flags_used = true;
+    if (f->wide_gemm_ready != 0 || f->sequence_ready != 0) mark_gemm_flags_used(f);
   return DYHIP_OK;
 }
 

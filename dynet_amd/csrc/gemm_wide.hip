@@ -846,7 +846,7 @@ int gemm_wide_run(dyhip_device* dev, bool a_kmajor, bool b_kmajor, size_t M, siz
   DYHIP_CHECK_STATUS(st);
   DYHIP_CHECK_LAUNCH();
   if (p.finish_in_kernel) {
-    dev->gemm_flags_used = true;
+    mark_gemm_flags_used(dev);
   } else {
     const dim3 grid(p.tiles, 16);
     if (a_kmajor && b_kmajor) hipLaunchKernelGGL((gemm_wide_fixup_kernel<true, true>), grid, dim3(kWideThreads), 0, dev->stream, g, p.segments);

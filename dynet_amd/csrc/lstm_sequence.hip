@@ -786,10 +786,10 @@ int launch_sequence(dyhip_device* dev, void (*kernel)(Args), unsigned instance, 
     dev->sequence_ready |= 1u << instance;
   }
   DYHIP_CHECK_HIP(zero_fill(a.sync.claims, p.sync_words * sizeof(unsigned), dev->stream));
-  dev->gemm_flags_used = true;
   const unsigned tiles = p.RT * p.CT, most = dev->sequence_blocks;
   hipLaunchKernelGGL(kernel, dim3(most > 0 && most < tiles ? most : tiles), dim3(kSeqThreads), lds, dev->stream, a);
   DYHIP_CHECK_LAUNCH();
+  mark_gemm_flags_used(dev);
   return DYHIP_OK;
 }
 

@@ -1,10 +1,11 @@
 """Results on their way to the host: by a kernel into page-locked memory up to 16 KiB of whole words, by a copy otherwise."""
 import threading
+import time
 
 import numpy as np
 import pytest
 
-from dynet_amd import DevTensor
+from dynet_amd import Device, DevTensor, DyhipError
 from dynet_amd.device import PinnedArray
 from tests.util import f32
 
@@ -58,3 +59,40 @@ def test_a_source_outside_the_gpus_memory_is_copied(dev):
     staging.array[:] = np.arange(8)
     assert np.array_equal(DevTensor(dev, staging.ptr, (8,), np.float32).numpy(), np.arange(8, dtype=np.float32))
     staging.close()
+
+
+def test_a_wait_that_gave_up_behind_another_threads_wait_is_reported():
+    """A thread waits for a queue with work in it while this one launches a product whose waits give up at once: the other
+    thread's read of the counter comes before that product, the next wait has to look again."""
+    d = Device(0, mem_mb=(1024, 64, 64, 64))
+    try:
+        M, N, K = 4352, 4096, 512  # cut tiles, finished inside the kernel
+        l, r, y, busy = d.empty((K, M)), d.empty((N, K)), d.empty((N, M)), d.empty(1 << 27)
+        for t in (l, r):
+            d.constant(t, 1.0)
+        for _ in range(3):
+            d.gemm_nn(M, N, K, l, r, 0.0, y)  # the wait below looks at the counter
+            for _ in range(300):  # of 512 MB each: 20 ms and more
+                d.constant(busy, 1.0)
+            errors = []
+
+            def wait():
+                try:
+                    d.sync()
+                except DyhipError as e:
+                    errors.append(e)
+
+            other = threading.Thread(target=wait)
+            other.start()
+            time.sleep(0.005)  # it waits now
+            d.set_gemm_handoff(0, False)
+            d.gemm_nn(M, N, K, l, r, 0.0, y)
+            d.set_gemm_handoff()
+            other.join()
+            wait()
+            assert len(errors) == 1 and "gave up" in str(errors[0])
+            d.sync()  # reported once
+        d.gemm_nn(M, N, K, l, r, 0.0, y)
+        assert np.all(y.numpy() == K)
+    finally:
+        d.close()
