@@ -267,10 +267,12 @@ static int wait_with_words(dyhip_device* q, void* dst, const void* src, size_t n
     DYHIP_CHECK_HIP(hipStreamSynchronize(q->stream));
     return DYHIP_OK;
   }
-  const unsigned n = static_cast<unsigned>(nbytes / sizeof(unsigned));
-  hipLaunchKernelGGL(mail_kernel, dim3(1), dim3(n <= 256 ? 64 : kMailThreads), 0, q->stream, static_cast<const unsigned*>(src),
-                     n, counter, q->mailbox->words, ++q->mailbox->ticket);
-  DYHIP_CHECK_LAUNCH();
+  // The launch's own status, not hipGetLastError: an error that some call before this one left behind is not the copy's.
+  const unsigned* words = static_cast<const unsigned*>(src);
+  unsigned n = static_cast<unsigned>(nbytes / sizeof(unsigned)), ticket = ++q->mailbox->ticket;
+  void* args[] = {&words, &n, &counter, &q->mailbox->words, &ticket};
+  DYHIP_CHECK_HIP(hipLaunchKernel(reinterpret_cast<const void*>(&mail_kernel), dim3(1), dim3(n <= 256 ? 64 : kMailThreads), args, 0,
+                                  q->stream));
   if (!mail_arrives(q->mailbox)) DYHIP_CHECK_HIP(hipStreamSynchronize(q->stream));
   if (nbytes > 0) std::memcpy(dst, q->mailbox->words, nbytes);
   if (counter != nullptr) *count = q->mailbox->words[kMailWords];

@@ -1,4 +1,5 @@
 """Results on their way to the host: by a kernel into page-locked memory up to 16 KiB of whole words, by a copy otherwise."""
+import ctypes as C
 import threading
 import time
 
@@ -96,3 +97,22 @@ def test_a_wait_that_gave_up_behind_another_threads_wait_is_reported():
         assert np.all(y.numpy() == K)
     finally:
         d.close()
+
+
+def test_an_error_that_another_call_left_behind_is_not_the_copys(dev):
+    """A program's own failed HIP call leaves its error with the runtime; reading results and waiting have nothing to do with it."""
+    hip = C.CDLL("libamdhip64.so.7")  # the runtime that the library is linked with: already loaded
+    x = dev.tensor(f32([1.0, 2.0]))
+    M, N, K = 4352, 4096, 512  # its waits are counted: the next wait reads the counter
+    l, r, y = dev.empty((K, M)), dev.empty((N, K)), dev.empty((N, M))
+    dev.constant(l, 1.0)
+    dev.constant(r, 1.0)
+    dev.sync()
+    assert hip.hipSetDevice(4096) != 0
+    assert np.array_equal(x.numpy(), [1.0, 2.0])
+    hip.hipGetLastError()
+    dev.gemm_nn(M, N, K, l, r, 0.0, y)
+    assert hip.hipSetDevice(4096) != 0
+    dev.sync()
+    hip.hipGetLastError()
+    assert np.all(y.numpy() == K)
