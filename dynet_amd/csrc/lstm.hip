@@ -12,6 +12,7 @@
 //
 // Layout: gates is 4H x B column-major, gate order i, f, o, g; c, h are H x B.
 #include <initializer_list>
+#include <type_traits>
 
 #include "gemm.h"
 #include "split3.h"
@@ -1406,18 +1407,18 @@ __global__ __launch_bounds__(256) void gemm_tn_vector_kernel(unsigned M, unsigne
 #pragma unroll
     for (int u = 0; u < 4; ++u) acc[c][u] = 0.f;
   }
-  for (unsigned k0 = 0; k0 < K4; k0 += 256) {
+  const auto round = [&](unsigned k0, auto whole) {
     float4 a[COLS][4], b[4];
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      const unsigned k = k0 + 64 * u + lane, kc = min(k, K4 - 1);
+      const unsigned k = k0 + 64 * u + lane, kc = whole ? k : min(k, K4 - 1);
       b[u] = b4[kc];
-      if (k >= K4) b[u] = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
       for (int c = 0; c < COLS; ++c) a[c][u] = a4[c][kc];
     }
 #pragma unroll
-    for (int u = 0; u < 4; ++u)
+    for (int u = 0; u < 4; ++u) {
+      if (!whole && k0 + 64 * u + lane >= K4) break;  // fetched again and not added: an infinity times zero is none
 #pragma unroll
       for (int c = 0; c < COLS; ++c) {
         acc[c][u] = fmaf(a[c][u].x, b[u].x, acc[c][u]);
@@ -1425,7 +1426,11 @@ __global__ __launch_bounds__(256) void gemm_tn_vector_kernel(unsigned M, unsigne
         acc[c][u] = fmaf(a[c][u].z, b[u].z, acc[c][u]);
         acc[c][u] = fmaf(a[c][u].w, b[u].w, acc[c][u]);
       }
-  }
+    }
+  };
+  unsigned k0 = 0;
+  for (; k0 + 256 <= K4; k0 += 256) round(k0, std::true_type{});
+  if (k0 < K4) round(k0, std::false_type{});
 #pragma unroll
   for (int c = 0; c < COLS; ++c) {
     const float t = wave_sum((acc[c][0] + acc[c][1]) + (acc[c][2] + acc[c][3]));

@@ -31,6 +31,22 @@ def test_transposed_matrix_times_vector_of_a_batch(dev, M, K, items, pad, beta):
     _check(y.numpy(), "imk,ik->im", a[:, :M * K].reshape(items, M, K), v, beta * y0)
 
 
+@pytest.mark.parametrize("K", [256, 1020, 1024, 1028])
+def test_transposed_matrix_of_a_batch_with_infinities(dev, K):
+    """An infinity in the last rows stays one: what a lane fetches past the end is not multiplied."""
+    M, items = 40, 64
+    rng = np.random.default_rng(K)
+    a, v = f32(rng.standard_normal((items, M, K))), f32(rng.standard_normal((items, K)))
+    v[:, -4:] = 0.5
+    a[1, 3, -1], a[2, 5, -4], a[3, 7, -2] = np.inf, -np.inf, np.nan
+    y = dev.empty((items, M))
+    dev.gemm_strided_batched(1, 0, M, 1, K, dev.tensor(a), M * K, dev.tensor(v), K, 0.0, y, M, items)
+    got = y.numpy()
+    assert got[1, 3] == np.inf and got[2, 5] == -np.inf and np.isnan(got[3, 7])
+    got[1, 3] = got[2, 5] = got[3, 7] = 0.0
+    assert np.all(np.isfinite(got))
+
+
 @pytest.mark.parametrize("K", [1, 32, 33, 35, 48, 49, 64, 65])  # depths in one round of loads a wavefront, and one more
 @pytest.mark.parametrize("M,items", [(256, 3), (260, 20), (1024, 8)])
 def test_matrix_times_vector_of_a_batch(dev, M, K, items):
