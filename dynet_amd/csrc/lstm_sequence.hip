@@ -89,12 +89,12 @@ struct SeqState {
     m = p[64];
     l = p[128];
   }
-  // value i of the eight; an infinity or NaN, or what is one times 2^16, is in its first part
+  // value i of the eight; see seq_split for what the parts hold where the first one is no number
   __device__ __forceinline__ static float value(const unsigned* step, unsigned lane, unsigned i) {
     const unsigned short* p = reinterpret_cast<const unsigned short*>(step) + lane * 8 + i;
     const float h = __uint_as_float(unsigned(p[0]) << 16), m = __uint_as_float(unsigned(p[512]) << 16),
                 l = __uint_as_float(unsigned(p[1024]) << 16);
-    return (h * 0.f == 0.f ? h + (m + l) : h) * (1.f / kSplitIn);
+    return h * 0.f == 0.f ? (h + (m + l)) * (1.f / kSplitIn) : __uint_as_float(unsigned(p[512]) << 16 | p[1024]);
   }
   // Where the pair of values that depth k is one of lies in a step of `width` depths and 64 / (width / 8) columns: the
   // first part's word; the others are 256 words on.
@@ -107,17 +107,26 @@ struct SeqState {
   }
 };
 // The parts of 2^16 times this thread's value and its neighbour's (threads 2i and 2i + 1 have neighbouring units), packed.
-// Each value by itself: split3_pair would spread an infinity to the other value of its pair.
+// Each value by itself: split3_pair would spread an infinity to the other value of its pair.  A value of about 2^111 or more,
+// an infinity and a NaN leave a first part that is no number, and the products with it are formed again by the fp32
+// instruction: with KEEP the other two parts hold such a value as it is.  That is rare, and a wavefront that has one
+// (seq_keeps) puts its parts a second time.
+template <bool KEEP>
 __device__ __forceinline__ void seq_split(float v, unsigned (&part)[3]) {
+  const unsigned bits = __float_as_uint(v);
+  bool keep = false;
   v *= kSplitIn;
 #pragma unroll
   for (int i = 0; i < 3; ++i) {
-    const unsigned mine = __builtin_bit_cast(unsigned, __builtin_convertvector(floatx2{v, 0.f}, bf16x2));
+    unsigned mine = __builtin_bit_cast(unsigned, __builtin_convertvector(floatx2{v, 0.f}, bf16x2));
     v -= __uint_as_float(mine << 16);
+    if (KEEP && i == 0) keep = (mine & 0x7f80u) == 0x7f80u;
+    if (KEEP && i > 0 && keep) mine = i == 1 ? bits >> 16 : bits & 0xffffu;
     const unsigned other = __builtin_amdgcn_update_dpp(0, mine, 0xB1, 0xF, 0xF, false);
     part[i] = threadIdx.x & 1 ? mine << 16 | other : other << 16 | mine;
   }
 }
+__device__ __forceinline__ bool seq_keeps(float v) { return !(fabsf(v) < 0x1p110f); }
 
 // Waits, with all threads of the block, until every row tile of a column tile has finished `want` timesteps.
 __device__ __forceinline__ void seq_wait(const SeqSync& y, unsigned ct, unsigned want, bool& dead) {
@@ -138,11 +147,19 @@ __device__ __forceinline__ void seq_wait(const SeqSync& y, unsigned ct, unsigned
   __syncthreads();
 }
 
-// After this block's part of the state has been written through: raises its flag.
+// After this block's part of the state has been written through: raises its flag.  What a timestep writes for later launches
+// (gates, c and h, or dpre) comes behind it: stored while the flags were on their way it held them up, all blocks' at once, by
+// 0.65 us at H = 1024, B = 128 backward (11.9 -> 11.2 us a timestep) and 0.4 at H = 650, B = 20 forward (5.1 -> 4.7).  Up to eight
+// row tiles there is too little of it, and the wait is the longer one (H = 128, B = 32 backward 3.2 -> 3.35; 16 tiles, H = 256,
+// 3.6 either way).
 __device__ __forceinline__ void seq_raise(const SeqSync& y, unsigned ct, unsigned rt, unsigned steps) {
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
   if (threadIdx.x == 0) __hip_atomic_store(y.flags + size_t(ct) * y.RT + rt, steps, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  if (y.RT > 8) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+  }
 }
 
 // Which block works on which tile.  Every tile has a block of its own in the grid; a block that runs takes its tile
@@ -294,12 +311,19 @@ struct SeqFwd {
   }
 
   __device__ __forceinline__ void publish(unsigned rt, unsigned t, float hv) {
-    unsigned part[3];
-    seq_split(hv, part);
     unsigned* to = a.state + (size_t(t) * a.sync.CT + ct) * a.ksteps * 768 + SeqState::word<16>(rt * UB + eu, col);
     const bool odd = threadIdx.x & 1;
-    SeqState::put(to + (odd ? 256 : 0), odd ? part[1] : part[0]);
-    if (!odd) SeqState::put(to + 512, part[2]);
+    const auto put = [&](const unsigned (&part)[3]) {
+      SeqState::put(to + (odd ? 256 : 0), odd ? part[1] : part[0]);
+      if (!odd) SeqState::put(to + 512, part[2]);
+    };
+    unsigned part[3];
+    seq_split<false>(hv, part);
+    put(part);
+    if (__builtin_expect(__any(seq_keeps(hv)), 0)) {
+      seq_split<true>(hv, part);
+      put(part);
+    }
   }
 
   // Cell update of this thread's (unit, column); h goes to the blocks that wait for it before anything else is written.
@@ -596,12 +620,23 @@ struct SeqBwd {
         const bool odd = threadIdx.x & 1;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          seq_split(in ? out[q] : 0.f, part[q]);
+          seq_split<false>(in ? out[q] : 0.f, part[q]);
           SeqState::put(to + SeqState::word<32>(q * Hp + ej, col % 16) + (odd ? 256 : 0), odd ? part[q][1] : part[q][0]);
         }
 #pragma unroll
         for (int q = 0; q < 4; q += 2)
           SeqState::put(to + SeqState::word<32>((q + odd) * Hp + ej, col % 16) + 512, odd ? part[q + 1][2] : part[q][2]);
+        const float largest = fmaxf(fmaxf(fabsf(out[0]), fabsf(out[1])), fmaxf(fabsf(out[2]), fabsf(out[3])));
+        if (__builtin_expect(__any(in && seq_keeps(largest)), 0)) {
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            unsigned kept[3];
+            seq_split<true>(in ? out[q] : 0.f, kept);
+            unsigned* at = to + SeqState::word<32>(q * Hp + ej, col % 16);
+            SeqState::put(at + (odd ? 256 : 0), odd ? kept[1] : kept[0]);
+            if (!odd) SeqState::put(at + 512, kept[2]);
+          }
+        }
       }
     }
     seq_raise(a.sync, ct, rt, s + 1);

@@ -401,8 +401,7 @@ int dyhip_lstm_step_backward_packed(dyhip_device* dev, unsigned H, unsigned B, c
  * gradient that reaches every h_t from outside the recurrence, and writes dpre of every timestep.  Wh is read as it lies.
  * dyhip_lstm_sequence_workspace: bytes that either call needs, on a 256-byte boundary; 0 where the sizes are not
  * supported (H beyond 1024, more tiles of units x columns than CUs): the single timesteps cover those.  Calls on queues
- * that overlap need a workspace each.  Same results as the timesteps up to fp32 summation order; a dpre of 2^111 or more
- * counts as infinite in the recurrent product. */
+ * that overlap need a workspace each.  Same results as the timesteps up to fp32 summation order. */
 int dyhip_lstm_sequence_workspace(dyhip_device* dev, unsigned H, unsigned B, unsigned T, size_t* bytes);
 int dyhip_lstm_sequence_forward(dyhip_device* dev, unsigned H, unsigned B, unsigned T, const float* Wh, const float* mask_h,
                                 const float* xproj, const float* b, int logistic_mode, float* gates, float* c, float* h,

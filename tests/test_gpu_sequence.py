@@ -196,6 +196,24 @@ def test_sequence_keeps_infinities_nans_and_small_values(dev):
     assert np.linalg.norm(got[:, rest] - ref[:, rest]) <= 1e-6 * np.linalg.norm(ref[:, rest])
 
 
+@pytest.mark.parametrize("power", [90, 110, 111, 118])
+def test_sequence_keeps_large_gradients(dev, power):
+    """Gradients up to fp32's range reach the timesteps before theirs: nothing counts as infinite that is not."""
+    k = Case(70, 20, 4, True)
+    k.dh[:, 11, :] *= np.float32(2.0 ** power)
+    k.dh[3, 13, 2] = np.float32(2.0 ** 120)
+    gates, c, _ = k.forward()
+    g32, c32 = _f(gates), _f(c)
+    ref = k.backward(g32, c32)
+    assert np.max(np.abs(ref)) < 2.0 ** 124
+    k.place(dev)
+    k.run_backward(dev, dev.tensor(g32), dev.tensor(c32))
+    got = _d(k.dpre.numpy())
+    for b in range(20):
+        for t in range(4):
+            assert np.linalg.norm(got[t, b] - ref[t, b]) <= 2e-6 * np.linalg.norm(ref[:, b])
+
+
 def test_sequence_reports_a_wait_that_gave_up_and_refuses_what_it_cannot_do(dev):
     k = Case(300, 40, 30, False).place(dev)
     k.run_forward(dev)
