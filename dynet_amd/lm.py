@@ -116,7 +116,13 @@ class LstmLM:
         self.d_logits = dev.empty((N, V), pool=DE)
         self.d_emb = dev.empty((T, B, E), pool=DE)
         self.d_h = [dev.empty((T, B, H), pool=DE) for _ in range(L)]
-        self.d_c = [dev.empty((T, B, H), pool=DE) for _ in range(L)]
+        # all timesteps of a layer as one launch each way where the sizes allow; the layers take turns with its scratch
+        # (a launch that takes about 20 us before its second timestep, then at H = 1024, B = 128 4.5 us a timestep less than a
+        # launch each; at H = 128, where that is 0.2 forward and 0.8 backward, from 16 timesteps on)
+        long_enough = T >= (16 if H == 128 else 5)
+        nseq = dev.lstm_sequence_workspace(H, B, T) if (path == "fused" and long_enough and not self.overlap
+                                                        and single_launch is None) else 0
+        self.d_c = [dev.empty((T, B, H), pool=DE) for _ in range(L)] if nseq == 0 else []  # the sequence keeps dc on chip
         self.d_gates = [dev.empty((T, B, 4 * H), pool=DE) for _ in range(L)]
         self.de_bytes = dev.pool(DE).used() - self.de_begin
         if self.defer:  # the gathered operands of a layer's recorded products
@@ -124,14 +130,26 @@ class LstmLM:
             self.gath_x = dev.empty((T, B, max(E, H)), pool=DE)
             self.gath_h = dev.empty((T, B, H), pool=DE)
         self.d_pre = [dev.empty((T, B, 4 * H), pool=DE) for _ in range(L)]  # overwritten, never accumulated into
-        # all timesteps of a layer as one launch each way where the sizes allow; the layers take turns with its scratch
-        # (a launch that takes about 20 us before its second timestep, then at H = 1024, B = 128 4.5 us a timestep less than a
-        # launch each; at H = 128, where that is 0.2 forward and 0.8 backward, from 16 timesteps on)
-        long_enough = T >= (16 if H == 128 else 5)
-        nseq = dev.lstm_sequence_workspace(H, B, T) if (path == "fused" and long_enough and not self.overlap
-                                                        and single_launch is None) else 0
-        self.sequence = nseq > 0
-        self.seq_ws, self.seq_bytes = dev.workspace(nseq)
+        # queue l runs layer l; queue 0 is the device itself
+        self.queues = [dev] + ([dev.fork() for _ in range(L - 1)] if self.overlap else [])
+        self.plan, self.plan_ws, self.plan_ws_bytes = dev.lookup_plan_buffers(N, V)
+        self.graph = None
+        # page-locked staging for the ids and the flattened label offsets, two sets used in turn: a set is
+        # rewritten only after a device sync that follows the copy that read it
+        from .device import DyhipError, PinnedArray
+        self._stage = [(PinnedArray((N,), np.uint32), PinnedArray((N,), np.uint32)) for _ in range(2)]
+        self._stage_at = 0
+        # Last, when all that either schedule needs is there: the sequence has a place for every timestep of the state (110 MB at
+        # H = 1024, B = 128, T = 35), and where that does not fit the single timesteps do.
+        self.seq_ws, self.seq_bytes = None, 0
+        if nseq > 0:
+            try:
+                self.seq_ws, self.seq_bytes = dev.workspace(nseq)
+            except DyhipError as e:
+                if e.status != lib.ERR_OUT_OF_MEMORY:
+                    raise
+                self.d_c = [dev.empty((T, B, H), pool=DE) for _ in range(L)]
+        self.sequence = self.seq_bytes > 0
         fb, bb = dev.lstm_cell_workspace(H, B)
         self.rec_f_bytes, self.rec_b_bytes = fb, bb
         self.rec_f = [dev.workspace(fb)[0] for _ in range(L)] if not self.sequence else []  # one per layer: layers run side by side
@@ -147,15 +165,6 @@ class LstmLM:
         nd = dev.lstm_packed_state16_floats(4 * H, B) if packed else 0
         self.h_packed = [[dev.empty((nh,), pool=FXS) for _ in range(2)] for _ in range(L)] if packed else []
         self.dpre_packed = [[dev.empty((nd,), pool=DE) for _ in range(2)] for _ in range(L)] if packed else []
-        # queue l runs layer l; queue 0 is the device itself
-        self.queues = [dev] + ([dev.fork() for _ in range(L - 1)] if self.overlap else [])
-        self.plan, self.plan_ws, self.plan_ws_bytes = dev.lookup_plan_buffers(N, V)
-        self.graph = None
-        # page-locked staging for the ids and the flattened label offsets, two sets used in turn: a set is
-        # rewritten only after a device sync that follows the copy that read it
-        from .device import PinnedArray
-        self._stage = [(PinnedArray((N,), np.uint32), PinnedArray((N,), np.uint32)) for _ in range(2)]
-        self._stage_at = 0
 
     @staticmethod
     def init_params(V, E, H, L, seed=0):

@@ -4,6 +4,7 @@ import numpy as np
 import pytest
 
 from oracle import lm_oracle
+from dynet_amd import DyhipError, lib
 from dynet_amd.lm import LstmLM
 from dynet_amd.synth import zipf_ids
 from util import assert_close, FWD_RTOL, GRAD_RTOL
@@ -186,6 +187,30 @@ def test_lm_step_matches_oracle_at_production_width(dev, wide_case, path, time_b
     for n in ref_p:  # SimpleSGD with that scale: p -= lr * scale * g
         want = params[n].astype(np.float64) - 0.1 * exact * ref_g[n].astype(np.float64)
         assert_close(new_p[n], want, GRAD_RTOL, f"param {n}", floor=_grad_floor(ref_p[n]))
+
+
+@pytest.mark.parametrize("V,E,H,L,B,T", [(50, 16, 32, 2, 8, 5), (300, 64, 256, 2, 16, 5)])
+def test_lm_without_memory_for_all_timesteps_of_the_state(dev, monkeypatch, V, E, H, L, B, T):
+    """Where the scratch of the one-launch layer does not fit, the timesteps run one by one, with the same results."""
+    rng = np.random.default_rng(29)
+    params = LstmLM.init_params(V, E, H, L, seed=2)
+    tokens = _tokens(rng, V, B, T)
+    need, workspace = dev.lstm_sequence_workspace(H, B, T), dev.workspace
+
+    def small_workspace(nbytes):
+        if nbytes == need:
+            raise DyhipError(lib.ERR_OUT_OF_MEMORY, "no memory")
+        return workspace(nbytes)
+
+    monkeypatch.setattr(dev, "workspace", small_workspace)
+    lm = LstmLM(dev, V, E, H, L, B, T, lr=0.1, clip=5.0, params=params)
+    assert not lm.sequence and lm.single_launch == (H % 128 == 0)
+    ref_p = {n: a.copy() for n, a in params.items()}
+    ref_loss, ref_g, _ = lm_oracle.step(ref_p, tokens, L, lr=0.1, clip=5.0)
+    assert_close(lm.step(tokens), ref_loss, FWD_RTOL * 4, "loss")
+    new_p = lm.get_params()
+    for n in ref_p:
+        assert_close(new_p[n], ref_p[n], GRAD_RTOL, f"param {n}", floor=_grad_floor(ref_p[n]))
 
 
 def test_lm_clipping_engages(dev):
