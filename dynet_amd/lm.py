@@ -116,11 +116,13 @@ class LstmLM:
         self.d_logits = dev.empty((N, V), pool=DE)
         self.d_emb = dev.empty((T, B, E), pool=DE)
         self.d_h = [dev.empty((T, B, H), pool=DE) for _ in range(L)]
-        # all timesteps of a layer as one launch each way where the sizes allow; the layers take turns with its scratch
-        # (a launch that takes about 20 us before its second timestep, then at H = 1024, B = 128 4.5 us a timestep less than a
-        # launch each; at H = 128, where that is 0.2 forward and 0.8 backward, from 16 timesteps on)
-        long_enough = T >= (16 if H == 128 else 5)
-        nseq = dev.lstm_sequence_workspace(H, B, T) if (path == "fused" and long_enough and not self.overlap
+        # all timesteps of a layer as one launch each way where the sizes allow, from five timesteps on; the layers take turns
+        # with its scratch.  Forward and backward of a layer, a launch a timestep and one launch, us in a graph at T = 3, 5, 8:
+        # H = 1024, B = 128 166 and 168, 245 and 229, 360 and 312; H = 384, B = 1 47 and 49, 70 and 68, 101 and 92; H = 256,
+        # B = 32 54 and 51, 76 and 67, 110 and 90; H = 128, B = 1 40 and 43, 56 and 56, 80 and 76; H = 128, B = 128 57 and 56,
+        # 79 and 72, 114 and 99; H = 64, B = 1 (two launches a timestep each way) 46 and 41, 75 and 54, 115 and 71.  Issued call
+        # by call it is the faster one from two timesteps on at the small sizes (H = 128, B = 1, T = 5 112 and 57).
+        nseq = dev.lstm_sequence_workspace(H, B, T) if (path == "fused" and T >= 5 and not self.overlap
                                                         and single_launch is None) else 0
         self.d_c = [dev.empty((T, B, H), pool=DE) for _ in range(L)] if nseq == 0 else []  # the sequence keeps dc on chip
         self.d_gates = [dev.empty((T, B, 4 * H), pool=DE) for _ in range(L)]

@@ -40,7 +40,7 @@ def test_lm_step_matches_oracle(dev, case, path, time_batched, overlap):
     for l in range(L):  # non-zero biases exercise the bias path
         params[f"b{l}"] = rng.normal(0, 0.1, 4 * H).astype(np.float32)
     ref_p = {n: a.copy() for n, a in params.items()}
-    # "fused" takes the single-launch forward step where the hidden size allows it (H = 128 here)
+    # "fused" takes one-launch layers from T = 5 on; the one-launch timestep is there where the hidden size allows it (H = 128)
     lm = LstmLM(dev, V, E, H, L, B, T, lr=0.1, clip=5.0, time_batched=time_batched, params=params,
                 path=path.split("_")[0], overlap=overlap, chunk=2, single_launch=None if path == "fused" else False,
                 defer_weight_grads=path == "nodes_deferred")
@@ -77,8 +77,8 @@ def test_lm_step_matches_oracle(dev, case, path, time_batched, overlap):
 def test_lm_step_with_dropout_matches_oracle(dev, case, rates, path, time_batched):
     """CompactVanillaLSTMBuilder's dropout (dynet/lstm.cc:964-982,1068-1073): masks drawn on the device once per
     step, in the builder's order, from the generator (recomputed here on the host from seed and position); the step
-    against the oracle's node-by-node composition with the same masks.  The fused path takes its one-launch
-    timesteps with the recurrent mask where the size allows (H = 128, 256), the plain products elsewhere."""
+    against the oracle's node-by-node composition with the same masks.  The fused path takes its one-launch layers from
+    five timesteps on; below, one-launch timesteps with the recurrent mask (H = 256) or the plain products (H = 20)."""
     from oracle import cpu_oracle as orc
 
     V, E, H, L, B, T = case
@@ -147,7 +147,10 @@ def wide_case():
     """The LM configuration's layer widths (E = 256, H = 1024, two layers, B = 128: the sizes that select the
     production kernels - large GEMM tiles, the single-launch timestep, split-K recurrent products) with a
     vocabulary and a sequence length small enough for one CPU core: the oracle step takes ~10 s, once."""
-    V, E, H, L, B, T = 300, 256, 1024, 2, 128, 3
+    return _wide(300, 256, 1024, 2, 128, 3)
+
+
+def _wide(V, E, H, L, B, T):
     rng = np.random.default_rng(23)
     params = LstmLM.init_params(V, E, H, L, seed=5)
     for l in range(L):
@@ -187,6 +190,41 @@ def test_lm_step_matches_oracle_at_production_width(dev, wide_case, path, time_b
     for n in ref_p:  # SimpleSGD with that scale: p -= lr * scale * g
         want = params[n].astype(np.float64) - 0.1 * exact * ref_g[n].astype(np.float64)
         assert_close(new_p[n], want, GRAD_RTOL, f"param {n}", floor=_grad_floor(ref_p[n]))
+
+
+@pytest.fixture()
+def one_launch_layers(dev, monkeypatch):
+    """How often a layer's timesteps were issued as one launch, forward and backward."""
+    calls = []
+    for name in ("lstm_sequence_forward", "lstm_sequence_backward"):
+        def counted(*a, _call=getattr(dev, name), **k):
+            calls.append(1)
+            return _call(*a, **k)
+
+        monkeypatch.setattr(dev, name, counted)
+    return calls
+
+
+# the shortest sequence of the one-launch layer, one less and a longer one
+@pytest.mark.parametrize("case", [(300, 64, 128, 2, 32, 5), (300, 64, 128, 2, 32, 4), (300, 64, 128, 2, 32, 16),
+                                  (60, 32, 1024, 1, 128, 5)])
+def test_lm_step_with_one_launch_layers_matches_oracle(dev, one_launch_layers, case):
+    test_lm_step_matches_oracle_at_production_width(dev, _wide(*case), "fused", True, False)
+    assert len(one_launch_layers) == (2 * case[3] if case[5] >= 5 else 0)
+
+
+@pytest.mark.parametrize("case,rates", [((300, 64, 128, 2, 32, 5), (0.3, 0.3)), ((200, 128, 256, 2, 64, 5), (0.25, 0.4)),
+                                        ((100, 32, 200, 2, 20, 6), (0.0, 0.4))])
+def test_lm_step_with_dropout_and_one_launch_layers_matches_oracle(dev, one_launch_layers, case, rates):
+    test_lm_step_with_dropout_matches_oracle(dev, case, rates, "fused", True)
+    assert len(one_launch_layers) == 2 * 2 * case[3]
+
+
+def test_lm_step_with_a_launch_a_timestep_matches_oracle(dev, one_launch_layers, monkeypatch):
+    monkeypatch.setattr(dev, "lstm_sequence_workspace", lambda *sizes: 0)
+    test_lm_step_matches_oracle(dev, (300, 64, 128, 2, 32, 6), "fused", True, False)
+    test_lm_step_with_dropout_matches_oracle(dev, (300, 64, 128, 2, 32, 6), (0.3, 0.3), "fused", True)
+    assert not one_launch_layers
 
 
 @pytest.mark.parametrize("V,E,H,L,B,T", [(50, 16, 32, 2, 8, 5), (300, 64, 256, 2, 16, 5)])
