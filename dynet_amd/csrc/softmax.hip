@@ -412,6 +412,8 @@ __global__ __launch_bounds__(256) void onehot_kernel(size_t rows, size_t total, 
 }
 
 // ---- argmax along dim 0, first maximum ---------------------------------------
+// At every length what a walk down the column with a strict > finds: NaNs are passed over, a column that starts with one and
+// one of nothing but -infinity have their maximum in row 0.
 // (value, index) of the better of two candidates: the greater value, the lower index among equal values; an index of
 // ~0 marks "none yet"
 __device__ __forceinline__ void argmax_take(float& bv, unsigned long long& bi, float ov, unsigned long long oi) {
@@ -423,7 +425,8 @@ __device__ __forceinline__ void argmax_take(float& bv, unsigned long long& bi, f
 
 // A thread's scan of elements first, first + step, ... of a column: eight loads in flight (one load and one compare
 // a step is one memory round trip a step: 50 000 rows x 512 columns took 93 us, 1.1 TB/s); ascending order, so a
-// strict > keeps the first maximum.  Entries past the end are fetched from the column's last row and skipped.
+// strict > keeps the first maximum.  Entries past the end are fetched from the column's last row and skipped.  Nothing
+// above -infinity leaves bi at ~0.
 __device__ __forceinline__ void argmax_scan(const float* __restrict__ px, size_t rows, size_t first, size_t step, float& bv,
                                             unsigned long long& bi) {
   for (size_t i0 = first; i0 < rows; i0 += 8 * step) {
@@ -436,12 +439,17 @@ __device__ __forceinline__ void argmax_scan(const float* __restrict__ px, size_t
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
       const size_t i = i0 + u * step;
-      if (i < rows && (bi == ~0ull || v[u] > bv)) {
+      if (i < rows && v[u] > bv) {
         bv = v[u];
         bi = i;
       }
     }
   }
+}
+
+// The row of a column's first maximum from what the scans found (~0: nothing above -infinity) and the column's first value.
+__device__ __forceinline__ long long argmax_row(unsigned long long bi, float first) {
+  return first != first || bi == ~0ull ? 0 : static_cast<long long>(bi);
 }
 
 __device__ __forceinline__ void argmax_wave(float& bv, unsigned long long& bi) {
@@ -476,8 +484,6 @@ __device__ __forceinline__ void argmax_wave_equal(float& bv, unsigned long long&
 // values before and after its 16-byte groups beside them; after that the time is the merge's.  us in a graph, with 32-bit loads
 // eight in flight and a merge through one thread, and now: 10 000 rows x 1 column 5.0 and 2.75, x 32 5.5 and 3.2, x 512 7.4 and
 // 4.3, 8192 x 1 3.6 and 2.6, 50 000 x 512 19.1 and 16.3 (6.3 TB/s), 2049 x 512 3.6 and 3.4.
-// A column of nothing but -infinity has its first maximum in row 0, and so has one with a NaN there; other NaNs are passed
-// over: what a walk down the column with a strict > finds.
 template <int T, int U>
 __global__ __launch_bounds__(T) void argmax_cols_kernel(size_t rows, const float* __restrict__ x,
                                                         long long* __restrict__ idx) {
@@ -535,11 +541,13 @@ __global__ __launch_bounds__(256) void argmax_cols_wave_kernel(size_t rows, unsi
                                                                long long* __restrict__ idx) {
   const unsigned c = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (c >= cols) return;
+  const float* px = x + size_t(c) * rows;
+  const float first = px[0];
   float bv = -INFINITY;
   unsigned long long bi = ~0ull;
-  argmax_scan(x + size_t(c) * rows, rows, threadIdx.x & 63, 64, bv, bi);
+  argmax_scan(px, rows, threadIdx.x & 63, 64, bv, bi);
   argmax_wave(bv, bi);
-  if ((threadIdx.x & 63) == 0) idx[c] = static_cast<long long>(bi);
+  if ((threadIdx.x & 63) == 0) idx[c] = argmax_row(bi, first);
 }
 
 // one thread per column (at most 32 rows: a block per column left 252 of 256 threads idle on 4-row columns)
@@ -547,10 +555,12 @@ __global__ __launch_bounds__(256) void argmax_cols_thread_kernel(size_t rows, un
                                                                  long long* __restrict__ idx) {
   const unsigned c = blockIdx.x * 256 + threadIdx.x;
   if (c >= cols) return;
+  const float* px = x + size_t(c) * rows;
+  const float first = px[0];
   float bv = -INFINITY;
   unsigned long long bi = ~0ull;
-  argmax_scan(x + size_t(c) * rows, rows, 0, 1, bv, bi);
-  idx[c] = static_cast<long long>(bi);
+  argmax_scan(px, rows, 0, 1, bv, bi);
+  idx[c] = argmax_row(bi, first);
 }
 
 static void launch_argmax_cols(dyhip_device* dev, size_t rows, unsigned bd, const float* x, long long* idx);
@@ -610,7 +620,7 @@ __global__ __launch_bounds__(256) void col_chunk_kernel(size_t rows, const float
       if (i >= r1) continue;
       if (MODE == 0) ms_push1(ms, x[u]);
       else if (MODE == 1) dot += pb != nullptr ? x[u] * y[u] : x[u];
-      else if (bi == ~0ull || x[u] > bv) {
+      else if (x[u] > bv) {
         bv = x[u];
         bi = i;
       }
@@ -654,7 +664,7 @@ __global__ __launch_bounds__(256) void col_chunk_kernel(size_t rows, const float
     if (threadIdx.x == 0) {
       for (int k = 1; k < 4; ++k) argmax_take(bv, bi, l0[k], li[k]);
       part[2 * at] = bv;
-      reinterpret_cast<unsigned*>(part)[2 * at + 1] = static_cast<unsigned>(bi - r0);  // row inside the chunk
+      reinterpret_cast<unsigned*>(part)[2 * at + 1] = bi == ~0ull ? 0 : static_cast<unsigned>(bi - r0);  // row inside the chunk
     }
   }
 }
@@ -699,6 +709,7 @@ __global__ __launch_bounds__(64) void col_finish_kernel(size_t rows, unsigned ch
     s = wave_sum(s);
     if (lane == 0) out0[b] = s;
   } else {
+    const float first = x[size_t(b) * rows];
     float bv = -INFINITY;
     unsigned long long bi = ~0ull;
     for (unsigned c = lane; c < chunks; c += 64) {
@@ -707,9 +718,8 @@ __global__ __launch_bounds__(64) void col_finish_kernel(size_t rows, unsigned ch
       argmax_take(bv, bi, v, i);
     }
     argmax_wave(bv, bi);
-    if (lane == 0) idx[b] = static_cast<long long>(bi);
+    if (lane == 0) idx[b] = argmax_row(bi, first);
   }
-  (void)rows;
 }
 
 static void launch_argmax_cols(dyhip_device* dev, size_t rows, unsigned bd, const float* x, long long* idx) {
@@ -717,7 +727,7 @@ static void launch_argmax_cols(dyhip_device* dev, size_t rows, unsigned bd, cons
   if (col_chunked(dev, rows, bd, &chunks)) {
     float* part = static_cast<float*>(dev->gemm_ws);
     hipLaunchKernelGGL(col_chunk_kernel<2>, dim3(chunks, bd), dim3(256), 0, dev->stream, rows, x, nullptr, part);
-    hipLaunchKernelGGL(col_finish_kernel<2>, dim3(bd), dim3(64), 0, dev->stream, rows, chunks, part, nullptr, nullptr,
+    hipLaunchKernelGGL(col_finish_kernel<2>, dim3(bd), dim3(64), 0, dev->stream, rows, chunks, part, x, nullptr,
                        nullptr, nullptr, nullptr, idx);
     return;
   }

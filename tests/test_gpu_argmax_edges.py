@@ -3,6 +3,7 @@ import numpy as np
 import pytest
 
 from dynet_amd import DevTensor
+from oracle import cpu_oracle as orc
 from tests.util import f32
 
 pytestmark = pytest.mark.gpu
@@ -31,3 +32,32 @@ def test_first_maximum_of_a_column(dev, rows, offset):
     want = np.where(np.isnan(x), -np.inf, x).argmax(axis=1)
     want[16] = 0
     assert np.array_equal(idx.numpy(), want)
+
+
+# a thread, a wavefront, a block and chunks of a column
+@pytest.mark.parametrize("rows,cols", [(1, 20), (5, 20), (32, 20), (33, 20), (64, 20), (100, 20), (2048, 20), (2049, 20), (8193, 20),
+                                       (65536, 20), (70001, 20), (65536, 80)])
+def test_not_a_number_is_passed_over_at_every_length(dev, rows, cols):
+    rng = np.random.default_rng(rows)
+    x = f32(rng.standard_normal((cols, rows)))
+    x[0, 0] = np.nan
+    x[1, 1:] = np.nan
+    x[2, :-1] = np.nan
+    x[3] = np.nan
+    x[4] = -np.inf
+    x[5] = -np.inf
+    x[5, rows // 2:] = np.nan
+    x[6] = -np.inf
+    x[6, rows - 1] = -3e38
+    for c in range(7, 14):
+        x[c, rng.random(rows) < 0.5] = np.nan
+    x[14, : rows // 2] = -np.inf
+    x[15, 1:: 64] = np.nan  # what one lane of a wavefront reads first
+    x[16, 1: 64] = np.nan
+    x[17] = np.inf
+    x[17, 0] = -np.inf
+    idx, fx = dev.empty(cols, np.int64), dev.empty((cols, rows))
+    dev.argmax_cols(rows, cols, dev.tensor(x), idx)
+    assert np.array_equal(idx.numpy(), orc.argmax_cols(rows, cols, x))
+    dev.argmax_onehot_forward(rows, cols, dev.tensor(x), idx, fx)
+    assert np.array_equal(fx.numpy().argmax(axis=1), orc.argmax_cols(rows, cols, x))
