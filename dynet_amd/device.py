@@ -14,7 +14,7 @@ import math
 import numpy as np
 
 from . import lib
-from .lib import cdll
+from .lib import calls as cdll
 
 _vp = C.c_void_p
 _sz = C.c_size_t

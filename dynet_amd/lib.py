@@ -56,9 +56,12 @@ def _load():
     return C.CDLL(LIB_PATH)
 
 
+# ``cdll``: any ctypes objects as arguments; ``calls``: the same library for the package's own calls, with the argument types.
 cdll = _load()
-_declare(cdll)
 cdll.dyhip_last_error.restype = C.c_char_p
+cdll.dyhip_last_error.argtypes = []
+calls = _load()
+_declare(calls)
 
 
 def last_error():

@@ -36,6 +36,16 @@ def test_status_convention_and_last_error():
     assert "null device" in lib.last_error()
 
 
+def test_plain_handle_takes_ctypes_objects_of_any_type():
+    """A program's own calls through lib.cdll are not held to the argument types that the package declares for its own."""
+    p = C.c_void_p(None)
+    assert lib.cdll.dyhip_pool_create_host(b"small", C.c_uint(4096), C.c_ulong(0), C.byref(p)) == lib.OK
+    used = C.c_ulonglong(1)
+    assert lib.cdll.dyhip_pool_used(p, C.byref(used)) == lib.OK and used.value == 0
+    assert lib.cdll.dyhip_pool_set_used(p, C.c_int(0)) == lib.OK
+    assert lib.cdll.dyhip_pool_destroy(p) == lib.OK
+
+
 def test_pool_rounds_to_alignment_and_bumps():
     pool = Pool.create_host("cpu pool", 1 << 20)
     try:
