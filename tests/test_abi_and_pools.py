@@ -4,6 +4,10 @@ AlignedMemoryPool (dynet/aligned-mem-pool.cc:8-91; scenario of
 tests/test-mem.cc:36-48: an allocation larger than the pool forces growth).
 No compute entry point is called here."""
 import ctypes as C
+import os
+import re
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -44,6 +48,29 @@ def test_plain_handle_takes_ctypes_objects_of_any_type():
     assert lib.cdll.dyhip_pool_used(p, C.byref(used)) == lib.OK and used.value == 0
     assert lib.cdll.dyhip_pool_set_used(p, C.c_int(0)) == lib.OK
     assert lib.cdll.dyhip_pool_destroy(p) == lib.OK
+
+
+def test_declared_argument_types_are_those_of_the_header():
+    kinds = {"int": "i", "unsigned": "u", "float": "f", "size_t": "z", "unsigned long long": "q"}
+    text = re.sub(r"/\*.*?\*/", "", open(lib.HEADER_PATH).read(), flags=re.S)
+    want = set()
+    for name, args in re.findall(r"\bdyhip_([a-z0-9_]+)\s*\(([^)]*)\)\s*;", text):
+        args = [a.strip() for a in args.split(",") if a.strip() not in ("", "void")]
+        want.add(name + ":" + "".join("p" if "*" in a or "[" in a else kinds[" ".join(a.split()[:-1])] for a in args))
+    assert {w.split(":")[0] for w in want} == {n[len("dyhip_"):] for n in lib.declared_symbols()}
+    assert set(lib._ARGUMENTS.split()) == want
+
+
+def test_import_needs_the_built_library_and_no_header(tmp_path):
+    package = os.path.dirname(lib.LIB_PATH)
+    os.mkdir(tmp_path / "dynet_amd")
+    for f in os.listdir(package):
+        if f.endswith((".py", ".so")):
+            os.symlink(os.path.join(package, f), tmp_path / "dynet_amd" / f)
+    code = ("from dynet_amd import lib\nfrom dynet_amd.device import Pool\nimport os\n"
+            "assert not os.path.exists(lib.HEADER_PATH), lib.HEADER_PATH\n"
+            "p = Pool.create_host('p', 4096)\nassert p.allocate(64) > 2 ** 32\np.destroy()")
+    subprocess.run([sys.executable, "-c", code], check=True, cwd=tmp_path, env={**os.environ, "PYTHONPATH": str(tmp_path)})
 
 
 def test_pool_rounds_to_alignment_and_bumps():
