@@ -832,7 +832,7 @@ enum { kNnGates = 0, kNnBias = 1, kNnAxpby = 2 };
 
 // A block's row tile.  Blocks go to the XCDs round robin.  Where M is no multiple of 32 two row tiles share a 128-byte line
 // of every k, and with tiles dealt round two L2s fetch it: each XCD takes `each` consecutive row tiles instead (a tile past
-// the last one is computed on the last row and dropped).  us in a graph, dealt round and consecutive: 10 000 x 64 x 1024
+// the last one is computed on the last row and dropped; a way out for its block at the top costs the others 3 %).  us in a graph, dealt round and consecutive: 10 000 x 64 x 1024
 // 28.5 and 26.0, 50 000 x 32 x 1024 55.3 and 51.4, 2600 x 64 x 1300 14.4 and 11.5, 9000 x 32 x 650 13.3 and 12.4, 10 000 x
 // 32 x 1024 15.0 and 14.8.  M a multiple of 32: 16 384 x 32 x 1024 15.6 and 16.4, 12 000 x 32 x 1024 14.4 and 14.9.
 __device__ __forceinline__ unsigned nn_row_tile(unsigned each) {
@@ -1152,10 +1152,14 @@ int skinny_nn_gemm(dyhip_device* dev, size_t M, size_t N, int nseg, const GemmSe
     if (dev->gemm_ws == nullptr || dev->gemm_ws_bytes < sizeof(float) * M * N * splits) splits = 1;
     if (splits == 1 && masks == nullptr) splits = 0;
   }
-  // consecutive row tiles of an XCD, 0: dealt round (also where the padding to 8 XCDs would cost a round of the CUs: 2600 x 20
-  // with masks and three blocks to a depth of 1300, 246 blocks 10.2 us and 264 12.2)
+  // consecutive row tiles of an XCD, 0: dealt round.  Runs pay where there are more blocks than CUs, and from a quarter as many
+  // on with 512 deep (us, dealt round and runs: 10 001 x 64 x 256, 314 blocks, 13.0 and 12.0; 2500 x 64 x 1024, 158, 9.6 and 9.1;
+  // 2500 x 32 x 1024, 79, 9.0 and 8.85; gates of 650 x 9, 82, 12.5 and 12.7; but 2600 x 128 x 256, 164, 6.8 and 6.85; 420 x 32 x
+  // 1024, 14, 8.5 and 8.6; 33 x 128 x 256, 8, 4.65 and 4.73), and not where the padding to 8 XCDs would cost a round of the
+  // CUs: 2600 x 20 with masks and three blocks to a depth of 1300, 246 blocks 10.2 us and 264 12.2.
   const unsigned deep = splits > 1 ? splits : 1;
-  unsigned each = M % 32 == 0 ? 0 : (rt + 7) / 8;
+  const bool runs = M % 32 != 0 && (blocks * deep > cus || (4 * blocks * deep > cus && Kt >= 512));
+  unsigned each = runs ? (rt + 7) / 8 : 0;
   if (cdiv(8 * each * ct * deep, cus) > cdiv(blocks * deep, cus)) each = 0;
   const dim3 grid(each == 0 ? rt : 8 * each, ct), block(256);
   if (splits > 0) {

@@ -11,7 +11,8 @@ pytestmark = pytest.mark.gpu
 # one and two row tiles of 32 a block, the depth in one block and over several; a last tile of one row; tiles padded to a
 # multiple of eight, none to pad, and where padding would cost a round of the CUs (85 x 3 of 256)
 @pytest.mark.parametrize("M,N,K", [(33, 32, 64), (257, 40, 128), (1000, 32, 256), (2600, 20, 1300), (2599, 64, 1300),
-                                   (5001, 33, 96), (10000, 17, 64), (2700, 96, 128), (2705, 70, 520), (16417, 32, 64)])
+                                   (5001, 33, 96), (10000, 17, 64), (2700, 96, 128), (2705, 70, 520), (16417, 32, 64),
+                                   (10001, 64, 256), (2500, 32, 1024)])
 def test_narrow_products_over_ragged_rows(dev, M, N, K):
     rng = np.random.default_rng(M + N)
     W, x, b = f32(rng.standard_normal((K, M))), f32(rng.standard_normal((N, K))), f32(rng.standard_normal(M))
