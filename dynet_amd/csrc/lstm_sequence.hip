@@ -29,7 +29,11 @@ typedef float sums4 __attribute__((ext_vector_type(4)));
 typedef float float4u __attribute__((ext_vector_type(4), aligned(4)));
 
 constexpr unsigned kSeqRedBytes = kSeqWaves * 32 * 32 * sizeof(float);
-constexpr unsigned kSeqPatience = 64;  // polls before a waiting block looks for a tile that no block has taken
+// Polls, about a microsecond apart, before a waiting block looks for a tile that no block has taken.  What holds CUs has mostly
+// ended by then, and a block with two tiles reads its weights again for every timestep: a model of H = 1024, B = 128, T = 35
+// beside a queue of large products 4.1 ms with 8 polls, 3.4 with 64, 2.77 with 256 and with 1024 (3.19 with a launch a timestep);
+// beside another such model 3.0 to 3.5, 2.7, 2.7 and 2.7 ms for both (3.11).
+constexpr unsigned kSeqPatience = 256;
 
 // Which block works on which tile, and how far the tiles are; zero at the start of a launch.
 struct SeqSync {
