@@ -555,7 +555,8 @@ static int gemm_nn_thin_run(dyhip_device* dev, size_t M, size_t N, int nseg, con
   hipLaunchKernelGGL((gemm_nn_thin_kernel<NB, UN>), grid, block, 0, dev->stream, M4, static_cast<unsigned>(N), chunk, s0, s1, \
                      slabs0, C, beta, bias, partial, sa, sb, sc)
   // a batch's depth of 33 to 64 in one round of loads: with eight in flight a second, mostly empty one followed (512 x 1 x
-  // 35 in 128 items 3.8 -> 3.2 us, 256 x 1 x 35 3.5 -> 2.9, 1024 x 1 x 35 3.4 -> 3.3)
+  // 35 in 128 items 3.8 -> 3.2 us, 256 x 1 x 35 3.5 -> 2.9, 1024 x 1 x 35 3.4 -> 3.3).  A single item's depth is cut into slabs of
+  // 32 and less above, or is the row kernel's: one round of eight each
   if (N == 1 && items > 1 && K > 8 * kGemvWaves && K <= 12 * kGemvWaves) DYHIP_GEMV(1, 12);
   else if (N == 1 && items > 1 && K > 12 * kGemvWaves && K <= 16 * kGemvWaves) DYHIP_GEMV(1, 16);
   else if (N == 1) DYHIP_GEMV(1, 8);

@@ -15,7 +15,7 @@ import sys
 import tempfile
 
 HERE = os.path.dirname(os.path.abspath(__file__))
-SRCS = ["elementwise", "cwise", "reduce", "softmax", "lookup", "gemm", "gemm_wide", "gemm_direct", "gemm_tile", "gemm_small", "lstm", "misc", "trainer", "random"]
+SRCS = ["elementwise", "cwise", "reduce", "softmax", "lookup", "gemm", "gemm_wide", "gemm_direct", "gemm_tile", "gemm_small", "lstm", "lstm_sequence", "misc", "trainer", "random"]
 FLAGS = ["-O3", "-std=c++17", "--offload-arch=gfx950", "-ffp-contract=off", "-Xclang", "-target-feature", "-Xclang",
          "-packed-fp32-ops", "-Wno-unused-function", "-Wno-unknown-warning-option", "-I" + os.path.join(HERE, "../../include"),
          "-I" + HERE, "--cuda-device-only", "-S"]
@@ -24,14 +24,14 @@ HOT = ["ew_vec4_kernel<2, true, 0, true, 2, dyhip::AccMul2", "ew_vec4_kernel<1, 
        "ln_fwd_wave_kernel<4, true>", "ln_bwd_wave_kernel<4, true, 8, true, true>", "ln_bwd_team_kernel<4, true>",
        "combine_partials_vec_kernel<64>", "cwise_bcast2_kernel<2, 4, true>", "cwise_reduce_row_kernel<6, true, true>",
        "lookup_gather_kernel<HIP_vector_type<float, 4u>, false, true>", "plan_direct_kernel<16>", "plan_group_kernel<true>",
-       "scatter_runs_kernel<HIP_vector_type<float, 4u>, true>", "lse_cols_kernel<true, true>", "pnls_bwd_kernel<true, true, true>",
-       "lstm_step_fwd_kernel<false, 2>", "lstm_step_bwd_kernel", "skinny_tn_kernel<true, true>", "skinny_nn_kernel<2, 0, 16>", "skinny_nn_kernel<1, 1, 16>", "gemm_tn_mid_kernel<5>",
+       "scatter_runs_kernel<HIP_vector_type<float, 4u>, true>", "lse_cols_kernel<true, dyhip::DeviceIds>", "argmax_cols_kernel<1024, 4>", "pnls_bwd_kernel<true, true, true>",
+       "lstm_step_fwd_kernel<false, 2>", "lstm_step_bwd_kernel", "lstm_sequence_fwd_kernel<1, 4>", "lstm_sequence_fwd_kernel<2, 8>", "lstm_sequence_bwd_kernel<1, 8>", "lstm_sequence_bwd_kernel<2, 16>", "skinny_tn_kernel<true, true>", "skinny_nn_kernel<2, 0, 16>", "skinny_nn_kernel<1, 1, 16>", "gemm_tn_mid_kernel<5>",
        "gemm_wide_kernel<false, false>", "gemm_wide_kernel<false, true>", "gemm_shallow_nt_kernel", "gemm_tile_kernel<false, false>",
        "gemm_direct_kernel<true, true, 1, 1, 8, true>", "gemm_direct_kernel<false, true, 2, 1, 8, true>", "gemm_direct_kernel<false, false, 2, 2, 4, true>",
        "skinny_nn_deep_kernel<1, 8, 0, true>", "lstm_step_fwd_small_kernel<true>",
-       "gather_segments_kernel<true, true>", "sgd_scaled_kernel<true, true>", "philox",
-       "gemm_nn_mid_kernel<true>", "gemm_nn_rows_kernel<1, 8, 4>", "gemm_nn_thin_kernel<1>", "gemm_nt_thin_kernel<32, 4>",
-       "gemm_tn_thin_kernel<4, 2>", "ln_fwd_group_kernel<16, 1, 2, true>", "ln_bwd_group_kernel<16, 1, true>",
+       "gather_segments_kernel<true, true>", "sgd_scaled_kernel<true, true>", "sgd_rows_kernel<HIP_vector_type<float, 4u>", "lookup_gather_host_kernel<64u, HIP_vector_type<float, 4u>, false>", "philox",
+       "gemm_nn_mid_kernel<true>", "gemm_nn_rows_kernel<1, 8, 4>", "gemm_nn_thin_kernel<1, 8>", "gemm_nt_thin_kernel<32, 4>",
+       "gemm_tn_thin_kernel<4, 2>", "gemm_tn_vector_kernel<2>", "ln_fwd_group_kernel<16, 1, 2, true>", "ln_bwd_group_kernel<16, 1, true>",
        "sum_group_kernel<false, false>", "gemm_small_kernel<4, 4, 4>", "gemm_small_kernel<1, 4, 8>", "gemm_small_kernel<4, 4, 1>", "gemm_nt_fewrows_kernel<20>", "col_chunk_kernel<0>",
        "radix_scatter_kernel<true>", "radix_scan_kernel", "moment_chunk_kernel<1>", "rows_slab_kernel<false>",
        "batch_reduce_flat_kernel<false>", "pick_range_flat_kernel<false>", "softmax_resident_kernel<0, 256, 4>", "moment_resident_kernel<1, 256, 4>"]

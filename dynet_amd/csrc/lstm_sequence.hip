@@ -7,12 +7,12 @@
 // alone, multiplies on the bf16 matrix cores, runs the cell update of its (unit, column) pairs and hands its part of the
 // new state to the blocks that work on the same columns.
 //
-// us a timestep in a graph, a launch each -> 35 in one launch, forward / backward: H = 1024, B = 128 13.7 / 14.2 -> 9.1 /
-// 11.0; H = 512, B = 64 6.1 / 8.7 -> 4.6 / 4.7; H = 650, B = 20 (two launches each) 11.4 / 9.2 -> 5.4 / 6.0.  What bounds
-// it at H = 1024, B = 128, forward, by stamps inside the kernel: 1.5 us until the last block's flag is seen, 5.4 for the
-// state's way from the L2 (192 KB a CU) and the products (2.9 of matrix cores), 1.4 for the sums in LDS, 0.4 cell update,
-// 0.4 until the state is in memory; backward the product is 8 us, 768 KB of state a CU at the 85 GB/s that a CU gets from
-// its L2.  Small layers: the hand-over.
+// us a timestep in a graph, a launch each -> 35 in one launch, forward / backward: H = 1024, B = 128 13.7 / 15.1 -> 8.5 /
+// 10.9; H = 512, B = 64 5.9 / 8.6 -> 3.95 / 4.3; H = 650, B = 20 (two launches each) 11.2 / 9.0 -> 4.7 / 5.3.  What bounds
+// it at H = 1024, B = 128, forward, by stamps inside the kernel (when a timestep took 9.1): 1.5 us until the last block's flag
+// is seen, 5.4 for the state's way from the L2 (192 KB a CU) and the products (2.9 of matrix cores), 1.4 for the sums in LDS,
+// 0.4 cell update, 0.4 until the state is in memory; backward the product is 8 us, 768 KB of state a CU, 96 GB/s.  Small
+// layers: the hand-over.
 #include <initializer_list>
 
 #include "common.h"

@@ -19,8 +19,8 @@ What differs from DyNet's node-at-a-time execution (results agree to fp32 roundi
   * ``path="fused"`` (default) runs layer by layer: one GEMM forms Wx*x for all timesteps, a timestep is then
     the recurrent GEMM Wh*h plus one cell kernel (gates + c + h); backward mirrors it, and dx, dWx, dWh, db are
     GEMMs/reductions over all timesteps;
-  * all timesteps of a layer are one kernel each way where the sizes allow (``sequence``; not with overlap=True or an
-    explicit ``single_launch``);
+  * all timesteps of a layer are one kernel each way where the sizes allow and its scratch fits (``sequence``; not with
+    overlap=True or an explicit ``single_launch``, nor for fewer than five timesteps);
   * else a timestep of the fused path is one kernel forward (recurrent product + cell update) and one backward (Wh^T *
     dpre of the step above + cell backward), both reading their operands from packed copies in matrix-core
     fragment order that the previous timestep's kernel wrote (``single_launch``, where the sizes allow);
