@@ -1599,11 +1599,12 @@ static int thin_tn_run(dyhip_device* dev, size_t M, size_t N, size_t K, const fl
   const unsigned items = batch != nullptr && batch->count > 1 ? batch->count : 1;
   const size_t sa = items > 1 ? batch->stride_a : 0, sb = items > 1 ? batch->stride_b : 0, sc = items > 1 ? batch->stride_c : 0;
   // one column, enough of them for a thousand wavefronts (35 x 1 x 1024 in 128 items 4.8 -> 3.2 us, 35 x 1 x 256 4.1 -> 3.2,
-  // 12 x 1 x 1024 in 64 items 3.0 either way; one column of A a wavefront 3.3, three 3.2, streaming loads 3.2-3.8), and A no
-  // larger than the L2s together: beyond, the streaming kernel below is the faster one (in 128 items, this kernel and that one:
-  // 64 x 1 x 1024, 34 MB, 7.0 and 7.1 us; 35 x 1 x 2048, 37 MB, 8.5 and 8.2; 64 x 1 x 2048 14.1 and 11.5; 130 x 1 x 1024
-  // 12.7 and 11.8)
-  if (N == 1 && items > 1 && M * items >= 2048 && M * K * items * sizeof(float) <= (size_t(32) << 20)) {
+  // 12 x 1 x 1024 in 64 items 3.0 either way; one column of A a wavefront 3.3, three 3.2, streaming loads 3.2-3.8).  With more
+  // than 512 deep only where A is no larger than the L2s together: the streaming kernel below and this one, us in 128 items, A of
+  // 32, 40, 64 and 512 MB: 512 deep 9.2 and 7.8, 10.6 and 10.3, 14.5 and 13.7, 99 and 91; 768 deep 8.6 and 7.6, 9.5 and 9.6, 12.8
+  // and 13.6, 83 and 89; 2048 deep 8.4 and 8.3, 9.1 and 10.1, 12.3 and 14.4, 77 and 88; 256 deep 13 and 8, 16 and 11, 23 and 15,
+  // 160 and 100.
+  if (N == 1 && items > 1 && M * items >= 2048 && (K <= 512 || M * K * items * sizeof(float) <= (size_t(32) << 20))) {
     const dim3 vgrid(static_cast<unsigned>(cdiv<size_t>(M, 8)), items);
     hipLaunchKernelGGL((gemm_tn_vector_kernel<2>), vgrid, dim3(256), 0, dev->stream, static_cast<unsigned>(M),
                        static_cast<unsigned>(K / 4), A, lda, B, beta, C, sa, sb, sc);

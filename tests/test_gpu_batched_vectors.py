@@ -21,7 +21,7 @@ def _check(got, subscripts, a, b, y0):
 # one-column kernel (M * items >= 2048) and one fewer
 @pytest.mark.parametrize("M,K,items,pad", [(35, 1024, 64, 0), (1, 256, 2048, 0), (1, 260, 2047, 0), (2, 1020, 1024, 8),
                                            (9, 1028, 228, 4), (33, 2052, 70, 0), (8, 508, 300, 0),
-                                           (64, 1024, 128, 0), (64, 1028, 128, 0)])  # 32 MB of A, and more
+                                           (64, 1024, 128, 0), (64, 1028, 128, 0), (160, 512, 128, 0)])  # 32 MB of A, and more
 @pytest.mark.parametrize("beta", [0.0, 1.0])
 def test_transposed_matrix_times_vector_of_a_batch(dev, M, K, items, pad, beta):
     rng = np.random.default_rng(M * K)
